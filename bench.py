@@ -641,7 +641,7 @@ def phase_profile(torch, dev, synthetic, pack_weights, tq1_matmul_words, tq1_lin
         print(json.dumps({
             "phase_profile": name, "K": K, "N": N, "M": batch, "waves_per_launch": len(phase_times["start"]) // 3,
             "kernel": "wide_gemm_kernel" if wide else (f"strip_gemv_kernel ({m1_form(handle, N, K)})" if strip else
-                                                        ("lut_gemv_kernel" if lut else "direct_gemm_kernel")),
+                                                        ("lut_gemv_kernel" if lut else "trit_gemm_kernel")),
             "gemv_graph_us": round(graph_ms * 1e3, 3),
             "xcc_span_us": quantiles(spans),
             "phases_after_xcc_first_wave_start": {ph: quantiles(v) for ph, v in phase_times.items() if v},

@@ -33,8 +33,8 @@
  * undefined.
  *
  * Activations x are [M][columns] row-major, outputs y are [M][rows] row-major,
- * both of `dtype` (TERNEL_TQ1_F16 is the graded type; BF16 also runs the wide
- * MFMA form, F32 the LUT path only), fp32 accumulation throughout.
+ * both of `dtype` (F16 runs every form; BF16 the matmul path and the MFMA
+ * forms' automatic choice, F32 the matmul path), fp32 accumulation throughout.
  *
  * Workspaces: a split workspace starts with a fixed 64 KiB region of
  * arrival counters whose last 32-bit word is the workspace's error word,
@@ -162,6 +162,11 @@ int ternel_tq1_tiled_from_words(const uint32_t *packed, int64_t rows, int64_t co
  * same form in Z = ceil(groups / 40) K chunks per strip, whose row partials
  * meet in exchange slots in the 64 KiB counter region: its workspace is that
  * region alone, left empty by every call.
+ * Batches (M > 1) with both left automatic run the DIRECT form's kernel of
+ * ternel_tq1_gemm where it is faster (most matrices from M = 3; fp32, as three
+ * bf16 terms per value, exactly, from about M = 4-10 by matrix size), with
+ * the same arithmetic per block: acc = fma(scale, sum of +-x, acc) in fp32. x
+ * that is not 16-byte aligned takes the LUT23 kernel.
  * ws: at least ternel_tq1_matmul_workspace_bytes(...) bytes (0 when the split
  * resolves to 1 or the unsplit form above runs; ws may then be NULL); see the
  * workspace contract above.
@@ -198,8 +203,9 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
  * src/ternel_mlx/kernels.py:1043-1188, re-chosen for CDNA4):
  *   TERNEL_TQ1_GEMM_TILE   (prefill) 128x128 output tiles, weights decoded to
  *                          fp16 (t-1)*scale tiles in LDS;
- *   TERNEL_TQ1_GEMM_DIRECT (M <= 64) weights decoded straight into MFMA
- *                          operand registers, activations staged in LDS,
+ *   TERNEL_TQ1_GEMM_DIRECT (M <= 64) trits decoded straight into MFMA
+ *                          operand registers, block scales applied to the
+ *                          fp32 group sums, activations staged in LDS,
  *                          split-K reduced in the same launch in chunk order;
  *   TERNEL_TQ1_GEMM_WIDE   (M > 32, prefill) weights decoded into operand
  *                          registers of 8 waves of 32 rows, 256-row output
@@ -208,13 +214,15 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
  *                          LDS, K split stream-K over one workgroup per CU
  *                          with an ordered in-launch reduction (k_split must
  *                          be 0/1; columns < 2^22);
- *   TERNEL_TQ1_GEMM_AUTO   DIRECT for M <= 32 (M <= 48 for matrices under
+ *   TERNEL_TQ1_GEMM_AUTO   DIRECT for M <= 32 (M <= 64 for matrices under
  *                          16 MiB of packed weights); WIDE up to M = 64;
  *                          above, WIDE when it has at least CUs/4 output
  *                          tiles or 15 (tile, group) steps per CU, TILE
  *                          otherwise (and for a fixed k_split > 1).
- * bf16 activations (dtype TERNEL_TQ1_BF16) run the WIDE form only (form AUTO
- * or WIDE, no fixed k_split; size the workspace with form WIDE): a pre-pass
+ * bf16 activations (dtype TERNEL_TQ1_BF16) take form AUTO or WIDE and no fixed
+ * k_split (size the workspace with form WIDE). Up to 32 rows (64 for matrices
+ * under 24 MiB of packed weights) they run the DIRECT form's kernel on bf16
+ * MFMAs, as they are; above, the WIDE form after a pre-pass that
  * scales each row by a power of two into fp16's range and converts it (exact:
  * bf16's 8-bit significand fits fp16's 11 bits; values more than 2^28 below
  * the row's largest lose bits), and the fp32 sums are scaled back and rounded
@@ -263,9 +271,10 @@ int ternel_tq1_linear(const uint32_t *packed, const void *x, void *y, int64_t M,
 size_t ternel_tq1_linear_workspace_bytes(int64_t M, int64_t rows, int64_t columns, int dtype);
 
 /*
- * The kernel ternel_tq1_linear launches for this shape: TERNEL_TQ1_KERNEL_LUT23
- * or one of the TERNEL_TQ1_GEMM_* forms (never AUTO); negative on a rejected
- * shape or dtype. Host-only, touches no device. The counterpart of the
+ * The path ternel_tq1_linear takes for this shape: TERNEL_TQ1_KERNEL_LUT23
+ * (ternel_tq1_matmul, with its automatic choice of kernel) or one of the
+ * TERNEL_TQ1_GEMM_* forms of ternel_tq1_gemm (never AUTO; WIDE for every bf16
+ * batch it takes); negative on a rejected shape or dtype. Host-only, touches no device. The counterpart of the
  * reference's select_gemm / select_lut23 decisions (src/ternel_mlx/modules.py
  * :320-423), exposed so that a dispatch sweep can be replayed through the rule.
  */
@@ -280,10 +289,9 @@ int ternel_tq1_linear_kernel(int64_t M, int64_t rows, int64_t columns, int dtype
  * two unfused layers would return them, and SiLU(g) * u is computed in fp32.
  * z is [M][rows / 2] in the activation type. No counterpart in the reference
  * (its MLP runs gate_proj, up_proj and the activation as separate mlx ops,
- * src/ternel_mlx/packed_model.py:72-92). Batches that ternel_tq1_linear sends
- * to the LUT23 kernel (up to 3 rows, 4 for matrices under 16 MiB, and every
- * fp32 batch) run it with the pair exchange in its epilogue; larger fp16 and
- * bf16 batches run the GEMM into the workspace and one elementwise pass. Workspace
+ * src/ternel_mlx/packed_model.py:72-92). The LUT23, strip and direct-form
+ * kernels have the pair exchange in their epilogues; batches of the wide and
+ * tile forms run the GEMM into the workspace and one elementwise pass. Workspace
  * from ternel_tq1_swiglu_workspace_bytes, same contract as ternel_tq1_linear's.
  */
 int ternel_tq1_swiglu(const uint32_t *packed, const void *x, void *z, int64_t M, int64_t rows, int64_t columns,

@@ -104,6 +104,44 @@ __host__ __device__ inline uint32_t selector_entry(int i) {
     return selector_pair(n % 3, n / 3);
 }
 
+// Pair tables: the same pairs of trits directly as two 16-bit MFMA operand
+// values, -1, 0 and +1 in a type whose 1 has the bits `one` (fp16 0x3c00, bf16
+// 0x3f80). Tables read eight bytes at a time hold two dwords per entry:
+//   T27a[a / 9] = (a2, a3), (a4, 0)      T27b[b % 27] = (0, b0), (b1, b2)
+//   T9a[a % 9] = (a0, a1), unused        T9b[b / 27] = (b3, b4), one dword
+// Each table spans at most 58 dwords, so a wave's lookups into one never
+// conflict in the 64 LDS banks. Digits of illegal bytes (3) give zero.
+constexpr int kPairT27a = 0;     // 29 entries of two dwords
+constexpr int kPairT27b = 58;    // 27 entries of two dwords
+constexpr int kPairT9a = 112;    // 9 entries of two dwords
+constexpr int kPairT9b = 130;    // 10 entries
+constexpr int kPairEntries = 140;
+
+__host__ __device__ __attribute__((always_inline)) inline uint32_t trit_value(int d, uint32_t one) {
+    return d == 0 ? one | 0x8000u : (d == 2 ? one : 0u);
+}
+__host__ __device__ __attribute__((always_inline)) inline uint32_t trit_pair(int d_even, int d_odd, uint32_t one) {
+    return trit_value(d_even, one) | (trit_value(d_odd, one) << 16);
+}
+
+// Dword i of the concatenated pair tables.
+__host__ __device__ inline uint32_t pair_entry(int i, uint32_t one) {
+    if (i < kPairT27b) {
+        const int h = i >> 1;
+        return (i & 1) ? trit_pair(h / 9, 1, one) : trit_pair(h % 3, (h / 3) % 3, one);
+    }
+    if (i < kPairT9a) {
+        const int m = (i - kPairT27b) >> 1;
+        return (i & 1) ? trit_pair((m / 3) % 3, m / 9, one) : trit_pair(1, m % 3, one);
+    }
+    if (i < kPairT9b) {
+        const int l = (i - kPairT9a) >> 1;
+        return (i & 1) ? 0u : trit_pair(l % 3, l / 3, one);
+    }
+    const int n = i - kPairT9b;
+    return trit_pair(n % 3, n / 3, one);
+}
+
 // Tail-table entry of a tail byte: the byte itself, clamped to the table.
 __host__ __device__ __attribute__((always_inline)) inline uint32_t tail_entry(uint32_t p) {
     return p < kMaxTailByte ? p : kMaxTailByte;

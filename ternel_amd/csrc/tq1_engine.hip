@@ -1546,46 +1546,29 @@ __global__ __launch_bounds__(kThreads) void mfma_gemm_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// direct_gemm_kernel: the "direct fragments" form for small batches (M <= 64).
-//
-// Weights never touch LDS: each lane decodes half of one block straight into
-// the A operand of v_mfma_f32_32x32x16_f16 (weight rows x K); the activations
-// are the B operand (K x batch). A workgroup (4 waves, 128 weight rows) copies
-// a window of its K chunk's activations into LDS (through registers for up to
-// 16 rows, by LDS-DMA for more), then each wave runs the window's groups with
-// no barrier: a wave owns 32 weight rows, lane l decodes half h = l / 32 of
-// row l % 32's block and reads 5 of the block's 7 words. NB = ceil(M / 32)
-// tiles.
+// Decoding a block into MFMA operands (the trit and wide kernels).
 //
 // K order. The dot product over a group does not depend on the order of its
 // 128 terms, so both operands use one fixed permutation that makes the two
-// halves decode with the same code: half h takes code bytes 12h .. 12h+11
-// (trits 60h .. 60h+59) as positions 0..59, then positions 60..63 are trits
-// 120..123 (digits 0-3 of code byte 24) for h = 0, and trits 124..127 (digit 4
-// of code byte 24, the three tail trits) for h = 1. MFMA step s takes positions
-// 8s .. 8s+7 of half h as its K slice 16s + 8h. The activation rows are staged
-// in that order: logical 4-half unit u holds physical unit u (u < 15), 30
-// (u = 15), u - 1 (16 <= u < 31) or 31 (u = 31).
-//
-// Weights. A lane turns its half block into 32 dwords of fp16 weight pairs:
-// each pair of code bytes is split two bytes per 16-bit-packed operation and
-// indexes six small selector tables in LDS (tq1_bytes.h, half_block_selectors
-// below), and one v_perm_b32 per pair selects the pair's two fp16 values from
-// {-s, z, +s} (z is 0, or NaN for a non-finite scale, as (t - 1) * s gives).
-// Every byte value, legal or not, indexes inside the tables (checked on the
-// CPU over all of them). The wide form decodes the same way; the LDS-tile
-// form keeps the 24-bit digit carriers of tq1_bytes.h.
+// halves of a block decode with the same code: half h takes code bytes 12h ..
+// 12h+11 (trits 60h .. 60h+59) as positions 0..59, then positions 60..63 are
+// trits 120..123 (digits 0-3 of code byte 24) for h = 0, and trits 124..127
+// (digit 4 of code byte 24, the three tail trits) for h = 1. MFMA step s takes
+// positions 8s .. 8s+7 of half h as its K slice 16s + 8h. The activation rows
+// are staged in that order: logical 4-value unit u holds physical unit u (u <
+// 15), 30 (u = 15), u - 1 (16 <= u < 31) or 31 (u = 31).
 // ---------------------------------------------------------------------------
 constexpr int kBufferRsrcFlags = 0x00020000;  // gfx9 raw buffer resource: 32-bit data format
 constexpr int kDirectWaves = 4;
 constexpr int kDirectThreads = kDirectWaves * 64;
 constexpr int kDirectRows = kDirectWaves * 32;          // weight rows per workgroup
-constexpr int kDirectLdsBytes = 160 * 1024 - 1024;      // dynamic LDS budget (gfx950: 160 KiB per workgroup)
-constexpr int kDirectStride = kBlockWeights + 8;      // halves per staged activation row
+constexpr int kDirectStride = kBlockWeights + 8;      // 2-byte values per staged activation row
 
-
-// The 32 selector dwords of one half block (pairs of weights, in the direct K
-// order), from the selector tables in LDS (sel_bytes, tq1_bytes.h): u[0..3]
+// The wide form's weights are fp16 (t - 1) * scale: one v_perm_b32 per pair
+// selects the two values from {-s, z, +s} (z is 0, or NaN for a non-finite
+// scale, as (t - 1) * s gives). The 32 selector dwords of one half block
+// (pairs of weights, in the K order above) come from the selector tables in
+// LDS (sel_bytes, tq1_bytes.h): u[0..3]
 // hold the half's twelve code bytes at bytes 2..13, w6 code byte 24 (byte 2)
 // and the tail byte (byte 3). Code bytes 2w, 2w+1 (window w) give pairs
 // 5w .. 5w+4; pairs 30 and 31 are code byte 24's first four weights in the
@@ -1657,307 +1640,417 @@ __device__ __forceinline__ uint32_t full_selector(const uint32_t (&sel)[32], con
     return q == 30 ? sel[30] | late[6] : (q < 30 && q % 5 == 2 ? sel[q] | late[q / 5] : sel[q]);
 }
 
-__device__ __forceinline__ void half_block_selectors(const uint32_t (&u)[4], uint32_t w6, bool upper,
-                                                     const char *sel_bytes, uint32_t (&sel)[32]) {
-    uint32_t late[7];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const WindowSplits s = window_splits(u, k);
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            window_selectors(s, k, e, sel_bytes, sel, late);
-            sel[5 * (2 * k + e) + 2] |= late[2 * k + e];
-        }
-    }
-    tail_selectors(w6, upper, sel_bytes, sel, late);
-    sel[30] |= late[6];
-}
-
-// One pipeline step of direct_gemm_kernel: the MFMAs of the current group
-// (weights already decoded in a_mfma, activations in LDS buffer `buf`) with the
-// decode of the next group (words u, other -> a_dec): its 32 selector dwords
-// from the tables in LDS up front, then at stage st the four weight pairs MFMA
-// step st of the following group will need.
-template <int NB, bool kMfma = true>
-__device__ __forceinline__ void direct_step(float16v (&acc)[NB], const uint32_t (&a_mfma)[32], uint32_t (&a_dec)[32],
-                                            const uint32_t (&u)[4], uint32_t other, bool upper,
-                                            const _Float16 *xb, const char *sel_bytes,
-                                            uint32_t scale_mask = 0xffffu) {
-    // scale_mask 0 turns a padding group's weights into +-0.
-    uint32_t table_hi, table_lo;
-    scale_tables((upper ? other : u[0]) & scale_mask, table_hi, table_lo);
-    uint32_t sel[32];
-#pragma unroll
-    for (int st = 0; st < 8; ++st) {
-        half8 bf[NB];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-            bf[nb] = *reinterpret_cast<const half8 *>(xb + nb * 32 * kDirectStride + st * 8);
-        if (st == 0) half_block_selectors(u, upper ? u[3] : other, upper, sel_bytes, sel);
-#pragma unroll
-        for (int p = 4 * st; p < 4 * st + 4; ++p) a_dec[p] = __builtin_amdgcn_perm(table_hi, table_lo, sel[p]);
-        if (!kMfma) continue;
-        half8 af;
-        {
-            uint4 v = {a_mfma[4 * st], a_mfma[4 * st + 1], a_mfma[4 * st + 2], a_mfma[4 * st + 3]};
-            af = *reinterpret_cast<half8 *>(&v);
-        }
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[nb], acc[nb], 0, 0, 0);
-    }
-}
-
-// MFMA steps of one group with weights already decoded (no decode).
-template <int NB>
-__device__ __forceinline__ void direct_mfma(float16v (&acc)[NB], const uint32_t (&a)[32], const _Float16 *xb) {
-#pragma unroll
-    for (int st = 0; st < 8; ++st) {
-        half8 af;
-        {
-            uint4 v = {a[4 * st], a[4 * st + 1], a[4 * st + 2], a[4 * st + 3]};
-            af = *reinterpret_cast<half8 *>(&v);
-        }
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const half8 bf = *reinterpret_cast<const half8 *>(xb + nb * 32 * kDirectStride + st * 8);
-            acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf, acc[nb], 0, 0, 0);
-        }
-    }
-}
-
 // Logical 4-half unit u of a staged activation row holds physical unit
 // direct_source_unit(u) of the group (the K order above).
 __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (u == 15 ? 30 : (u < 31 ? u - 1 : 31)); }
 
-// Three waves per SIMD (168 VGPRs at most; the two-tile form keeps one 8-byte
-// value in scratch, reloaded once per eight-group loop pass): a CU then holds
-// three workgroups, so the grid (about 2.7 workgroups per CU at the 27B
-// shapes) runs in one round.
-template <int NB, int SR>
-__global__ __launch_bounds__(kDirectThreads, 3) void direct_gemm_kernel(
-    const uint32_t *__restrict__ packed, const _Float16 *__restrict__ x, _Float16 *__restrict__ y,
-    float *__restrict__ partial, unsigned *__restrict__ counters, int M, int N, int G, int chunk_groups,
-    int k_split, int window) {
-    static_assert(SR <= 32 * NB && SR >= 8, "staged rows");
-    extern __shared__ __attribute__((aligned(16))) _Float16 xs[];  // window x SR rows x kDirectStride halves
+// ---------------------------------------------------------------------------
+// trit_gemm_kernel: y = x @ W^T for small batches (M <= 32, or 64 with two
+// MFMA tiles) of fp16, bf16 and fp32 activations.
+//
+// What bounds it: the decode. A wave turns 32 rows x one block into MFMA
+// operands while the words stream, so the loop is VALU and LDS issue, not
+// bytes (gate/up's 19.5 MB stream in 4.8 us; 21 group steps per SIMD of about
+// 95 VALU and 35 LDS instructions take about that too), and everything below
+// keeps the instructions per trit down. Measured on MI355X (us, cold weights,
+// gate/up / down / QKV), against the form it replaced, which permuted fp16
+// (t - 1) * scale weights together and took only fp16 (bf16 ran the wide form
+// after a scaling pass, fp32 the LUT23 kernel): fp16 M=8 17.9 / 20.3 / 12.8 ->
+// 14.1 / 14.3 / 9.9, M=32 20.6 / 23.6 / 15.5 -> 18.1 / 21.3 / 13.3; bf16 M=8
+// 27.2 / 34.8 / 24.6 -> 14.1 / 14.3 / 9.9; fp32 QKV M=24 41.9 -> 19.9.
+//
+// Weights never touch LDS: lane l of a wave decodes half l / 32 of the block
+// of weight row l % 32 straight into an operand of v_mfma_f32_32x32x16, in the
+// K order of the direct forms (half h: code bytes 12h .. 12h+11 as positions
+// 0..59, then four trits of code byte 24 and the tail). The trits themselves
+// are the operand: -1, 0 and +1 in the activations' MFMA type, looked up in
+// pairs (pair tables in LDS, tq1_bytes.h: two dwords per code byte pair half,
+// no permute per pair), and the block's scale multiplies the fp32 group sums,
+// acc = fma(scale, sum, acc), the LUT23 kernels' order. So one kernel serves
+// every activation type with no conversion of the weights or activations:
+//   fp16, bf16  the activations as they are (products with -1/0/+1 exact);
+//   fp32        each value as three bf16 terms (its significand's upper,
+//               middle and lower 8 bits: exact), three MFMAs per K slice.
+// The weights are the MFMA's second operand, so a lane's 16 sums belong to one
+// weight row -- its own: the scale is a per-lane scalar, an output row's
+// stores are contiguous, and only the sums of real activation rows are
+// multiplied, stored and reduced (4 of 16 up to 8 rows, 8 up to 16).
+//
+// A workgroup (4 waves, 128 weight rows) stages windows of W groups of its K
+// chunk's activations in LDS; words are requested four groups ahead across
+// windows. K is split over workgroups with the in-launch ordered reduction of
+// the LUT23 kernel (partials as 16-byte device-coherent quads, the last
+// arriver adds the chunks in order).
+// A chunk of several windows loads the next one's activations when it gets
+// there, with the CU's other workgroups at work: kept in registers from a
+// window ahead they took the kernel to two waves per SIMD or into scratch
+// (M=32, gate/up 22.5 against 21.2 us, the fused 34816 rows 42.8 / 36.8).
+// A non-finite scale: (t - 1) * scale is NaN for a zero trit, which scale *
+// sum does not give. With kTritIeeeScales (the GEMM entry points, whose other
+// forms decode weights) a wave that meets one rewrites that group's operand
+// as +-inf / NaN and scales by 1; without it (ternel_tq1_matmul's batches) the
+// result is the LUT23 kernel's fma.
+// ---------------------------------------------------------------------------
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+template <typename T>
+struct TritOperand {  // bf16 and (as three bf16 terms) fp32
+    static constexpr uint32_t kOne = 0x3f80u;
+    static constexpr int kPlanes = sizeof(T) == 4 ? 3 : 1;
+    static __device__ __forceinline__ float16v mfma(u32x4 a, u32x4 b, float16v c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                       0, 0, 0);
+    }
+};
+template <>
+struct TritOperand<_Float16> {
+    static constexpr uint32_t kOne = 0x3c00u;
+    static constexpr int kPlanes = 1;
+    static __device__ __forceinline__ float16v mfma(u32x4 a, u32x4 b, float16v c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0,
+                                                      0, 0);
+    }
+};
+
+// An fp32 value as three bf16 terms, bits in the upper half of each: hi + mid
+// + lo == v exactly (the subtractions are exact: each term takes the leading
+// 8 significand bits left). inf and NaN go in hi alone.
+__device__ __forceinline__ void split_bf16x3(float v, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+    const uint32_t u = __float_as_uint(v);
+    if ((u & 0x7f800000u) == 0x7f800000u) {
+        hi = (u & 0x007fffffu) ? u | 0x00400000u : u;
+        mid = lo = 0u;
+        return;
+    }
+    hi = u & 0xffff0000u;
+    const float r = v - __uint_as_float(hi);
+    mid = __float_as_uint(r) & 0xffff0000u;
+    lo = __float_as_uint(r - __uint_as_float(mid));
+}
+
+// Keeps every register of `sum` allocated until `after` has been computed.
+__device__ __forceinline__ void keep_live(float &after, const float16v &sum) {
+    asm volatile("" : "+v"(after) : "v"(sum));
+}
+
+// 16-bit half E of `pair` times S (4 or 8), as a table byte offset.
+template <int E, int S>
+__device__ __forceinline__ uint32_t pair_offset(uint32_t pair) {
+    uint32_t r;
+    if constexpr (E == 0)
+        asm("v_mad_u32_u16 %0, %1, %2, 0" : "=v"(r) : "v"(pair), "n"(S));
+    else
+        asm("v_mad_u32_u16 %0, %1, %2, 0 op_sel:[1,0,0,0]" : "=v"(r) : "v"(pair), "n"(S));
+    return r;
+}
+
+// One half block as MFMA operand dwords: dword q is a[q], OR late[...] for
+// dwords 5w + 2 (a code byte's fifth trit from one table, the next byte's
+// first from another) and 30.
+struct TritHalf {
+    uint32_t a[32], late[7];
+
+    __device__ __forceinline__ uint32_t dword(int q) const {
+        return q == 30 ? a[30] | late[6] : (q < 30 && q % 5 == 2 ? a[q] | late[q / 5] : a[q]);
+    }
+    // Dwords 5w .. 5w + 4 of window w = 2k + E (code bytes a = 2w, b = 2w + 1
+    // of the half) from the splits of windows 2k and 2k + 1.
+    template <int E>
+    __device__ __forceinline__ void window(const WindowSplits &s, int k, const char *tab) {
+        const int w = 2 * k + E;
+        const uint2 t27a = *reinterpret_cast<const uint2 *>(tab + pair_offset<E, 8>(s.ha) + 4 * tq1_bytes::kPairT27a);
+        const uint2 t27b = *reinterpret_cast<const uint2 *>(tab + pair_offset<E, 8>(s.lb) + 4 * tq1_bytes::kPairT27b);
+        a[5 * w] = *reinterpret_cast<const uint32_t *>(tab + pair_offset<E, 8>(s.la) + 4 * tq1_bytes::kPairT9a);
+        a[5 * w + 1] = t27a.x;
+        a[5 * w + 2] = t27a.y;
+        late[w] = t27b.x;
+        a[5 * w + 3] = t27b.y;
+        a[5 * w + 4] = *reinterpret_cast<const uint32_t *>(tab + pair_offset<E, 4>(s.hb) + 4 * tq1_bytes::kPairT9b);
+    }
+    // Dwords 30 and 31: code byte 24's first four trits in the lower half; its
+    // fifth and the tail's three in the upper.
+    __device__ __forceinline__ void tail(uint32_t w6, bool upper, const char *tab) {
+        const uint32_t mask = 0u - static_cast<uint32_t>(upper);
+        const uint32_t p24 = (w6 >> 16) & 0xffu;
+        const uint32_t t = tq1_bytes::tail_entry(w6 >> 24);
+        const uint32_t h24 = (p24 * 57u) >> 9, l24 = p24 - 9u * h24;
+        const uint32_t lead = ((8 * t + 4 * tq1_bytes::kPairT27b) & mask) | ((8 * l24 + 4 * tq1_bytes::kPairT9a) & ~mask);
+        const uint2 first = *reinterpret_cast<const uint2 *>(tab + lead);
+        const uint2 h = *reinterpret_cast<const uint2 *>(tab + 8 * h24 + 4 * tq1_bytes::kPairT27a);
+        a[30] = first.x;
+        late[6] = h.y & mask;
+        a[31] = (first.y & mask) | (h.x & ~mask);
+    }
+    // A lane whose scale is inf or NaN: the operand becomes (t - 1) * scale.
+    template <uint32_t ONE>
+    __device__ __forceinline__ void non_finite(uint32_t scale_bits) {
+        constexpr uint32_t kExp = ONE == 0x3c00u ? 0x7c007c00u : 0x7f807f80u;
+        constexpr uint32_t kLow = ONE == 0x3c00u ? 0x04000400u : 0x00800080u;  // the lowest exponent bit, set in 1
+        const uint32_t nan = (scale_bits & 0x3ffu) ? kLow >> 1 : 0u;
+        const uint32_t sign = (scale_bits & 0x8000u) ? 0x80008000u : 0u;
+#pragma unroll
+        for (int q = 0; q < 32; ++q) {
+            const uint32_t d = dword(q);
+            a[q] = (d | kExp | ((~d & kLow) >> 1) | nan) ^ sign;
+        }
+#pragma unroll
+        for (int w = 0; w < 7; ++w) late[w] = 0u;
+    }
+};
+
+constexpr int kTritGlu = 1;         // write SiLU(row 2r) * (row 2r + 1)
+constexpr int kTritIeeeScales = 2;  // zero trits of a non-finite scale are NaN
+
+// Groups staged at once: 8 of up to 16 rows, fewer of more (and of fp32's
+// three planes), so that three workgroups' windows (two of 64 rows) fit a
+// CU's LDS (M=32 in windows of 8, two workgroups: QKV 16.8 us against 14.3).
+constexpr int trit_window(int value_bytes, int staged_rows) {
+    return value_bytes == 4 ? 64 / staged_rows : (staged_rows <= 16 ? 8 : 4);
+}
+
+// Vector registers for three waves per SIMD (two for the two-tile form, whose
+// sums take 64).
+template <typename T, int SR, bool MULTI>
+__global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_kernel(
+    const uint32_t *__restrict__ packed, const T *__restrict__ x, T *__restrict__ y, float *__restrict__ partial,
+    unsigned *__restrict__ counters, int M, int N, int G, int chunk_groups, int k_split, int flags) {
+    using Op = TritOperand<T>;
+    constexpr int P = Op::kPlanes;
+    constexpr int NB = SR > 32 ? 2 : 1;
+    constexpr int W = trit_window(sizeof(T), SR);
+    constexpr int U = W > 4 ? W : 4;                 // loop body, groups (the word ring is four deep)
+    constexpr int RQ = SR >= 32 ? 4 : SR / 8;        // quads of sums per tile that belong to staged rows
+    constexpr int kVec = 16 / static_cast<int>(sizeof(T));
+    constexpr int kRowChunks = kBlockWeights / kVec;  // 16-byte chunks of a row's group
+    constexpr int kChunks = W * SR * kRowChunks / kDirectThreads;  // per thread
+    static_assert(W * SR * kRowChunks % kDirectThreads == 0, "whole chunks per thread");
+    constexpr int kPlane = W * SR * kDirectStride;   // halves
+    __shared__ __align__(16) uint16_t xs[P * kPlane];
+    __shared__ __align__(16) uint32_t pairs[tq1_bytes::kPairEntries];
     __shared__ unsigned s_last;
-    __shared__ uint32_t selectors[tq1_bytes::kSelEntries];
 
     const int tid = threadIdx.x;
-    if (tid < tq1_bytes::kSelEntries) selectors[tid] = tq1_bytes::selector_entry(tid);  // read after the first barrier
-    const char *const sel_bytes = reinterpret_cast<const char *>(selectors);
+    if (tid < tq1_bytes::kPairEntries) pairs[tid] = tq1_bytes::pair_entry(tid, Op::kOne);
+    const char *const tab = reinterpret_cast<const char *>(pairs);
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS-DMA bases go in M0
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool upper = lane >= 32;
     const int row0 = blockIdx.x * kDirectRows + wave * 32;
     const int g_begin = blockIdx.y * chunk_groups;
     const int cg = chunk_groups;
+    const int64_t K = static_cast<int64_t>(G) * kBlockWeights;
     const int direct_wave_id = (blockIdx.y * gridDim.x + blockIdx.x) * kDirectWaves + wave;
     (void)direct_wave_id;
     TQ1_PHASE(direct_wave_id, 0);  // wave start
     TQ1_PHASE_XCC(direct_wave_id);
-    const int64_t K = static_cast<int64_t>(G) * kBlockWeights;
 
-    // Rows past the padded last tile load the last padded row (discarded).
-    const int load_row = min(row0 + (lane & 31), ceil_div_dev(N, kTileRows) * kTileRows - 1);
-    const uint32_t *wrow = packed + static_cast<int64_t>(load_row / kTileRows) * G * kTileGroupWords + (load_row % kTileRows);
-    const int wfirst = (upper ? 3 : 0) * kTileRows;
-    const int wother = (upper ? 0 : 6) * kTileRows;
-    const int src_half = direct_source_unit(lane >> 1) * 4 + (lane & 1) * 2;
+    // A wave's 32 rows lie in one 64-row tile: a uniform base and a lane
+    // offset (waves past the last tile load, and discard, the last).
+    const int load_tile = min(row0 / kTileRows, ceil_div_dev(N, kTileRows) - 1);
+    const uint32_t *const tile_words = packed + (static_cast<int64_t>(load_tile) * G + g_begin) * kTileGroupWords;
+    const uint32_t wrow = static_cast<uint32_t>(row0 % kTileRows + (lane & 31)) * 4u;  // bytes
+    const uint32_t wfirst = wrow + (upper ? 3 : 0) * kTileRows * 4;
+    const uint32_t wother = wrow + (upper ? 0 : 6) * kTileRows * 4;
+    uint32_t ring[4][5];  // words of group v in ring[v % 4]: 3h .. 3h + 3 and the other end word
+    auto load_words = [&](uint32_t (&w)[5], int v) __attribute__((always_inline)) {
+        const char *const p = reinterpret_cast<const char *>(tile_words) + min(v, cg - 1) * (kTileGroupWords * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = *reinterpret_cast<const uint32_t *>(p + wfirst + j * (kTileRows * 4));
+        w[4] = *reinterpret_cast<const uint32_t *>(p + wother);
+    };
 
-    // B fragments: activation row (lane & 31) (+32 for the second tile); rows
-    // past SR read row SR - 1 (their MFMA columns are never stored).
-    const int brow = min(lane & 31, SR - 1);
-    const int bofs = brow * kDirectStride + (upper ? 64 : 0);
+    // Activations of the window at group w0 (rows past M and groups past the
+    // chunk re-read the last), as physical 16-byte chunks; written to LDS in
+    // the K order as 4-value units.
+    uint4 xc[kChunks];
+    auto load_x = [&](int w0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kChunks; ++k) {
+            const int j = tid + k * kDirectThreads;
+            const int r = j / kRowChunks, q = r / SR, m = r - q * SR;
+            xc[k] = *reinterpret_cast<const uint4 *>(x + static_cast<int64_t>(min(m, M - 1)) * K +
+                                                     static_cast<int64_t>(g_begin + min(w0 + q, cg - 1)) * kBlockWeights +
+                                                     (j % kRowChunks) * kVec);
+        }
+    };
+    auto target_unit = [](int u) { return u < 15 ? u : (u < 30 ? u + 1 : (u == 30 ? 15 : 31)); };
+    auto store_x = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kChunks; ++k) {
+            const int j = tid + k * kDirectThreads;
+            const int r = j / kRowChunks, c = j % kRowChunks;
+            uint16_t *row = xs + r * kDirectStride;
+            if constexpr (P == 1) {
+                *reinterpret_cast<uint2 *>(row + target_unit(2 * c) * 4) = uint2{xc[k].x, xc[k].y};
+                *reinterpret_cast<uint2 *>(row + target_unit(2 * c + 1) * 4) = uint2{xc[k].z, xc[k].w};
+            } else {
+                const uint32_t v[4] = {xc[k].x, xc[k].y, xc[k].z, xc[k].w};
+                uint32_t t[3][4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) split_bf16x3(__uint_as_float(v[e]), t[0][e], t[1][e], t[2][e]);
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+                    *reinterpret_cast<uint2 *>(row + p * kPlane + target_unit(c) * 4) =
+                        uint2{__builtin_amdgcn_perm(t[p][1], t[p][0], 0x07060302u),
+                              __builtin_amdgcn_perm(t[p][3], t[p][2], 0x07060302u)};
+            }
+        }
+    };
+    // Rows past SR read row SR - 1 (their sums are never stored).
+    const uint16_t *const xfrag = xs + min(lane & 31, SR - 1) * kDirectStride + (upper ? 64 : 0);
+    auto frag = [&](int slot, int p, int nb, int st) __attribute__((always_inline)) {
+        return *reinterpret_cast<const u32x4 *>(xfrag + p * kPlane + (slot * SR + nb * 32) * kDirectStride + st * 8);
+    };
 
-    float16v acc[NB];
+    float acc[NB][RQ * 4];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[nb][r] = 0.0f;
+        for (int r = 0; r < RQ * 4; ++r) acc[nb][r] = 0.0f;
+    TritHalf half;
+    float scale = 0.0f;  // of the group in `half`
 
-    constexpr int CH = 4;  // groups of words per prefetch set
-    for (int w0 = 0; w0 < cg; w0 += window) {
-        const int wn = min(window, cg - w0);
-        const int gw = g_begin + w0;
-        auto load_chunk = [&](uint32_t (&w)[CH][5], int q) {
+    // The scale of words w, with the operand of a non-finite one rewritten.
+    auto finish_decode = [&](const uint32_t (&w)[5]) __attribute__((always_inline)) {
+        const uint32_t bits = (upper ? w[4] : w[0]) & 0xffffu;
+        scale = half_bits_to_float(bits);
+        if constexpr (sizeof(T) == 2) {
+            const bool bad = (bits & 0x7c00u) == 0x7c00u;
+            if (__builtin_expect((flags & kTritIeeeScales) && __any(bad), 0)) {
+                if (bad) {
+                    half.template non_finite<Op::kOne>(bits);
+                    scale = 1.0f;
+                }
+            }
+        }
+    };
+    auto decode = [&](const uint32_t (&w)[5]) __attribute__((always_inline)) {
+        const uint32_t u[4] = {w[0], w[1], w[2], w[3]};
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const uint32_t *p = wrow + static_cast<int64_t>(gw + min(q + c, wn - 1)) * kTileGroupWords;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) w[c][j] = p[wfirst + j * kTileRows];
-                w[c][4] = p[wother];
-            }
-        };
-        auto xb = [&](int q) { return xs + q * SR * kDirectStride + bofs; };
-
-        if (w0) __syncthreads();  // every wave is done with the previous window's activations
-        // The window's activations, staged in LDS in the K order above
-        // (logical unit u of a row, 4 halves, from physical unit
-        // direct_source_unit(u); rows past M re-read row M - 1). Up to 16
-        // staged rows, 32 rows in windows of up to 4 groups and 64 in windows
-        // of up to 2 (the planner's windows there): as 16-byte physical chunks
-        // loaded into registers (8 per thread at 16 rows x 8 groups, 32 x 4 or
-        // 64 x 2) ahead of the first word set, each written to LDS after it
-        // as two 8-byte units at their K-order positions -- loads complete in
-        // order, so the writes wait for the activations only while the words
-        // are in flight. Otherwise by LDS-DMA (one padded row per instruction)
-        // waited for before any word is requested, as a second register pass
-        // would wait for the words too. The second word set is requested after
-        // the staging barrier, so no wave reaches the barrier late for issuing
-        // it behind the CU's memory queue (M=8-32, every 27B shape, 1-3 %
-        // faster on MI355X). (Measured on MI355X, gate/up: M=16 20.7 -> 19.0
-        // us and M=8 19.2 -> 18.3 us with 8-byte units in registers, 17.1 us
-        // at M=8 with 16-byte chunks; M=32 in 8-group windows 27.8 us with
-        // LDS-DMA against 32.4 with registers, 20.3 us in 4-group windows with
-        // registers.)
-        uint32_t wa[CH][5], wb[CH][5];
-        if (SR <= 16 || wn * SR * 16 <= 8 * kDirectThreads) {
-            constexpr int kUnits = 16;  // per thread
-            const int units = wn * SR * 32;
-            auto unit_source = [&](int i) {
-                const int r = i >> 5, q = r / SR, m = r - q * SR;
-                return reinterpret_cast<const uint2 *>(x + static_cast<int64_t>(min(m, M - 1)) * K +
-                                                       static_cast<int64_t>(gw + q) * kBlockWeights +
-                                                       direct_source_unit(i & 31) * 4);
-            };
-            auto unit_target = [&](int i) {
-                return reinterpret_cast<uint2 *>(xs + (i >> 5) * kDirectStride + (i & 31) * 4);
-            };
-            // Indices past the window are clamped (those threads load and write
-            // the last unit again, the same value): no load or write behind a
-            // branch, where the compiler's wait counts turn conservative.
-            const int first = min(units, kUnits * kDirectThreads);
-            // 16-byte physical chunks: chunk j is row-group j / 16, physical
-            // units 2 (j % 16) and 2 (j % 16) + 1, written to their K-order
-            // positions (the inverse of direct_source_unit).
-            auto target_unit = [](int u) { return u < 15 ? u : (u < 30 ? u + 1 : (u == 30 ? 15 : 31)); };
-            const int first_chunks = first / 2;
-            uint4 xc[kUnits / 2];
-#pragma unroll
-            for (int k = 0; k < kUnits / 2; ++k) {
-                const int j = min(tid + k * kDirectThreads, first_chunks - 1);
-                const int r = j >> 4, q = r / SR, m = r - q * SR;
-                xc[k] = *reinterpret_cast<const uint4 *>(x + static_cast<int64_t>(min(m, M - 1)) * K +
-                                                         static_cast<int64_t>(gw + q) * kBlockWeights + (j & 15) * 8);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            load_chunk(wa, 0);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = 0; k < kUnits / 2; ++k) {
-                const int j = min(tid + k * kDirectThreads, first_chunks - 1);
-                const int r = j >> 4, c = j & 15;
-                *reinterpret_cast<uint2 *>(xs + r * kDirectStride + target_unit(2 * c) * 4) = uint2{xc[k].x, xc[k].y};
-                *reinterpret_cast<uint2 *>(xs + r * kDirectStride + target_unit(2 * c + 1) * 4) = uint2{xc[k].z, xc[k].w};
-            }
-            // (Windows of more than 8 groups at 16 rows: the rest after the words.)
-            for (int i = first + tid; i < units; i += kDirectThreads) *unit_target(i) = *unit_source(i);
-        } else {
-            for (int r = wave; r < wn * SR; r += kDirectWaves) {
-                const int q = r / SR, m = r - q * SR;
-                const _Float16 *src = x + static_cast<int64_t>(min(m, M - 1)) * K +
-                                      static_cast<int64_t>(gw + q) * kBlockWeights + src_half;
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                                 (__attribute__((address_space(3))) void *)(xs + r * kDirectStride),
-                                                 4, 0, 0);
-            }
-            wait_vector_memory();
-            load_chunk(wa, 0);
+        for (int k = 0; k < 3; ++k) {
+            const WindowSplits s = window_splits(u, k);
+            half.template window<0>(s, k, tab);
+            half.template window<1>(s, k, tab);
         }
-        if (w0 == 0) TQ1_PHASE(direct_wave_id, 1);  // first window's activations staged
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-        load_chunk(wb, CH);
-        __builtin_amdgcn_sched_barrier(0);
-
-        // Pipeline over the window (no barriers): MFMAs of group q interleaved
-        // with the decode of q+1; words come in sets of four groups issued four
-        // steps before their first decode. Decoded weights alternate with
-        // period 2 and word sets with period 8, so the loop body is 8 steps and
-        // no register is copied (a copy would wait for its prefetch).
-        uint32_t a0[32], a1[32];
-        {
-            const uint32_t u[4] = {wa[0][0], wa[0][1], wa[0][2], wa[0][3]};
-            direct_step<NB, false>(acc, a1, a0, u, wa[0][4], upper, xb(0), sel_bytes);
-        }
-        auto step = [&](const uint32_t (&a_mfma)[32], uint32_t (&a_dec)[32], const uint32_t (&w)[5], int q) {
-            const uint32_t u[4] = {w[0], w[1], w[2], w[3]};
-            direct_step<NB>(acc, a_mfma, a_dec, u, w[4], upper, xb(q), sel_bytes);
-        };
-        int q = 0;
-        for (; q + 2 * CH <= wn; q += 2 * CH) {
-            step(a0, a1, wa[1], q + 0);
-            step(a1, a0, wa[2], q + 1);
-            step(a0, a1, wa[3], q + 2);
-            step(a1, a0, wb[0], q + 3);
-            // The fences keep the scheduler from sinking the prefetch toward its use.
-            __builtin_amdgcn_sched_barrier(0);
-            load_chunk(wa, q + 2 * CH);
-            __builtin_amdgcn_sched_barrier(0);
-            step(a0, a1, wb[1], q + 4);
-            step(a1, a0, wb[2], q + 5);
-            step(a0, a1, wb[3], q + 6);
-            step(a1, a0, wa[0], q + 7);
-            __builtin_amdgcn_sched_barrier(0);
-            load_chunk(wb, q + 3 * CH);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // Four groups left (a window of 4 or 8k + 4 groups): a0 holds group q
-        // decoded and wa the words of groups q .. q+3 -- prefetched by the
-        // loop above or, for a 4-group window, before it -- so they run the
-        // same pipeline.
-        if (wn - q == CH) {
-            step(a0, a1, wa[1], q + 0);
-            step(a1, a0, wa[2], q + 1);
-            step(a0, a1, wa[3], q + 2);
-            direct_mfma<NB>(acc, a1, xb(q + 3));
-            q += CH;
-        }
-        // Other remainders: a0 holds group q decoded; the next group's words
-        // are loaded where they are needed.
-        for (; q < wn; ++q) {
-            direct_mfma<NB>(acc, a0, xb(q));
-            if (q + 1 < wn) {
-                const uint32_t *p = wrow + static_cast<int64_t>(gw + q + 1) * kTileGroupWords;
-                const uint32_t u[4] = {p[wfirst], p[wfirst + kTileRows], p[wfirst + 2 * kTileRows], p[wfirst + 3 * kTileRows]};
-                direct_step<NB, false>(acc, a1, a0, u, p[wother], upper, xb(q + 1), sel_bytes);
-            }
-        }
-    }
-
-    TQ1_PHASE(direct_wave_id, 5);  // every group summed
-    // D[i][j] of a 32x32 tile sits in lane j + 32 * ((i / 4) % 2), item 4 * (i / 8) + i % 4;
-    // here i is a weight row of the wave and j an activation row.
-    if (k_split > 1) {
-        // Partials in quads, only the lanes of real activation rows: values
-        // 4q .. 4q+3 of tile nb in lane j + 32 h (j < S = min(M, 32)) sit at
-        // ((nb * 4 + q) * 2 S + h * S + j) * 4 of the (chunk, wave) region, so
-        // a lane stores and loads them with four 16-byte device-coherent (sc1)
-        // buffer accesses, each instruction covering 2 S * 16 contiguous bytes.
-        // The chunk, tile and quad offsets are wave-uniform (scalar).
-        constexpr int kDeviceCoherent = 16;  // cache policy SC1
-        const int S = min(M, 32);
-        const int frag = NB * 32 * S;
-        const int64_t chunk_stride = static_cast<int64_t>(kDirectWaves) * frag;
-        const int j = lane & 31;
-        const float *wave_base = partial + static_cast<int64_t>(blockIdx.x) * k_split * chunk_stride +
-                                 static_cast<int64_t>(wave) * frag;
-        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float *>(wave_base), 0, static_cast<int>(k_split * chunk_stride * 4), kBufferRsrcFlags);
-        // lanes past the real rows load row S - 1 again (never stored)
-        const uint32_t voff = static_cast<uint32_t>(((lane >> 5) * S + min(j, S - 1)) * 16);
-        auto value_offset = [&](int z, int nb, int q) {
-            return static_cast<int>((z * chunk_stride + (nb * 4 + q) * 2 * S * 4) * 4);
-        };
+        half.tail(upper ? w[3] : w[4], upper, tab);
+        finish_decode(w);
+    };
+    // MFMAs of the group in `half` from window slot `slot`; with DECODE, the
+    // decode of words w over the operand dwords each stage has consumed.
+    auto group = [&](int slot, const uint32_t (&w)[5], auto with_decode) __attribute__((always_inline)) {
+        constexpr bool kDecode = decltype(with_decode)::value;
+        const uint32_t u[4] = {w[0], w[1], w[2], w[3]};
+        float16v sum[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
-            if (nb * 32 + j < M)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const f32x4 v4 = {acc[nb][4 * q], acc[nb][4 * q + 1], acc[nb][4 * q + 2], acc[nb][4 * q + 3]};
+            for (int r = 0; r < 16; ++r) sum[nb][r] = 0.0f;
+        WindowSplits s;
+#pragma unroll
+        for (int st = 0; st < 8; ++st) {
+            u32x4 b[P][NB];
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) b[p][nb] = frag(slot, p, nb, st);
+            const u32x4 wt = {half.dword(4 * st), half.dword(4 * st + 1), half.dword(4 * st + 2), half.dword(4 * st + 3)};
+#pragma unroll
+            for (int p = P - 1; p >= 0; --p)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) sum[nb] = Op::mfma(b[p][nb], wt, sum[nb]);
+            if constexpr (kDecode) {
+                // window w's dwords end at 5w + 4: after the stage that reads it
+                if (st == 0) s = window_splits(u, 0);
+                if (st == 1) half.template window<0>(s, 0, tab);
+                if (st == 2) {
+                    half.template window<1>(s, 0, tab);
+                    s = window_splits(u, 1);
+                }
+                if (st == 3) half.template window<0>(s, 1, tab);
+                if (st == 4) {
+                    half.template window<1>(s, 1, tab);
+                    s = window_splits(u, 2);
+                }
+                if (st == 6) half.template window<0>(s, 2, tab);
+                if (st == 7) {
+                    half.template window<1>(s, 2, tab);
+                    half.tail(upper ? w[3] : w[4], upper, tab);
+                }
+            }
+        }
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < RQ * 4; ++r) acc[nb][r] = fmaf(scale, sum[nb][r], acc[nb][r]);
+        // All 16 sums stay live until the fmas above have waited for the last
+        // MFMA: the compiler would reuse the registers of the unused ones at
+        // once, and its hazard checks do not see the decode's inline asm
+        // write them while the MFMA still does.
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) keep_live(acc[nb][0], sum[nb]);
+        if constexpr (kDecode) finish_decode(w);
+    };
+
+    // The first window's activations, then the first four groups' words:
+    // loads complete in order, so the LDS writes wait for the activations only.
+    load_x(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) load_words(ring[v], v);
+    __builtin_amdgcn_sched_barrier(0);
+    store_x();
+    TQ1_PHASE(direct_wave_id, 1);  // first window's activations staged
+    __syncthreads();
+    decode(ring[0]);
+    load_words(ring[0], 4);
+    int q = 0;
+    for (bool more = q + 1 < cg; more;) {
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            if (!more) break;
+            group(i % W, ring[(i + 1) % 4], std::true_type{});
+            __builtin_amdgcn_sched_barrier(0);
+            load_words(ring[(i + 1) % 4], q + 5);
+            __builtin_amdgcn_sched_barrier(0);
+            ++q;
+            if constexpr (MULTI) {
+                if ((i + 1) % W == 0) {  // group q starts a window
+                    load_x(q);
+                    __syncthreads();
+                    store_x();
+                    __syncthreads();
+                }
+            }
+            more = q + 1 < cg;
+        }
+    }
+    group(q % W, ring[0], std::false_type{});
+
+    TQ1_PHASE(direct_wave_id, 5);  // every group summed
+    // Sum r of tile nb: activation row 32 nb + 8 (r / 4) + 4 (lane / 32) + r % 4,
+    // weight row row0 + lane % 32.
+    if (k_split > 1) {
+        // Partials in quads: (chunk, wave, tile, quad) runs of 64 lanes x 16
+        // bytes, the quads of real activation rows only.
+        constexpr int kDeviceCoherent = 16;  // cache policy SC1
+        const int quads = NB == 1 ? (M + 7) >> 3 : 4;
+        const int wave_bytes = NB * quads * 1024;
+        const float *base = partial + static_cast<int64_t>(blockIdx.x) * k_split * (kDirectWaves * wave_bytes / 4) +
+                            wave * (wave_bytes / 4);
+        const int chunk_bytes = kDirectWaves * wave_bytes;
+        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float *>(base), 0, k_split * chunk_bytes - wave * wave_bytes, kBufferRsrcFlags);
+        const uint32_t voff = static_cast<uint32_t>(lane * 16);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int e = 0; e < RQ; ++e)
+                if (e < quads) {
+                    const f32x4 v4 = {acc[nb][4 * e], acc[nb][4 * e + 1], acc[nb][4 * e + 2], acc[nb][4 * e + 3]};
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v4), rp, voff,
-                                                           value_offset(blockIdx.y, nb, q), kDeviceCoherent);
+                                                           static_cast<int>(blockIdx.y) * chunk_bytes +
+                                                               (nb * quads + e) * 1024,
+                                                           kDeviceCoherent);
                 }
         // Every store acknowledged at the coherence point before the arrival
         // is counted; the compiler barriers keep the stores above the wait.
@@ -1973,76 +2066,72 @@ __global__ __launch_bounds__(kDirectThreads, 3) void direct_gemm_kernel(
         __syncthreads();
         TQ1_PHASE(direct_wave_id, 7);  // arrival counted
         if (!s_last) return;
+        // The chunks in chunk order. A round trip carries a batch of chunks of
+        // one or two quads, the batch the smallest of three sizes that holds
+        // the split (a batch past the last chunk re-reads it and adds
+        // nothing): every load of this tail is latency that nothing hides,
+        // re-reads included (gate/up M=32, 5 chunks: 21.2 us with batches of
+        // 17, 18.6 with 5; down M=32, 17 chunks: 24.5 with 16, 21.8 with 17).
+        constexpr int kPair = RQ >= 2 ? 2 : 1;
+        auto reduce = [&](auto batch_size) __attribute__((always_inline)) {
+            constexpr int kBatch = decltype(batch_size)::value;
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+            for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[nb][r] = 0.0f;
-        // The chunks are added in chunk order, all loads of a batch issued
-        // before its first add (a batch past the last chunk re-reads it and
-        // adds nothing): one tile and up to 8 chunks in one batch; more chunks
-        // (down: 17) one half of the 16 values at a time with up to 17 chunks
-        // of it per batch, 34 loads in flight; two tiles 4 chunks per batch.
-        auto load4 = [&](int z, int nb, int q) {
-            return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 rp, voff, value_offset(min(z, k_split - 1), nb, q),
-                                                 kDeviceCoherent));
-        };
-        if (NB == 1 && k_split > 8) {
-            constexpr int kHalfBatch = 17;
-            for (int z0 = 0; z0 < k_split; z0 += kHalfBatch) {
+                for (int e0 = 0; e0 < RQ; e0 += kPair) {
+                    f32x4 total[kPair];
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    f32x4 v[kHalfBatch][2];
+                    for (int e = 0; e < kPair; ++e) total[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    for (int z0 = 0; z0 < k_split; z0 += kBatch) {
+                        f32x4 v[kBatch][kPair];
 #pragma unroll
-                    for (int u = 0; u < kHalfBatch; ++u)
+                        for (int z = 0; z < kBatch; ++z)
 #pragma unroll
-                        for (int q = 0; q < 2; ++q) v[u][q] = load4(z0 + u, 0, 2 * h + q);
+                            for (int e = 0; e < kPair; ++e)
+                                v[z][e] = __builtin_bit_cast(
+                                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               rp, voff,
+                                               min(z0 + z, k_split - 1) * chunk_bytes +
+                                                   (nb * quads + min(e0 + e, quads - 1)) * 1024,
+                                               kDeviceCoherent));
 #pragma unroll
-                    for (int u = 0; u < kHalfBatch; ++u)
-                        if (z0 + u < k_split)
+                        for (int z = 0; z < kBatch; ++z)
+                            if (z0 + z < k_split)
 #pragma unroll
-                            for (int q = 0; q < 2; ++q)
+                                for (int e = 0; e < kPair; ++e) total[e] += v[z][e];
+                    }
 #pragma unroll
-                                for (int e = 0; e < 4; ++e) acc[0][8 * h + 4 * q + e] += v[u][q][e];
+                    for (int e = 0; e < kPair; ++e)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) acc[nb][4 * (e0 + e) + c] = total[e][c];
                 }
-            }
-        } else {
-            constexpr int kBatch = NB == 1 ? 8 : 4;
-            for (int z0 = 0; z0 < k_split; z0 += kBatch) {
-                f32x4 v[kBatch][NB][4];
-#pragma unroll
-                for (int u = 0; u < kBatch; ++u)
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) v[u][nb][q] = load4(z0 + u, nb, q);
-#pragma unroll
-                for (int u = 0; u < kBatch; ++u)
-                    if (z0 + u < k_split)
-#pragma unroll
-                        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) acc[nb][4 * q + e] += v[u][nb][q][e];
-            }
-        }
+        };
+        if (k_split <= 5)
+            reduce(std::integral_constant<int, 5>{});
+        else if (k_split <= 10)
+            reduce(std::integral_constant<int, 10>{});
+        else
+            reduce(std::integral_constant<int, 17>{});
         if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         TQ1_PHASE(direct_wave_id, 8);  // fix-up sums done
     }
+    const int n = row0 + (lane & 31);
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        const int m = nb * 32 + (lane & 31);
-        if (m >= M) continue;
-        _Float16 *yrow = y + static_cast<int64_t>(m) * N;
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int n = row0 + 8 * q + 4 * (lane >> 5);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (n + e < N) yrow[n + e] = static_cast<_Float16>(acc[nb][4 * q + e]);
+        for (int r = 0; r < RQ * 4; ++r) {
+            const int m = nb * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            const T own = from_f32<T>(acc[nb][r]);
+            if (flags & kTritGlu) {
+                // Rows 2r and 2r + 1, a gate and its up, sit in adjacent lanes
+                // (every lane takes part in the exchange).
+                const float partner = __shfl_xor(to_f32<T>(own), 1, 64);
+                if (m < M && n < N && (lane & 1) == 0)
+                    y[static_cast<int64_t>(m) * (N / 2) + n / 2] = swiglu_pair<T>(own, from_f32<T>(partner));
+            } else if (m < M && n < N) {
+                y[static_cast<int64_t>(m) * N + n] = own;
+            }
         }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -3277,47 +3366,71 @@ int launch_gemm(const uint32_t *packed, const void *x, void *y, int64_t M, int64
 constexpr int64_t kDirectMaxBatch = 64;
 // Auto split: at least this many workgroups (4 waves each) to fill 256 CUs twice.
 constexpr int64_t kDirectTargetWorkgroups = 512;
-
-struct DirectPlan {
-    int nb;
-    int staged_rows;
-    int k_split;
-    int chunk_groups;
-    int window;  // groups of activations staged in LDS at once
-    int64_t row_blocks;
-    size_t lds_bytes;
-    size_t partial_bytes;
-};
+// Fewer than this many workgroups of 8-group chunks: 4-group chunks.
+constexpr int64_t kDirectMinWorkgroups = 224;
 
 int direct_staged_rows(int64_t M) { return M <= 8 ? 8 : (M <= 16 ? 16 : (M <= 32 ? 32 : 64)); }
 
-int plan_direct(int64_t M, int64_t rows, int64_t columns, int k_split, DirectPlan *plan) {
+// The trit kernel (trit_gemm_kernel): at most 64 rows of fp16 and bf16
+// activations, 32 of fp32, in one launch.
+struct TritPlan {
+    int staged_rows;
+    int k_split;
+    int chunk_groups;
+    int64_t row_blocks;
+    int64_t launch_rows;  // activation rows per launch
+    size_t partial_bytes;
+};
+
+// Split partials of one launch, at most: of the GEMM entry points, and of
+// ternel_tq1_matmul, whose split also has to fit the static scratch of its
+// workspace-free twin.
+constexpr int64_t kTritPartialBytes = int64_t{64} << 20;
+constexpr int64_t kTritMatmulPartialBytes = int64_t{16} << 20;
+
+// batches: a batch past one launch's rows runs as several launches of nearly
+// equal size (ternel_tq1_matmul); otherwise it is refused.
+int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, TritPlan *plan, bool batches = false) {
     const int64_t G = columns / kBlockWeights;
-    if (M > kDirectMaxBatch)
+    const bool f32 = dtype == TERNEL_TQ1_F32;
+    const int64_t most = f32 ? 32 : kDirectMaxBatch;
+    if (M > most && !batches)
         return fail(TERNEL_TQ1_EINVAL, "the direct-fragment form takes at most %lld activation rows, got %lld",
-                    static_cast<long long>(kDirectMaxBatch), static_cast<long long>(M));
-    plan->nb = M > 32 ? 2 : 1;
-    plan->staged_rows = direct_staged_rows(M);
+                    static_cast<long long>(most), static_cast<long long>(M));
+    plan->launch_rows = ceil_div(M, ceil_div(M, most));
+    const int64_t m = plan->launch_rows;
+    plan->staged_rows = direct_staged_rows(m);
     plan->row_blocks = ceil_div(rows, kDirectRows);
+    const int64_t quads = plan->staged_rows > 32 ? 8 : ceil_div(m, 8);
+    const int64_t split_bytes = plan->row_blocks * kDirectWaves * quads * 1024;
+    const int64_t most_bytes = batches ? kTritMatmulPartialBytes : kTritPartialBytes;
     if (k_split < 0) return fail(TERNEL_TQ1_EINVAL, "k split must be positive, got %d", k_split);
     if (k_split == 0) {
-        // Measured on MI355X: chunks of a multiple of 8 groups keep the whole
-        // K chunk in the 8-step pipeline; take the smallest such split that
-        // reaches the workgroup target, else the largest such split. At 32
-        // and 64 staged rows chunks of a multiple of 4 qualify too, whose last
-        // four groups run the same pipeline (QKV and O at M=32 then run 640
-        // workgroups instead of 320: 16.9 and 17.2 us against 18.4 and 18.3,
-        // measured with 8-group windows; at M=40-64 QKV 20.7-22.6 us against
-        // 23.2-25.2, O 22.8-24.8 against 24.1-26.0); at up to 16 rows 4-group
-        // chunks measured slower.
-        const int64_t granule = plan->staged_rows >= 32 ? 4 : 8;
-        int best = 0;
-        for (int64_t k = 1; k <= G; ++k) {
-            if (G % k || (G / k) % granule) continue;
-            best = static_cast<int>(k);
-            if (plan->row_blocks * k >= kDirectTargetWorkgroups) break;
+        // The smallest split into chunks of a multiple of `granule` groups
+        // that reaches the workgroup target, else the largest such split.
+        // Chunks of 8 amortise a workgroup's start and its share of the
+        // reduction best where they still give about one workgroup per CU
+        // (M=8, us, 8 / 4 groups: out_proj, 240 workgroups, 8.7 / 8.9; QKV,
+        // 320, 9.9 / 10.5), chunks of 4 where they do not (4096 square, 128:
+        // 7.8 / 7.0; k_proj, 40: 7.2 / 6.2; 2 groups: 8.3, 7.9) and at 17-32
+        // rows, whose window is 4 groups (QKV M=32 13.8 / 13.5).
+        auto widest = [&](int64_t granule) {
+            int best = 0;
+            for (int64_t k = 1; k <= G; ++k) {
+                if (G % k || (G / k) % granule) continue;
+                if (k > 1 && (k * split_bytes > most_bytes || plan->row_blocks > kUsableCounters)) break;
+                best = static_cast<int>(k);
+                if (plan->row_blocks * k >= kDirectTargetWorkgroups) break;
+            }
+            return best;
+        };
+        int best = plan->staged_rows == 32 ? 0 : widest(8);
+        if (plan->row_blocks * best < kDirectMinWorkgroups) best = std::max(best, widest(4));
+        if (!best) {
+            best = largest_divisor_split(G, plan->row_blocks, kDirectTargetWorkgroups);
+            if (best * split_bytes > most_bytes || plan->row_blocks > kUsableCounters) best = 1;
         }
-        k_split = best ? best : largest_divisor_split(G, plan->row_blocks, kDirectTargetWorkgroups);
+        k_split = best;
     }
     if (G % k_split)
         return fail(TERNEL_TQ1_EINVAL, "k split %d does not divide the tensor's %lld groups per row", k_split,
@@ -3328,55 +3441,59 @@ int plan_direct(int64_t M, int64_t rows, int64_t columns, int k_split, DirectPla
                     static_cast<long long>(plan->row_blocks), kUsableCounters);
     plan->k_split = k_split;
     plan->chunk_groups = static_cast<int>(G / k_split);
-    const size_t group_bytes = static_cast<size_t>(plan->staged_rows) * kDirectStride * sizeof(_Float16);
-    int window = static_cast<int>(kDirectLdsBytes / group_bytes);
-    // Windows of 34.8 KiB of activations: three workgroups per CU, and the
-    // window fits the register staging. 32 staged rows: 4 groups, measured on
-    // MI355X at M=17-32 gate/up 19.2-20.7 us against 26.2-26.9 in 8-group
-    // windows, down 20.7-22.5 against 27.5-28.8, QKV and O 13.7-15.5 against
-    // 15.3-17.1. Two tiles (64 staged rows): 2 groups, at M=40-64 gate/up
-    // 31.6-32.8 us against 38.2-39.5 in 4-group windows with two workgroups
-    // per CU (and 53.0 at M=40 in 8-group windows, one per CU), down
-    // 33.7-35.5 against 40.7-43.1, QKV and O 23.2-25.9 against 24.9-27.2.
-    if (plan->staged_rows == 32 && window > 4) window = 4;
-    if (plan->nb == 2 && window > 2) window = 2;
-    if (window >= plan->chunk_groups)
-        window = plan->chunk_groups;
-    else if (window >= 8)
-        window -= window % 8;
-    plan->window = window;
-    plan->lds_bytes = static_cast<size_t>(window) * group_bytes;
-    // Partials of the real activation columns only (at most 32 per tile).
-    plan->partial_bytes = k_split > 1 ? static_cast<size_t>(k_split) * plan->row_blocks * kDirectRows *
-                                            std::min<int64_t>(M, 32) * plan->nb * sizeof(float)
-                                      : 0;
+    plan->partial_bytes = k_split > 1 ? static_cast<size_t>(k_split) * split_bytes : 0;
     return TERNEL_TQ1_OK;
 }
 
-template <int NB, int SR>
-int launch_direct_kernel(const uint32_t *packed, const void *x, void *y, int64_t M, int64_t rows, int G,
-                         const DirectPlan &plan, float *partial, unsigned *counters, hipStream_t stream) {
-    int rc = ensure_lds_attribute(reinterpret_cast<const void *>(&direct_gemm_kernel<NB, SR>), kDirectLdsBytes);
-    if (rc != TERNEL_TQ1_OK) return rc;
+size_t trit_workspace_bytes(const TritPlan &plan) { return plan.k_split > 1 ? kPartialOffset + plan.partial_bytes : 0; }
+
+template <typename T, int SR>
+void launch_trit_kernel(const uint32_t *packed, const T *x, T *y, int64_t M, int64_t rows, int G, const TritPlan &plan,
+                        float *partial, unsigned *counters, int flags, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>(plan.row_blocks), static_cast<unsigned>(plan.k_split));
-    hipLaunchKernelGGL((direct_gemm_kernel<NB, SR>), grid, dim3(kDirectThreads), plan.lds_bytes, stream, packed,
-                       static_cast<const _Float16 *>(x), static_cast<_Float16 *>(y), partial, counters,
-                       static_cast<int>(M), static_cast<int>(rows), G, plan.chunk_groups, plan.k_split, plan.window);
-    TQ1_LAUNCH_CHECK();
-    return TERNEL_TQ1_OK;
+    if (plan.chunk_groups > trit_window(sizeof(T), SR))
+        hipLaunchKernelGGL((trit_gemm_kernel<T, SR, true>), grid, dim3(kDirectThreads), 0, stream, packed, x, y, partial,
+                           counters, static_cast<int>(M), static_cast<int>(rows), G, plan.chunk_groups, plan.k_split,
+                           flags);
+    else
+        hipLaunchKernelGGL((trit_gemm_kernel<T, SR, false>), grid, dim3(kDirectThreads), 0, stream, packed, x, y, partial,
+                           counters, static_cast<int>(M), static_cast<int>(rows), G, plan.chunk_groups, plan.k_split,
+                           flags);
 }
 
-int launch_direct(const uint32_t *packed, const void *x, void *y, int64_t M, int64_t rows, int64_t columns,
-                  const DirectPlan &plan, void *ws, hipStream_t stream) {
+template <typename T>
+int launch_trit_typed(const uint32_t *packed, const void *x, void *y, int64_t M, int64_t rows, int64_t columns,
+                      const TritPlan &plan, void *ws, hipStream_t stream, int flags) {
     unsigned *counters = plan.k_split > 1 ? static_cast<unsigned *>(ws) : nullptr;
     float *partial =
         plan.k_split > 1 ? reinterpret_cast<float *>(static_cast<char *>(ws) + kPartialOffset) : nullptr;
     const int G = static_cast<int>(columns / kBlockWeights);
-    switch (plan.staged_rows) {
-        case 8: return launch_direct_kernel<1, 8>(packed, x, y, M, rows, G, plan, partial, counters, stream);
-        case 16: return launch_direct_kernel<1, 16>(packed, x, y, M, rows, G, plan, partial, counters, stream);
-        case 32: return launch_direct_kernel<1, 32>(packed, x, y, M, rows, G, plan, partial, counters, stream);
-        default: return launch_direct_kernel<2, 64>(packed, x, y, M, rows, G, plan, partial, counters, stream);
+    const int64_t out_width = (flags & kTritGlu) ? rows / 2 : rows;
+    for (int64_t m0 = 0; m0 < M; m0 += plan.launch_rows) {
+        const int64_t m = std::min(plan.launch_rows, M - m0);
+        const T *xm = static_cast<const T *>(x) + m0 * columns;
+        T *ym = static_cast<T *>(y) + m0 * out_width;
+        switch (plan.staged_rows) {
+            case 8: launch_trit_kernel<T, 8>(packed, xm, ym, m, rows, G, plan, partial, counters, flags, stream); break;
+            case 16: launch_trit_kernel<T, 16>(packed, xm, ym, m, rows, G, plan, partial, counters, flags, stream); break;
+            case 32: launch_trit_kernel<T, 32>(packed, xm, ym, m, rows, G, plan, partial, counters, flags, stream); break;
+            default:
+                if constexpr (sizeof(T) == 2)
+                    launch_trit_kernel<T, 64>(packed, xm, ym, m, rows, G, plan, partial, counters, flags, stream);
+                break;
+        }
+        TQ1_LAUNCH_CHECK();
+    }
+    return TERNEL_TQ1_OK;
+}
+
+// x is 16-byte aligned (columns is a multiple of 128, so every row is).
+int launch_trit(const uint32_t *packed, const void *x, void *y, int64_t M, int64_t rows, int64_t columns, int dtype,
+                const TritPlan &plan, void *ws, hipStream_t stream, int flags) {
+    switch (dtype) {
+        case TERNEL_TQ1_F16: return launch_trit_typed<_Float16>(packed, x, y, M, rows, columns, plan, ws, stream, flags);
+        case TERNEL_TQ1_BF16: return launch_trit_typed<bf16_t>(packed, x, y, M, rows, columns, plan, ws, stream, flags);
+        default: return launch_trit_typed<float>(packed, x, y, M, rows, columns, plan, ws, stream, flags);
     }
 }
 
@@ -3526,9 +3643,10 @@ int launch_wide(const uint32_t *packed, const void *x, void *y, const WidePlan &
 // against 58.1 the other way). The tile form also serves a fixed K split above
 // 32 rows and rows too long for the wide form's 32-bit buffer offsets.
 constexpr int64_t kAutoDirectMaxBatch = 32;
-constexpr int64_t kAutoDirectMaxBatchSmall = 48;
+constexpr int64_t kAutoDirectMaxBatchSmall = 64;
 constexpr int64_t kAutoSmallMatrixBytes = 16ll << 20;
 constexpr int64_t kAutoWideMaxBatch = 64;
+constexpr int64_t kTritBf16MatrixBytes = 24ll << 20;
 int wide_blocks(int64_t M, int64_t tiles_n, int64_t groups, int64_t cus);
 int device_cu_count();
 int resolve_gemm_form(int64_t M, int64_t rows, int64_t columns, int form, int k_split) {
@@ -3572,6 +3690,37 @@ bool linear_uses_lut(int64_t M, int64_t rows, int64_t columns, int dtype) {
 // LUT23 kernel: bf16 activations run the wide form.
 int linear_gemm_form(int64_t M, int64_t rows, int64_t columns, int dtype) {
     return dtype == TERNEL_TQ1_BF16 ? TERNEL_TQ1_GEMM_WIDE : TERNEL_TQ1_GEMM_AUTO;
+}
+
+// The trit kernel runs the direct form (fp16), and in the wide form's place the
+// bf16 batches it is faster for.
+bool gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int form) {
+    if (form == TERNEL_TQ1_GEMM_DIRECT) return true;
+    if (dtype != TERNEL_TQ1_BF16 || form != TERNEL_TQ1_GEMM_WIDE) return false;
+    WidePlan wide;  // what the wide form refuses is left for it to refuse
+    return (M <= kAutoDirectMaxBatch ||
+            (M <= kDirectMaxBatch && rows * (columns / kBlockWeights) * kBlockBytes < kTritBf16MatrixBytes)) &&
+           plan_wide(M, rows, columns, 0, &wide) == TERNEL_TQ1_OK;
+}
+
+// ternel_tq1_matmul's batches with the configuration left automatic: the trit
+// kernel decodes a weight once per batch where the LUT23 kernel looks it up
+// once per vector. Measured on MI355X (us, LUT23 / trit):
+//   fp16 and bf16, M=2: gate/up 13.3 / 12.5, 4096 square 7.4 / 7.0, k_proj
+//   6.7 / 6.1, but QKV 8.8 / 9.4, out_proj 8.1 / 8.8 (matrices of 4-12 MB);
+//   M=3: gate/up 16.0 / 12.1, QKV 9.8 / 9.4, out_proj 9.2 / 8.7, 4096 square
+//   7.7 / 7.0; a 48-row matrix (one row block) 5.2 / 5.4 at M=3, 5.7 / 5.5 at 8.
+//   fp32 (three MFMAs per K slice): gate/up M=4 19.2 / 19.4, M=6 25.9 / 20.0;
+//   QKV M=4 10.9 / 13.9, M=6 14.7 / 13.8; out_proj M=6 12.2 / 11.6; 4096
+//   square M=8 9.8 / 10.7; k_proj M=8 8.1 / 10.3. The LUT23 kernel's time per
+//   vector grows with the matrix and the trit kernel's fixed cost does not, so
+//   the line is a product of both.
+bool matmul_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int batch_tile, int k_split) {
+    if (batch_tile != 0 || k_split != 0 || M < 2) return false;
+    const int64_t bytes = rows * (columns / kBlockWeights) * kBlockBytes;
+    if (dtype == TERNEL_TQ1_F32) return M >= 4 && (M - 2) * (bytes + (1 << 19)) >= 30 << 20;
+    if (rows <= kDirectRows) return M >= 8;
+    return M >= 3 || bytes < 4 << 20 || bytes >= 12 << 20;
 }
 
 int check_packed_pointer(const void *packed) {
@@ -3632,6 +3781,7 @@ int launch_get_rows(const uint32_t *table, int64_t rows, int64_t columns, const 
 // per device by noalloc_scratch().
 constexpr int64_t kNoAllocPartialBytes = int64_t{16} << 20;
 constexpr size_t kNoAllocScratchBytes = kPartialOffset + kNoAllocPartialBytes;
+static_assert(kTritMatmulPartialBytes <= kNoAllocPartialBytes, "the trit kernel's split fits the scratch");
 static __device__ __align__(256) unsigned scratch[kNoAllocScratchBytes / sizeof(unsigned)];
 
 constexpr int kScratchDevices = 64;
@@ -3857,7 +4007,15 @@ size_t ternel_tq1_matmul_workspace_bytes(int64_t M, int64_t rows, int64_t column
     }
     LutPlan plan;
     if (plan_lut(M, rows, columns, batch_tile, k_split, &plan) != TERNEL_TQ1_OK) return 0;
-    return plan.counter_bytes + plan.partial_bytes;
+    size_t need = plan.counter_bytes + plan.partial_bytes;
+    TritPlan trit;  // the workspace of whichever kernel runs (unaligned activations take the LUT23 kernel)
+    if (matmul_uses_trit(M, rows, columns, TERNEL_TQ1_F32, batch_tile, k_split) &&
+        plan_trit(M, rows, columns, TERNEL_TQ1_F32, 0, &trit, true) == TERNEL_TQ1_OK)
+        need = std::max(need, trit_workspace_bytes(trit));
+    if (matmul_uses_trit(M, rows, columns, TERNEL_TQ1_F16, batch_tile, k_split) &&
+        plan_trit(M, rows, columns, TERNEL_TQ1_F16, 0, &trit, true) == TERNEL_TQ1_OK)
+        need = std::max(need, trit_workspace_bytes(trit));
+    return need;
 }
 
 int ternel_tq1_matmul(const uint32_t *packed, const void *x, void *y, int64_t M, int64_t rows, int64_t columns,
@@ -3884,6 +4042,17 @@ int ternel_tq1_matmul(const uint32_t *packed, const void *x, void *y, int64_t M,
             default:
                 return launch_strip<float>(packed, x, y, geo, s, false, ws);
         }
+    }
+    if (matmul_uses_trit(M, rows, columns, dtype, batch_tile, k_split) && !(reinterpret_cast<uintptr_t>(x) & 15u)) {
+        TritPlan trit;
+        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true)) != TERNEL_TQ1_OK) return rc;
+        if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
+        if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
+        const size_t need = trit_workspace_bytes(trit);
+        if (need && (!ws || ws_bytes < need))
+            return fail(TERNEL_TQ1_EINVAL, "workspace of %zu bytes is smaller than the %zu the split needs", ws_bytes,
+                        need);
+        return launch_trit(packed, x, y, M, rows, columns, dtype, trit, ws, static_cast<hipStream_t>(stream), 0);
     }
     LutPlan plan;
     if ((rc = plan_lut(M, rows, columns, batch_tile, k_split, &plan)) != TERNEL_TQ1_OK) return rc;
@@ -3929,6 +4098,16 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
                 return launch_strip<float>(packed, x, y, geo, s, false, ws);
         }
     }
+    if (matmul_uses_trit(M, rows, columns, dtype, batch_tile, k_split) && !(reinterpret_cast<uintptr_t>(x) & 15u)) {
+        TritPlan trit;  // its partials fit the scratch
+        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true)) != TERNEL_TQ1_OK) return rc;
+        if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
+        if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        void *ws = nullptr;
+        if (trit.k_split > 1 && (rc = noalloc_scratch(s, &ws)) != TERNEL_TQ1_OK) return rc;
+        return launch_trit(packed, x, y, M, rows, columns, dtype, trit, ws, s, 0);
+    }
     LutPlan plan;
     if ((rc = plan_lut(M, rows, columns, batch_tile, k_split, &plan, kNoAllocPartialBytes)) != TERNEL_TQ1_OK)
         return rc;
@@ -3958,14 +4137,18 @@ size_t ternel_tq1_gemm_workspace_bytes(int64_t M, int64_t rows, int64_t columns,
     if (check_geometry(M, rows, columns) != TERNEL_TQ1_OK) return 0;
     form = resolve_gemm_form(M, rows, columns, form, k_split);
     if (form == TERNEL_TQ1_GEMM_DIRECT) {
-        DirectPlan direct;
-        if (plan_direct(M, rows, columns, k_split, &direct) != TERNEL_TQ1_OK) return 0;
-        return direct.k_split > 1 ? kPartialOffset + direct.partial_bytes : 0;
+        TritPlan trit;
+        return plan_trit(M, rows, columns, TERNEL_TQ1_F16, k_split, &trit) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
     }
     if (form == TERNEL_TQ1_GEMM_WIDE) {
         WidePlan wide;
         if (plan_wide(M, rows, columns, k_split, &wide) != TERNEL_TQ1_OK) return 0;
-        return kPartialOffset + wide.partial_bytes + wide.xp_bytes;
+        TritPlan trit;
+        size_t small = 0;  // what a bf16 batch of this size uses
+        if (gemm_uses_trit(M, rows, columns, TERNEL_TQ1_BF16, form) &&
+            plan_trit(M, rows, columns, TERNEL_TQ1_BF16, 0, &trit) == TERNEL_TQ1_OK)
+            small = trit_workspace_bytes(trit);
+        return std::max(kPartialOffset + wide.partial_bytes + wide.xp_bytes, small);
     }
     if (form != TERNEL_TQ1_GEMM_TILE) return 0;
     GemmPlan plan;
@@ -3992,17 +4175,19 @@ int ternel_tq1_gemm(const uint32_t *packed, const void *x, void *y, int64_t M, i
         form = TERNEL_TQ1_GEMM_WIDE;
     }
     form = resolve_gemm_form(M, rows, columns, form, k_split);
-    if (form == TERNEL_TQ1_GEMM_DIRECT) {
-        DirectPlan direct;
-        if ((rc = plan_direct(M, rows, columns, k_split, &direct)) != TERNEL_TQ1_OK) return rc;
+    if (gemm_uses_trit(M, rows, columns, dtype, form)) {
+        TritPlan trit;
+        if ((rc = plan_trit(M, rows, columns, dtype, form == TERNEL_TQ1_GEMM_WIDE ? 0 : k_split, &trit)) != TERNEL_TQ1_OK)
+            return rc;
         if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
         if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
         if (reinterpret_cast<uintptr_t>(x) & 15u) return fail(TERNEL_TQ1_EINVAL, "activations must be 16-byte aligned");
-        const size_t need = direct.k_split > 1 ? kPartialOffset + direct.partial_bytes : 0;
+        const size_t need = trit_workspace_bytes(trit);
         if (need && (!ws || ws_bytes < need))
             return fail(TERNEL_TQ1_EINVAL, "workspace of %zu bytes is smaller than the %zu the split needs", ws_bytes,
                         need);
-        return launch_direct(packed, x, y, M, rows, columns, direct, ws, static_cast<hipStream_t>(stream));
+        return launch_trit(packed, x, y, M, rows, columns, dtype, trit, ws, static_cast<hipStream_t>(stream),
+                           kTritIeeeScales);
     }
     if (form == TERNEL_TQ1_GEMM_WIDE) {
         WidePlan wide;
@@ -4077,11 +4262,25 @@ int ternel_tq1_linear_kernel(int64_t M, int64_t rows, int64_t columns, int dtype
     return resolve_gemm_form(M, rows, columns, linear_gemm_form(M, rows, columns, dtype), 0);
 }
 
+// Whether the fused SwiGLU's GEMM is the trit kernel.
+static bool swiglu_gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype) {
+    return gemm_uses_trit(M, rows, columns, dtype,
+                          resolve_gemm_form(M, rows, columns, linear_gemm_form(M, rows, columns, dtype), 0));
+}
+
 size_t ternel_tq1_swiglu_workspace_bytes(int64_t M, int64_t rows, int64_t columns, int dtype) {
     if (check_geometry(M, rows, columns) != TERNEL_TQ1_OK || rows % 2) return 0;
-    if (linear_uses_lut(M, rows, columns, dtype))
-        return ternel_tq1_matmul_workspace_bytes(M, rows, columns, uses_strip_gemv(M, 0, 0, rows, columns, false) ? 0 : 1,
-                                                 0);
+    TritPlan trit;
+    if (linear_uses_lut(M, rows, columns, dtype)) {
+        const size_t lut = ternel_tq1_matmul_workspace_bytes(
+            M, rows, columns, uses_strip_gemv(M, 0, 0, rows, columns, false) ? 0 : 1, 0);
+        return matmul_uses_trit(M, rows, columns, dtype, 0, 0) &&
+                       plan_trit(M, rows, columns, dtype, 0, &trit, true) == TERNEL_TQ1_OK
+                   ? std::max(lut, trit_workspace_bytes(trit))
+                   : lut;
+    }
+    if (swiglu_gemm_uses_trit(M, rows, columns, dtype))
+        return plan_trit(M, rows, columns, dtype, 0, &trit) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
     return swiglu_pairs_offset(M, rows, columns, dtype) + static_cast<size_t>(M) * rows * sizeof(_Float16);
 }
 
@@ -4108,6 +4307,21 @@ int ternel_tq1_swiglu(const uint32_t *packed, const void *x, void *z, int64_t M,
             default:
                 return launch_strip<float>(packed, x, z, geo, s, true);
         }
+    }
+    // The trit kernel writes SiLU(g) * u itself.
+    const bool lut = linear_uses_lut(M, rows, columns, dtype);
+    const bool matmul_trit =
+        lut && matmul_uses_trit(M, rows, columns, dtype, 0, 0) && !(reinterpret_cast<uintptr_t>(x) & 15u);
+    if (matmul_trit || (!lut && swiglu_gemm_uses_trit(M, rows, columns, dtype))) {
+        TritPlan trit;
+        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, matmul_trit)) != TERNEL_TQ1_OK) return rc;
+        if (reinterpret_cast<uintptr_t>(x) & 15u) return fail(TERNEL_TQ1_EINVAL, "activations must be 16-byte aligned");
+        const size_t need = trit_workspace_bytes(trit);
+        if (need && (!ws || ws_bytes < need))
+            return fail(TERNEL_TQ1_EINVAL, "workspace of %zu bytes is smaller than the %zu the split needs", ws_bytes,
+                        need);
+        return launch_trit(packed, x, z, M, rows, columns, dtype, trit, ws, s,
+                           kTritGlu | (matmul_trit ? 0 : kTritIeeeScales));
     }
     if (linear_uses_lut(M, rows, columns, dtype)) {
         LutPlan plan;

@@ -98,7 +98,7 @@ class GemmConfig:
     decodes straight into MFMA operand registers (at most 64 activation rows),
     ``"wide"`` decodes into the operand registers of 256-row output tiles (32
     to 256 activation rows wide) split stream-K over the CUs (prefill; K split
-    0 or 1), ``"auto"`` takes ``"direct"`` up to 32 rows (48 for matrices under
+    0 or 1), ``"auto"`` takes ``"direct"`` up to 32 rows (64 for matrices under
     16 MiB of packed weights), ``"wide"`` up to 64 and, above, ``"wide"`` when
     it has enough tiles (CUs/4) or work per CU (15 steps) for its stream-K
     reduction to pay, ``"tile"`` otherwise (and, above 32 rows, whenever a K
@@ -379,11 +379,10 @@ def tq1_gemm_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTenso
                    config: GemmConfig | None = None) -> torch.Tensor:
     """``x @ W.T`` on the MFMA kernels (reference tq1_gemm, kernels.py:1287-1357).
 
-    The matrix cores take fp16 operands (weights are exact in fp16). fp16
-    activations run the form ``config`` names; bf16 ones run the wide form,
-    each row scaled by a power of two into fp16's range (exact: bf16's
-    significand fits fp16's) and the fp32 sums scaled back and rounded once to
-    bf16. fp32 activations -- whose significand fp16 would not hold -- and bf16
+    fp16 activations run the form ``config`` names. bf16 ones run on bf16
+    operands in small batches and the wide form above them, each row scaled by
+    a power of two into fp16's range (exact: bf16's significand fits fp16's)
+    and the fp32 sums scaled back and rounded once to bf16. fp32 activations -- whose significand fp16 would not hold -- and bf16
     ones with a fixed K split run through the LUT23 kernel, which computes in
     fp32 from the activations as given."""
     config = config or GemmConfig()

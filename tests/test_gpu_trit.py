@@ -1,0 +1,96 @@
+"""The trit kernel (small batches of fp16, bf16 and fp32 activations) against the fp64 oracle.
+
+Shapes sit where it can go wrong: row counts that are no multiple of a wave's
+32 or a workgroup's 128 rows, group counts below, at and past its windows (1,
+5, 9 and 17 groups unsplit, 40 split), batches on both sides of its 8-, 16-, 32-
+and 64-row tiles, a batch of several launches. Products of an activation with
+-1, 0 or +1 are exact (fp32 as three bf16 terms), so an output is held to the
+fp32 summation bound plus one rounding to its type.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import tq1_oracle as O
+from tests.gpu_util import layout, pack, random_blocks, to_dev
+from ternel_amd.kernels import tq1_linear_words, tq1_matmul_words, tq1_swiglu_words
+
+pytestmark = pytest.mark.gpu
+
+ROUNDOFF = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}
+
+
+def activations(batch: int, columns: int, dtype: torch.dtype, seed: int) -> torch.Tensor:
+    rng = np.random.default_rng(seed)
+    x = rng.normal(0.0, 1.0, size=(batch, columns))
+    if dtype != torch.float16:
+        x *= 10.0 ** rng.integers(-6, 7, size=columns)  # far past fp16's range
+    return to_dev(x.astype(np.float32)).to(dtype)
+
+
+def bound(x: np.ndarray, blocks: np.ndarray, want: np.ndarray, dtype: torch.dtype) -> np.ndarray:
+    rows, groups, _ = blocks.shape
+    weights = O.dense_weights(blocks, rows=rows, columns=groups * 128)
+    sums = (128 + groups) * float(np.finfo(np.float32).eps) * (np.abs(x) @ np.abs(weights).T)
+    return sums + ROUNDOFF[dtype] * (np.abs(want) + sums) + 2.0 ** -25 * (dtype == torch.float16)
+
+
+SHAPES = ((130, 128), (300, 640), (257, 1152), (96, 2176), (1024, 5120))
+CASES = [(dtype, rows, columns, batch) for dtype in (torch.float16, torch.bfloat16)
+         for rows, columns in SHAPES for batch in (5, 8, 9, 17, 32, 33, 64)]
+# fp32: matrices large enough for the trit kernel at each tile width, and batches of several launches
+CASES += [(torch.float32, 5121, 4608, 8), (torch.float32, 2562, 4608, 15), (torch.float32, 300, 640, 77),
+          (torch.float32, 257, 1152, 130), (torch.float32, 130, 128, 65)]
+
+
+@pytest.mark.parametrize(("dtype", "rows", "columns", "batch"), CASES)
+def test_small_batches_match_the_oracle(dtype, rows, columns, batch) -> None:
+    print(f"trit: {dtype} rows={rows} columns={columns} batch={batch}", flush=True)
+    blocks = random_blocks(rows, columns, seed=rows + columns + batch)
+    packed, lay = pack(blocks), layout(rows, columns)
+    x = activations(batch, columns, dtype, seed=batch)
+    got = tq1_linear_words(packed, x, layout=lay)
+    assert torch.equal(got, tq1_linear_words(packed, x, layout=lay))  # the same bits twice
+    x64 = x.double().cpu().numpy()
+    want = O.oracle_matmul(blocks, x64, rows=rows, columns=columns)
+    assert (np.abs(got.double().cpu().numpy() - want) <= bound(x64, blocks, want, dtype)).all()
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("batch", (2, 7, 30, 64))
+def test_the_fused_swiglu_is_the_linear_and_the_elementwise_step(dtype, batch) -> None:
+    rows, columns = 1030, 1152
+    packed, lay = pack(random_blocks(rows, columns, seed=batch)), layout(rows, columns)
+    x = to_dev(np.random.default_rng(batch).normal(0.0, 0.3, size=(batch, columns)).astype(np.float32)).to(dtype)
+    both = tq1_linear_words(packed, x, layout=lay).float()
+    gate, up = both[:, 0::2], both[:, 1::2]
+    want = (gate / (1.0 + torch.exp(-gate)) * up).to(dtype).float()
+    diff = (tq1_swiglu_words(packed, x, layout=lay).float() - want).abs()
+    # expf against torch's exp, then one rounding: at most a step of the type
+    assert bool((diff <= want.abs() * 2 * ROUNDOFF[dtype] + 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16, torch.float32))
+def test_non_finite_values_follow_the_entry_point(dtype) -> None:
+    """The GEMM path computes (t - 1) * scale (a zero trit of a non-finite scale
+    is NaN), the matmul path scale * sum as the LUT23 kernel does."""
+    rows, columns, batch = 640, 640, 80 if dtype == torch.float32 else 6
+    blocks = random_blocks(rows, columns, seed=3)
+    bits = {5: 0x7C00, 70: 0xFC00, 300: 0x7E00}  # +inf, -inf, NaN in a row's second group
+    for row, value in bits.items():
+        blocks[row, 1, 0:2] = np.frombuffer(np.uint16(value).tobytes(), dtype=np.uint8)
+    packed, lay = pack(blocks), layout(rows, columns)
+    x = to_dev(np.random.default_rng(4).normal(0.0, 1.0, size=(batch, columns)).astype(np.float32)).to(dtype)
+    x[1, 7], x[2, 639] = float("inf"), float("nan")
+    x64 = x.double().cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        products = O.oracle_matmul(blocks, x64, rows=rows, columns=columns)
+        tables = O.lut23_matmul(blocks, x64.astype(np.float32), rows=rows, columns=columns)
+    if dtype != torch.float32:
+        got = tq1_linear_words(packed, x, layout=lay).float().cpu().numpy()
+        assert O.compare(got, products)["pattern_mismatches"] == 0
+    got = tq1_matmul_words(packed, x, layout=lay).float().cpu().numpy()
+    assert O.compare(got, tables)["pattern_mismatches"] == 0
