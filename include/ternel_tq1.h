@@ -289,9 +289,9 @@ int ternel_tq1_linear_kernel(int64_t M, int64_t rows, int64_t columns, int dtype
  * two unfused layers would return them, and SiLU(g) * u is computed in fp32.
  * z is [M][rows / 2] in the activation type. No counterpart in the reference
  * (its MLP runs gate_proj, up_proj and the activation as separate mlx ops,
- * src/ternel_mlx/packed_model.py:72-92). The LUT23, strip and direct-form
- * kernels have the pair exchange in their epilogues; batches of the wide and
- * tile forms run the GEMM into the workspace and one elementwise pass. Workspace
+ * src/ternel_mlx/packed_model.py:72-92). Every kernel but the tile form
+ * has the pair exchange in its epilogue; the tile form's batches run the GEMM
+ * into the workspace and one elementwise pass. Workspace
  * from ternel_tq1_swiglu_workspace_bytes, same contract as ternel_tq1_linear's.
  */
 int ternel_tq1_swiglu(const uint32_t *packed, const void *x, void *z, int64_t M, int64_t rows, int64_t columns,

@@ -2189,7 +2189,7 @@ struct WideGeometry {
     int tiles_n;     // weight row blocks of 256
     int tiles;       // tiles_n * ceil(M / (32 NB))
     int units;       // tiles * G
-    int vector_rows; // y rows start 16-byte aligned (y aligned, N % 8 == 0)
+    int vector_rows; // y rows start 16-byte aligned (y aligned, its width a multiple of 8)
     int spin_limit;  // polls of the publication count before the last arriver gives up
 };
 
@@ -2337,7 +2337,10 @@ __device__ __forceinline__ void buffer_dma4(__amdgpu_buffer_rsrc_t rsrc, void *l
 
 // BF: the activations were bf16 (scale_rows_kernel): each output value is
 // the fp32 sum times its activation row's inv, rounded once to bf16.
-template <int NB, bool BF>
+// GLU: y is [M][N / 2], SiLU(row 2r) * (row 2r + 1). A separate elementwise
+// pass read and wrote what the sums' registers hold: 5120 -> 2 x 17408 at
+// M=512 194.6 -> 178.2 us, M=2048 708.7 -> 654.2 (fp16).
+template <int NB, bool BF, bool GLU>
 __global__ __launch_bounds__(kWideThreads) void wide_gemm_kernel(
     const uint32_t *__restrict__ packed, const _Float16 *__restrict__ xp, uint16_t *__restrict__ y,
     float *__restrict__ partial, unsigned *__restrict__ counters, const float *__restrict__ row_inv,
@@ -2622,39 +2625,69 @@ __global__ __launch_bounds__(kWideThreads) void wide_gemm_kernel(
         else
             return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
     };
+    using Out = std::conditional_t<BF, bf16_t, _Float16>;
+    auto store_run = [&](uint16_t *row, int n, int width, const uint4 &v) {  // 8 values from column n
+        if (geo.vector_rows && n + 8 <= width) {
+            *reinterpret_cast<uint4 *>(row + n) = v;
+        } else {
+            const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (n + e < width) row[n + e] = static_cast<uint16_t>(d[e >> 1] >> (16 * (e & 1)));
+        }
+    };
+    auto swap_halves = [&](uint32_t send) {  // the value lane ^ 32 sends
+        return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, static_cast<int>(send)));
+    };
     auto store_frag = [&](int t, int nb, const float *vals) {
         const int m = (t / geo.tiles_n) * kCols + nb * 32 + (lane & 31);
         float sc = 1.0f;
         if constexpr (BF) sc = row_inv[min(m, geo.M - 1)];
-        uint32_t h[4][2];
+        if constexpr (GLU) {
+            // Rows 2r and 2r + 1, a gate and its up, are neighbours in a lane:
+            // pair 4qq + 2(lane / 32) + k of the fragment's 16 from each
+            // other's registers, rounded to the output type first as the
+            // unfused layers would return them. The lower lane keeps pairs
+            // 0..7, the upper 8..15: one 16-byte store per lane.
+            uint32_t d[4];
 #pragma unroll
-        for (int qq = 0; qq < 4; ++qq)
+            for (int qq = 0; qq < 4; ++qq) {
+                uint16_t z[2];
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
-                h[qq][k] = out_bits(vals[4 * qq + 2 * k] * sc) | (out_bits(vals[4 * qq + 2 * k + 1] * sc) << 16);
-        // rows 8qq + 4(lane / 32) + e; the lower lane keeps runs qq = 0, 2, the upper qq = 1, 3
-        uint32_t r[4];
+                for (int k = 0; k < 2; ++k)
+                    z[k] = __builtin_bit_cast(uint16_t, swiglu_pair<Out>(from_f32<Out>(vals[4 * qq + 2 * k] * sc),
+                                                                         from_f32<Out>(vals[4 * qq + 2 * k + 1] * sc)));
+                d[qq] = z[0] | (static_cast<uint32_t>(z[1]) << 16);
+            }
+            const uint32_t r0 = swap_halves(upper ? d[0] : d[2]), r1 = swap_halves(upper ? d[1] : d[3]);
+            if (m >= geo.M) return;
+            store_run(y + static_cast<int64_t>(m) * (geo.N / 2),
+                      (t % geo.tiles_n) * (kWideRows / 2) + wave * 16 + (upper ? 8 : 0), geo.N / 2,
+                      upper ? uint4{r0, d[2], r1, d[3]} : uint4{d[0], r0, d[1], r1});
+        } else {
+            uint32_t h[4][2];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t send = upper ? h[(k >> 1) * 2][k & 1] : h[(k >> 1) * 2 + 1][k & 1];
-            r[k] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, static_cast<int>(send)));
-        }
-        if (m >= geo.M) return;
-        uint16_t *yrow = y + static_cast<int64_t>(m) * geo.N;
+            for (int qq = 0; qq < 4; ++qq)
 #pragma unroll
-        for (int run = 0; run < 2; ++run) {  // rows 16 run + 8 (lane / 32) .. + 8
-            const int n = (t % geo.tiles_n) * kWideRows + wave * 32 + 16 * run + (upper ? 8 : 0);
-            const uint32_t *own = h[2 * run + (upper ? 1 : 0)];
-            uint4 v;
-            if (upper) v = uint4{r[2 * run], r[2 * run + 1], own[0], own[1]};
-            else v = uint4{own[0], own[1], r[2 * run], r[2 * run + 1]};
-            if (geo.vector_rows && n + 8 <= geo.N) {
-                *reinterpret_cast<uint4 *>(yrow + n) = v;
-            } else {
-                const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+                for (int k = 0; k < 2; ++k)
+                    h[qq][k] = out_bits(vals[4 * qq + 2 * k] * sc) | (out_bits(vals[4 * qq + 2 * k + 1] * sc) << 16);
+            // rows 8qq + 4(lane / 32) + e; the lower lane keeps runs qq = 0, 2, the upper qq = 1, 3
+            uint32_t r[4];
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (n + e < geo.N) yrow[n + e] = static_cast<uint16_t>(d[e >> 1] >> (16 * (e & 1)));
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t send = upper ? h[(k >> 1) * 2][k & 1] : h[(k >> 1) * 2 + 1][k & 1];
+                r[k] = swap_halves(send);
+            }
+            if (m >= geo.M) return;
+            uint16_t *yrow = y + static_cast<int64_t>(m) * geo.N;
+#pragma unroll
+            for (int run = 0; run < 2; ++run) {  // rows 16 run + 8 (lane / 32) .. + 8
+                const int n = (t % geo.tiles_n) * kWideRows + wave * 32 + 16 * run + (upper ? 8 : 0);
+                const uint32_t *own = h[2 * run + (upper ? 1 : 0)];
+                uint4 v;
+                if (upper) v = uint4{r[2 * run], r[2 * run + 1], own[0], own[1]};
+                else v = uint4{own[0], own[1], r[2 * run], r[2 * run + 1]};
+                store_run(yrow, n, geo.N, v);
             }
         }
     };
@@ -2665,12 +2698,14 @@ __global__ __launch_bounds__(kWideThreads) void wide_gemm_kernel(
         for (int nb = 0; nb < NB; ++nb) {
             const int m = (t / geo.tiles_n) * kCols + nb * 32 + (lane & 31);
             if (m >= geo.M) continue;
-            uint16_t *yrow = y + static_cast<int64_t>(m) * geo.N;
+            // (with GLU a wave's 32 rows are 16 columns)
+            const int width = GLU ? geo.N / 2 : geo.N, own = GLU ? 16 : 32;
+            uint16_t *yrow = y + static_cast<int64_t>(m) * width;
 #pragma unroll 1
-            for (int run = 0; run < 2; ++run) {
-                const int n = (t % geo.tiles_n) * kWideRows + wave * 32 + 16 * run + (upper ? 8 : 0);
+            for (int run = 0; run < own / 16; ++run) {
+                const int n = (t % geo.tiles_n) * (own * kWideWaves) + wave * own + 16 * run + (upper ? 8 : 0);
                 for (int e = 0; e < 8; ++e)
-                    if (n + e < geo.N) yrow[n + e] = nan16;
+                    if (n + e < width) yrow[n + e] = nan16;
             }
         }
     };
@@ -3569,41 +3604,38 @@ int plan_wide(int64_t M, int64_t rows, int64_t columns, int k_split, WidePlan *p
     return TERNEL_TQ1_OK;
 }
 
-template <int NB, bool BF>
+template <int NB, bool BF, bool GLU>
 int launch_wide_kernel(const uint32_t *packed, const _Float16 *xp, void *y, float *partial, unsigned *counters,
                        const float *row_inv, const WideGeometry &geo, int workgroups, hipStream_t stream) {
-    int rc = ensure_lds_attribute(reinterpret_cast<const void *>(&wide_gemm_kernel<NB, BF>),
+    int rc = ensure_lds_attribute(reinterpret_cast<const void *>(&wide_gemm_kernel<NB, BF, GLU>),
                                   static_cast<int>(wide_lds_bytes(NB)));
     if (rc != TERNEL_TQ1_OK) return rc;
-    hipLaunchKernelGGL((wide_gemm_kernel<NB, BF>), dim3(static_cast<unsigned>(workgroups)), dim3(kWideThreads),
+    hipLaunchKernelGGL((wide_gemm_kernel<NB, BF, GLU>), dim3(static_cast<unsigned>(workgroups)), dim3(kWideThreads),
                        wide_lds_bytes(NB), stream, packed, xp, static_cast<uint16_t *>(y), partial, counters, row_inv,
                        geo);
     TQ1_LAUNCH_CHECK();
     return TERNEL_TQ1_OK;
 }
 
-template <bool BF>
+template <bool BF, bool GLU>
 int launch_wide_nb(const uint32_t *packed, const _Float16 *xp, void *y, float *partial, unsigned *counters,
                    const float *row_inv, const WidePlan &plan, const WideGeometry &geo, hipStream_t stream) {
+    const int wgs = plan.workgroups;
     switch (plan.nb) {
-        case 1:
-            return launch_wide_kernel<1, BF>(packed, xp, y, partial, counters, row_inv, geo, plan.workgroups, stream);
-        case 2:
-            return launch_wide_kernel<2, BF>(packed, xp, y, partial, counters, row_inv, geo, plan.workgroups, stream);
-        case 4:
-            return launch_wide_kernel<4, BF>(packed, xp, y, partial, counters, row_inv, geo, plan.workgroups, stream);
-        default:
-            return launch_wide_kernel<8, BF>(packed, xp, y, partial, counters, row_inv, geo, plan.workgroups, stream);
+        case 1: return launch_wide_kernel<1, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
+        case 2: return launch_wide_kernel<2, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
+        case 4: return launch_wide_kernel<4, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
+        default: return launch_wide_kernel<8, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
     }
 }
 
 int launch_wide(const uint32_t *packed, const void *x, void *y, const WidePlan &plan, void *ws, hipStream_t stream,
-                int dtype) {
+                int dtype, bool glu = false) {
     unsigned *counters = static_cast<unsigned *>(ws);
     float *partial = reinterpret_cast<float *>(static_cast<char *>(ws) + kPartialOffset);
     _Float16 *copy = reinterpret_cast<_Float16 *>(static_cast<char *>(ws) + kPartialOffset + plan.partial_bytes);
     WideGeometry geo = plan.geo;
-    geo.vector_rows = geo.N % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    geo.vector_rows = geo.N % (glu ? 16 : 8) == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
     if (dtype == TERNEL_TQ1_BF16) {
         float *row_inv = reinterpret_cast<float *>(copy + static_cast<int64_t>(geo.M) * geo.G * kBlockWeights);
         const int64_t K = static_cast<int64_t>(geo.G) * kBlockWeights;
@@ -3614,7 +3646,8 @@ int launch_wide(const uint32_t *packed, const void *x, void *y, const WidePlan &
             hipLaunchKernelGGL(scale_rows_kernel<false>, dim3(static_cast<unsigned>(geo.M)), dim3(kThreads), 0, stream,
                                static_cast<const uint16_t *>(x), copy, row_inv, K);
         TQ1_LAUNCH_CHECK();
-        return launch_wide_nb<true>(packed, copy, y, partial, counters, row_inv, plan, geo, stream);
+        return glu ? launch_wide_nb<true, true>(packed, copy, y, partial, counters, row_inv, plan, geo, stream)
+                   : launch_wide_nb<true, false>(packed, copy, y, partial, counters, row_inv, plan, geo, stream);
     }
     const _Float16 *xp = static_cast<const _Float16 *>(x);
     if (plan.nb > 2) {
@@ -3625,7 +3658,8 @@ int launch_wide(const uint32_t *packed, const void *x, void *y, const WidePlan &
         TQ1_LAUNCH_CHECK();
         xp = copy;
     }
-    return launch_wide_nb<false>(packed, xp, y, partial, counters, nullptr, plan, geo, stream);
+    return glu ? launch_wide_nb<false, true>(packed, xp, y, partial, counters, nullptr, plan, geo, stream)
+               : launch_wide_nb<false, false>(packed, xp, y, partial, counters, nullptr, plan, geo, stream);
 }
 
 // Automatic choice, from a sweep of every form over the 27B linears on MI355X
@@ -4281,6 +4315,8 @@ size_t ternel_tq1_swiglu_workspace_bytes(int64_t M, int64_t rows, int64_t column
     }
     if (swiglu_gemm_uses_trit(M, rows, columns, dtype))
         return plan_trit(M, rows, columns, dtype, 0, &trit) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
+    if (resolve_gemm_form(M, rows, columns, linear_gemm_form(M, rows, columns, dtype), 0) == TERNEL_TQ1_GEMM_WIDE)
+        return ternel_tq1_gemm_workspace_bytes(M, rows, columns, TERNEL_TQ1_GEMM_WIDE, 0);
     return swiglu_pairs_offset(M, rows, columns, dtype) + static_cast<size_t>(M) * rows * sizeof(_Float16);
 }
 
@@ -4339,11 +4375,22 @@ int ternel_tq1_swiglu(const uint32_t *packed, const void *x, void *z, int64_t M,
                 return launch_lut<float>(packed, x, z, M, rows, columns, plan, ws, s, true);
         }
     }
+    // So does the wide form; the tile form's output takes an elementwise pass.
+    const int gemm_form = linear_gemm_form(M, rows, columns, dtype);
+    if (resolve_gemm_form(M, rows, columns, gemm_form, 0) == TERNEL_TQ1_GEMM_WIDE) {
+        WidePlan wide;
+        if ((rc = plan_wide(M, rows, columns, 0, &wide)) != TERNEL_TQ1_OK) return rc;
+        if (reinterpret_cast<uintptr_t>(x) & 15u) return fail(TERNEL_TQ1_EINVAL, "activations must be 16-byte aligned");
+        const size_t need = kPartialOffset + wide.partial_bytes + wide.xp_bytes;
+        if (!ws || ws_bytes < need)
+            return fail(TERNEL_TQ1_EINVAL, "workspace of %zu bytes is smaller than the %zu a SwiGLU GEMM needs", ws_bytes,
+                        need);
+        return launch_wide(packed, x, z, wide, ws, s, dtype, true);
+    }
     const size_t need = ternel_tq1_swiglu_workspace_bytes(M, rows, columns, dtype);
     if (need == 0 || !ws || ws_bytes < need)
         return fail(TERNEL_TQ1_EINVAL, "workspace of %zu bytes is smaller than the %zu a SwiGLU GEMM needs", ws_bytes,
                     need);
-    const int gemm_form = linear_gemm_form(M, rows, columns, dtype);
     const size_t gemm = ternel_tq1_gemm_workspace_bytes(M, rows, columns, gemm_form, 0);
     void *pairs = static_cast<char *>(ws) + swiglu_pairs_offset(M, rows, columns, dtype);
     if ((rc = ternel_tq1_gemm(packed, x, pairs, M, rows, columns, dtype, gemm_form, 0, gemm ? ws : nullptr, gemm,
@@ -4352,12 +4399,8 @@ int ternel_tq1_swiglu(const uint32_t *packed, const void *x, void *z, int64_t M,
     const int64_t count = M * (rows / 2);
     int64_t grid = ceil_div(count, kThreads);
     if (grid > 65536) grid = 65536;
-    if (dtype == TERNEL_TQ1_BF16)
-        hipLaunchKernelGGL((swiglu_pairs_kernel<bf16_t>), dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s,
-                           static_cast<const bf16_t *>(pairs), static_cast<bf16_t *>(z), count);
-    else
-        hipLaunchKernelGGL((swiglu_pairs_kernel<_Float16>), dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s,
-                           static_cast<const _Float16 *>(pairs), static_cast<_Float16 *>(z), count);
+    hipLaunchKernelGGL((swiglu_pairs_kernel<_Float16>), dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s,
+                       static_cast<const _Float16 *>(pairs), static_cast<_Float16 *>(z), count);  // (bf16 is never tiled)
     TQ1_LAUNCH_CHECK();
     return TERNEL_TQ1_OK;
 }

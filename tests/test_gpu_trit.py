@@ -1,4 +1,5 @@
-"""The trit kernel (small batches of fp16, bf16 and fp32 activations) against the fp64 oracle.
+"""The trit kernel (small batches of fp16, bf16 and fp32 activations) against the fp64 oracle, and
+the SwiGLU epilogues of the MFMA kernels against the linear they follow.
 
 Shapes sit where it can go wrong: row counts that are no multiple of a wave's
 32 or a workgroup's 128 rows, group counts below, at and past its windows (1,
@@ -10,12 +11,15 @@ fp32 summation bound plus one rounding to its type.
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import tq1_oracle as O
 from tests.gpu_util import layout, pack, random_blocks, to_dev
+from ternel_amd import _lib
 from ternel_amd.kernels import tq1_linear_words, tq1_matmul_words, tq1_swiglu_words
 
 pytestmark = pytest.mark.gpu
@@ -59,10 +63,15 @@ def test_small_batches_match_the_oracle(dtype, rows, columns, batch) -> None:
     assert (np.abs(got.double().cpu().numpy() - want) <= bound(x64, blocks, want, dtype)).all()
 
 
-@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
-@pytest.mark.parametrize("batch", (2, 7, 30, 64))
-def test_the_fused_swiglu_is_the_linear_and_the_elementwise_step(dtype, batch) -> None:
-    rows, columns = 1030, 1152
+# the trit kernel's tiles, then the wide form's (fp16 takes it from 64 tiles of
+# 256 rows on); an output width that no 16-byte store divides, and one it does
+SWIGLU = [(dtype, 1030, 1152, batch) for dtype in (torch.float16, torch.bfloat16) for batch in (2, 7, 30, 64)]
+SWIGLU += [(torch.bfloat16, 1030, 1152, 70), (torch.bfloat16, 1030, 1152, 300), (torch.bfloat16, 1024, 1152, 300),
+           (torch.float16, 16390, 256, 70), (torch.float16, 16400, 256, 300)]
+
+
+@pytest.mark.parametrize(("dtype", "rows", "columns", "batch"), SWIGLU)
+def test_the_fused_swiglu_is_the_linear_and_the_elementwise_step(dtype, rows, columns, batch) -> None:
     packed, lay = pack(random_blocks(rows, columns, seed=batch)), layout(rows, columns)
     x = to_dev(np.random.default_rng(batch).normal(0.0, 0.3, size=(batch, columns)).astype(np.float32)).to(dtype)
     both = tq1_linear_words(packed, x, layout=lay).float()
@@ -94,3 +103,28 @@ def test_non_finite_values_follow_the_entry_point(dtype) -> None:
         assert O.compare(got, products)["pattern_mismatches"] == 0
     got = tq1_matmul_words(packed, x, layout=lay).float().cpu().numpy()
     assert O.compare(got, tables)["pattern_mismatches"] == 0
+
+
+def test_a_swiglu_reduction_that_gives_up_writes_nan() -> None:
+    """The wide form's bounded wait driven to give up from the host: every
+    output is the fused value or NaN, some are NaN, and the error word is set."""
+    rows, columns, batch = 1030, 5120, 300
+    packed, lay = pack(random_blocks(rows, columns, seed=5)), layout(rows, columns)
+    x = to_dev(np.random.default_rng(5).normal(0.0, 0.3, size=(batch, columns)).astype(np.float32)).to(torch.bfloat16)
+    want = tq1_swiglu_words(packed, x, layout=lay)
+    handle = _lib.lib()
+    need = handle.ternel_tq1_swiglu_workspace_bytes(batch, rows, columns, _lib.DTYPE_BF16)
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    out = torch.zeros((batch, rows // 2), dtype=torch.bfloat16, device="cuda")
+    old = handle.ternel_tq1_set_spin_limit(-1)
+    try:
+        _lib.check(handle.ternel_tq1_swiglu(packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, rows, columns,
+                                            _lib.DTYPE_BF16, ws.data_ptr(), need, 0))
+        torch.cuda.synchronize()
+    finally:
+        handle.ternel_tq1_set_spin_limit(old)
+    word = ctypes.c_int(0)
+    _lib.check(handle.ternel_tq1_workspace_error(ws.data_ptr(), need, ctypes.byref(word), 0))
+    nan = torch.isnan(out)
+    assert word.value == 2 and bool(nan.any())
+    assert torch.equal(out[~nan], want[~nan])
