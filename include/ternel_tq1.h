@@ -126,6 +126,16 @@ int ternel_tq1_deinterleave(const uint32_t *packed, int64_t rows, int64_t column
                             void *stream);
 
 /*
+ * ternel_tq1_interleave with ternel_tq1_validate's scan folded in, one pass
+ * over the blocks: counters as ternel_tq1_validate writes them; the caller
+ * drops the packed words when either is nonzero. Replaces validate_packed_codes
+ * and the reorder of a load (src/ternel_mlx/packing.py:29-48,
+ * src/bonsai_tq1/lut23_reorder.py:126-165).
+ */
+int ternel_tq1_interleave_checked(const uint8_t *blocks, int64_t rows, int64_t columns, uint32_t *packed,
+                                  uint64_t *counters, void *stream);
+
+/*
  * The reference's tiled pair -> packed words, on the device, with the
  * fail-closed scan folded in: codes is uint8 [rows/tile][G][26][tile], scales
  * uint16 (raw fp16 bits) [rows/tile][G][tile] (src/ternel_mlx/layout.py:100-108),

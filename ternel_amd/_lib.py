@@ -42,6 +42,7 @@ SIGNATURES = {
     "ternel_tq1_decode": (_int, [_p, _i64, _p, _p, _p]),
     "ternel_tq1_from_q2": (_int, [_p, _i64, _p, _p, _p]),
     "ternel_tq1_interleave": (_int, [_p, _i64, _i64, _p, _p]),
+    "ternel_tq1_interleave_checked": (_int, [_p, _i64, _i64, _p, _p, _p]),
     "ternel_tq1_deinterleave": (_int, [_p, _i64, _i64, _p, _p]),
     "ternel_tq1_words_from_tiled": (_int, [_p, _p, _i64, _i64, _i64, _p, _p, _p]),
     "ternel_tq1_tiled_from_words": (_int, [_p, _i64, _i64, _i64, _p, _p, _p]),

@@ -33,7 +33,7 @@ from typing import Mapping
 import numpy as np
 import torch
 
-from .format import BLOCK_BYTES, BLOCK_SIZE, FormatError, as_device_blocks, validate_packed_codes
+from .format import BLOCK_BYTES, BLOCK_SIZE, FormatError, as_device_blocks
 from .layout import SCALE_VIEW_DTYPE, PackedTensorLayout, pack_blocks, select_tile, unpack_blocks
 
 # Sidecar geometry (src/bonsai_tq1/format.py:14-30).
@@ -239,9 +239,7 @@ def upload(blocks, layout: PackedTensorLayout, *, device=None, validate: bool = 
     if tensor.shape[0] != layout.groups:
         raise FormatError(f"expected {layout.groups} blocks for {layout.rows}x{layout.columns}, "
                           f"got {tensor.shape[0]}")
-    if validate:
-        validate_packed_codes(tensor)
-    return pack_weights(tensor, layout=layout)
+    return pack_weights(tensor, layout=layout, validate=validate)
 
 
 def load_sidecar_tensor(path, name: str, *, device=None, validate: bool = True):

@@ -208,6 +208,24 @@ __global__ void zero_u64_kernel(unsigned long long *p, int n) {
 //                   b >= 27   <=>  bit7(b) | bit7((b & 0x7f) + 101)
 // (the additions never carry across bytes).
 // ---------------------------------------------------------------------------
+// Adds the illegal code bytes of block word j.
+__device__ __forceinline__ void count_illegal(uint32_t word, int j, uint32_t &bad_regular, uint32_t &bad_tail) {
+    const uint32_t regular_mask = j == 0 ? 0x80800000u : (j == 6 ? 0x00808080u : 0x80808080u);
+    const uint32_t tail_mask = j == 6 ? 0x80000000u : 0u;
+    const uint32_t low7 = word & 0x7f7f7f7fu;
+    bad_regular += __popc(word & (low7 + 0x0d0d0d0du) & regular_mask);
+    bad_tail += __popc((word | (low7 + 0x65656565u)) & tail_mask);
+}
+
+__device__ __forceinline__ void add_illegal(uint32_t bad_regular, uint32_t bad_tail, unsigned long long *counters) {
+    bad_regular = wave_sum_u32(bad_regular);
+    bad_tail = wave_sum_u32(bad_tail);
+    if ((threadIdx.x & 63) == 0) {
+        if (bad_regular) atomicAdd(&counters[0], static_cast<unsigned long long>(bad_regular));
+        if (bad_tail) atomicAdd(&counters[1], static_cast<unsigned long long>(bad_tail));
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void validate_kernel(const uint32_t *__restrict__ words,
                                                             int64_t nwords,
                                                             unsigned long long *counters) {
@@ -218,20 +236,11 @@ __global__ __launch_bounds__(kThreads) void validate_kernel(const uint32_t *__re
     uint32_t bad_regular = 0, bad_tail = 0;
     for (int64_t w = first; w < nwords; w += stride) {
         const uint32_t d = words[w];
-        const uint32_t regular_mask = j == 0 ? 0x80800000u : (j == 6 ? 0x00808080u : 0x80808080u);
-        const uint32_t tail_mask = j == 6 ? 0x80000000u : 0u;
-        const uint32_t low7 = d & 0x7f7f7f7fu;
-        bad_regular += __popc(d & (low7 + 0x0d0d0d0du) & regular_mask);
-        bad_tail += __popc((d | (low7 + 0x65656565u)) & tail_mask);
+        count_illegal(d, j, bad_regular, bad_tail);
         j += step;
         if (j >= kBlockWords) j -= kBlockWords;
     }
-    bad_regular = wave_sum_u32(bad_regular);
-    bad_tail = wave_sum_u32(bad_tail);
-    if ((threadIdx.x & 63) == 0) {
-        if (bad_regular) atomicAdd(&counters[0], static_cast<unsigned long long>(bad_regular));
-        if (bad_tail) atomicAdd(&counters[1], static_cast<unsigned long long>(bad_tail));
-    }
+    add_illegal(bad_regular, bad_tail, counters);
 }
 
 // ---------------------------------------------------------------------------
@@ -309,20 +318,65 @@ __global__ __launch_bounds__(kThreads) void q2_to_tq1_kernel(const uint8_t *__re
 
 // ---------------------------------------------------------------------------
 // interleave_kernel / deinterleave_kernel: canonical blocks <-> packed words.
-// One thread per packed word (writes coalesced) / per canonical word.
+//
+// Interleave, bound by memory: a workgroup turns 8 groups of one 64-row tile
+// around in LDS, so that it reads each row's run (224 contiguous bytes) and
+// writes the tile's words in order. A thread per packed word reading its word
+// where it lies fetched every 128-byte line about eight times (a wave's 64
+// rows are a row apart, and the workgroups that use the rest of a line run on
+// other XCDs). Neighbouring runs share lines, so each XCD takes a contiguous
+// range of the workgroups: 153,688 line reads for 17408 x 5120's 152,320.
+// CHECK counts illegal bytes on the way (validate_kernel's counts), which
+// saves a load its second pass over the blocks. Measured on MI355X, 17408 x
+// 5120: scan 7.6 us and permutation 25.0 before, 11.5 together now (in tiles of 16
+// groups 14.5, of 4 groups 14.2: fewer workgroups, and more of the lines
+// shared).
 // ---------------------------------------------------------------------------
+constexpr int kInterleaveGroups = 8;
+constexpr int kInterleaveWords = kInterleaveGroups * kBlockWords;  // 56 per row
+constexpr int kInterleaveStride = kInterleaveWords + 1;            // odd: a column's 64 rows in distinct banks
+
+template <bool CHECK>
 __global__ __launch_bounds__(kThreads) void interleave_kernel(const uint32_t *__restrict__ canonical,
-                                                              uint32_t *__restrict__ packed, int64_t rows,
-                                                              int64_t G, int64_t total_words) {
-    const int64_t w = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (w >= total_words) return;
-    const int lane = static_cast<int>(w % kTileRows);
-    const int64_t rest = w / kTileRows;
-    const int j = static_cast<int>(rest % kBlockWords);
-    const int64_t tg = rest / kBlockWords;
-    const int64_t g = tg % G;
-    const int64_t row = (tg / G) * kTileRows + lane;
-    packed[w] = row < rows ? canonical[(row * G + g) * kBlockWords + j] : 0u;
+                                                              uint32_t *__restrict__ packed, int64_t rows, int64_t G,
+                                                              int chunks, unsigned long long *counters) {
+    __shared__ uint32_t lds[kTileRows * kInterleaveStride];
+    const unsigned P = gridDim.x;
+    const unsigned p = (P & 7u) == 0 ? (blockIdx.x & 7u) * (P >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    const int64_t tile = p / static_cast<unsigned>(chunks);
+    const int64_t g0 = static_cast<int64_t>(p - static_cast<unsigned>(tile) * chunks) * kInterleaveGroups;
+    const int words = static_cast<int>(min(static_cast<int64_t>(kInterleaveGroups), G - g0)) * kBlockWords;  // per row
+    const int64_t row0 = tile * kTileRows;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr int kWaves = kThreads / 64, kRowsPerWave = kTileRows / kWaves, kRuns = (kInterleaveWords + 63) / 64;
+    uint32_t bad_regular = 0, bad_tail = 0;
+    // Rows wave, wave + 4, ..., all loads issued (clamped) before the first is
+    // used.
+    uint32_t v[kRowsPerWave][kRuns];
+#pragma unroll
+    for (int i = 0; i < kRowsPerWave; ++i) {
+        const int64_t row = min(row0 + wave + i * kWaves, rows - 1);
+        const uint32_t *src = canonical + (row * G + g0) * kBlockWords;
+#pragma unroll
+        for (int h = 0; h < kRuns; ++h) v[i][h] = src[min(lane + h * 64, words - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < kRowsPerWave; ++i) {
+        const int r = wave + i * kWaves;
+        const bool real = row0 + r < rows;
+#pragma unroll
+        for (int h = 0; h < kRuns; ++h) {
+            const int c = lane + h * 64;
+            if (c < words) {
+                if (CHECK && real) count_illegal(v[i][h], c % kBlockWords, bad_regular, bad_tail);
+                lds[r * kInterleaveStride + c] = real ? v[i][h] : 0u;
+            }
+        }
+    }
+    __syncthreads();
+    uint32_t *dst = packed + (tile * G + g0) * kTileGroupWords;
+    for (int c = wave; c < words; c += kWaves) dst[c * kTileRows + lane] = lds[lane * kInterleaveStride + c];
+    if constexpr (CHECK) add_illegal(bad_regular, bad_tail, counters);
 }
 
 // ---------------------------------------------------------------------------
@@ -369,12 +423,7 @@ __global__ __launch_bounds__(kThreads) void words_from_tiled_kernel(const uint8_
         }
         packed[w] = word;
     }
-    bad_regular = wave_sum_u32(bad_regular);
-    bad_tail = wave_sum_u32(bad_tail);
-    if ((threadIdx.x & 63) == 0) {
-        if (bad_regular) atomicAdd(&counters[0], static_cast<unsigned long long>(bad_regular));
-        if (bad_tail) atomicAdd(&counters[1], static_cast<unsigned long long>(bad_tail));
-    }
+    add_illegal(bad_regular, bad_tail, counters);
 }
 
 __global__ __launch_bounds__(kThreads) void tiled_from_words_kernel(const uint32_t *__restrict__ packed,
@@ -3807,6 +3856,30 @@ int launch_get_rows(const uint32_t *table, int64_t rows, int64_t columns, const 
     return TERNEL_TQ1_OK;
 }
 
+template <bool CHECK>
+static int launch_interleave(const uint8_t *blocks, int64_t rows, int64_t columns, uint32_t *packed, uint64_t *counters,
+                             void *stream) {
+    g_last_error[0] = '\0';
+    int rc;
+    if ((rc = check_geometry(1, rows, columns)) != TERNEL_TQ1_OK) return rc;
+    if (!blocks || !packed || (CHECK && !counters)) return fail(TERNEL_TQ1_EINVAL, "null pointer");
+    if ((reinterpret_cast<uintptr_t>(blocks) | reinterpret_cast<uintptr_t>(packed)) & 3u)
+        return fail(TERNEL_TQ1_EINVAL, "blocks and packed weights must be 4-byte aligned");
+    const int64_t G = columns / kBlockWeights, chunks = ceil_div(G, kInterleaveGroups);
+    const int64_t grid = ceil_div(rows, kTileRows) * chunks;
+    if (grid > INT32_MAX) return fail(TERNEL_TQ1_EINVAL, "too many blocks for one interleave launch");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    auto *cnt = reinterpret_cast<unsigned long long *>(counters);
+    if (CHECK) {
+        hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, s, cnt, 2);
+        TQ1_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(interleave_kernel<CHECK>, dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s,
+                       reinterpret_cast<const uint32_t *>(blocks), packed, rows, G, static_cast<int>(chunks), cnt);
+    TQ1_LAUNCH_CHECK();
+    return TERNEL_TQ1_OK;
+}
+
 // The split-K workspace of ternel_tq1_matmul_noalloc as a file-scope device
 // array (counter region, then at most kNoAllocPartialBytes of fp32 partials),
 // for callers that cannot allocate. Each device the library runs on holds its
@@ -3960,18 +4033,12 @@ int ternel_tq1_decode(const uint8_t *blocks, int64_t nblocks, uint8_t *scales_ou
 }
 
 int ternel_tq1_interleave(const uint8_t *blocks, int64_t rows, int64_t columns, uint32_t *packed, void *stream) {
-    g_last_error[0] = '\0';
-    int rc;
-    if ((rc = check_geometry(1, rows, columns)) != TERNEL_TQ1_OK) return rc;
-    if (!blocks || !packed) return fail(TERNEL_TQ1_EINVAL, "null pointer");
-    if ((reinterpret_cast<uintptr_t>(blocks) | reinterpret_cast<uintptr_t>(packed)) & 3u)
-        return fail(TERNEL_TQ1_EINVAL, "blocks and packed weights must be 4-byte aligned");
-    const int64_t total = packed_words(rows, columns);
-    hipLaunchKernelGGL(interleave_kernel, dim3(static_cast<unsigned>(ceil_div(total, kThreads))), dim3(kThreads), 0,
-                       static_cast<hipStream_t>(stream), reinterpret_cast<const uint32_t *>(blocks), packed, rows,
-                       columns / kBlockWeights, total);
-    TQ1_LAUNCH_CHECK();
-    return TERNEL_TQ1_OK;
+    return launch_interleave<false>(blocks, rows, columns, packed, nullptr, stream);
+}
+
+int ternel_tq1_interleave_checked(const uint8_t *blocks, int64_t rows, int64_t columns, uint32_t *packed,
+                                  uint64_t *counters, void *stream) {
+    return launch_interleave<true>(blocks, rows, columns, packed, counters, stream);
 }
 
 static int check_tiled(int64_t rows, int64_t columns, int64_t tile) {

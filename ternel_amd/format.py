@@ -113,7 +113,10 @@ def validate_blocks(blocks) -> None:
 
 def validate_packed_codes(blocks) -> None:
     """Load-time full scan with the message of src/ternel_mlx/packing.py:29-48."""
-    regular, tail = count_invalid_bytes(blocks)
+    check_packed_code_counts(*count_invalid_bytes(blocks))
+
+
+def check_packed_code_counts(regular: int, tail: int) -> None:
     if regular or tail:
         raise FormatError(
             f"packed codes contain out-of-range base-3 bytes: regular={regular} "

@@ -34,7 +34,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .format import BLOCK_BYTES, BLOCK_SIZE, CODE_SLOTS, FormatError, as_device_blocks
+from .format import BLOCK_BYTES, BLOCK_SIZE, CODE_SLOTS, FormatError, as_device_blocks, check_packed_code_counts
 from .layout import PackedTensorLayout
 
 ACTIVATION_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
@@ -150,17 +150,27 @@ def packed_shape(layout: PackedTensorLayout) -> tuple[int, int, int, int]:
     return (math.ceil(layout.rows / TILE_ROWS), layout.groups_per_row, BLOCK_WORDS, TILE_ROWS)
 
 
-def pack_weights(blocks, *, layout: PackedTensorLayout) -> torch.Tensor:
-    """Canonical blocks (host or device) -> packed device words (exact permutation)."""
+def pack_weights(blocks, *, layout: PackedTensorLayout, validate: bool = False) -> torch.Tensor:
+    """Canonical blocks (host or device) -> packed device words (exact permutation);
+    with ``validate`` every byte is scanned on the way and the reference's
+    ``validate_packed_codes`` error raised when any is out of range."""
     device_blocks = as_device_blocks(blocks)
     if device_blocks.shape[0] != layout.groups:
         raise FormatError(
             f"expected {layout.groups} blocks for {layout.rows}x{layout.columns}, got {device_blocks.shape[0]}"
         )
     packed = torch.empty(packed_shape(layout), dtype=torch.int32, device=device_blocks.device)
-    assert packed.numel() == _lib.lib().ternel_tq1_packed_words(layout.rows, layout.columns)
-    _lib.check(_lib.lib().ternel_tq1_interleave(device_blocks.data_ptr(), layout.rows, layout.columns,
-                                                packed.data_ptr(), _stream(device_blocks.device)))
+    handle = _lib.lib()
+    assert packed.numel() == handle.ternel_tq1_packed_words(layout.rows, layout.columns)
+    stream = _stream(device_blocks.device)
+    if not validate:
+        _lib.check(handle.ternel_tq1_interleave(device_blocks.data_ptr(), layout.rows, layout.columns,
+                                                packed.data_ptr(), stream))
+        return packed
+    counters = torch.empty(2, dtype=torch.int64, device=device_blocks.device)
+    _lib.check(handle.ternel_tq1_interleave_checked(device_blocks.data_ptr(), layout.rows, layout.columns,
+                                                    packed.data_ptr(), counters.data_ptr(), stream))
+    check_packed_code_counts(*counters.tolist())
     return packed
 
 
@@ -553,14 +563,7 @@ def words_from_tiled(codes: torch.Tensor, scales: torch.Tensor, *, layout: Packe
         codes.data_ptr(), scales.data_ptr(), layout.rows, layout.columns, layout.tile, packed.data_ptr(),
         counters.data_ptr(), _stream(codes.device)))
     if validate:
-        regular, tail = (int(v) for v in counters.cpu())
-        if regular or tail:
-            from .format import MAX_FULL_CODE_BYTE, MAX_TAIL_CODE_BYTE
-
-            raise FormatError(
-                f"packed codes contain out-of-range base-3 bytes: regular={regular} "
-                f"(max {MAX_FULL_CODE_BYTE}), tail={tail} (max {MAX_TAIL_CODE_BYTE})"
-            )
+        check_packed_code_counts(*counters.tolist())
     return packed
 
 

@@ -28,7 +28,7 @@ import numpy as np
 import torch
 from torch import nn
 
-from .format import BLOCK_BYTES, FormatError, as_device_blocks, validate_packed_codes
+from .format import BLOCK_BYTES, FormatError, as_device_blocks
 from .kernels import (
     GemmConfig,
     MatmulConfig,
@@ -113,8 +113,8 @@ class _PackedWeight(nn.Module):
     def load_blocks(self, blocks, *, validate: bool = True) -> None:
         """Load canonical blocks (any shape holding ``rows * G`` 28-byte blocks).
 
-        Every byte is scanned on the GPU first (fail-closed), then the blocks are
-        permuted into the packed words.
+        Every byte is scanned on the GPU (fail-closed) as the blocks are permuted
+        into the packed words, which replace the module's only if all are legal.
         """
         tensor = as_device_blocks(blocks)
         if tensor.shape[0] != self.layout.groups:
@@ -122,9 +122,7 @@ class _PackedWeight(nn.Module):
                 f"expected {self.layout.groups} blocks for {self.layout.rows}x{self.layout.columns}, "
                 f"got {tensor.shape[0]}"
             )
-        if validate:
-            validate_packed_codes(tensor)
-        self.packed = pack_weights(tensor, layout=self.layout)
+        self.packed = pack_weights(tensor, layout=self.layout, validate=validate)
 
     def load_packed(self, codes, scales, *, validate: bool = True) -> None:
         """Load the reference's tiled ``codes`` (u8) / ``scales`` (<u2) arrays:
