@@ -50,7 +50,10 @@
  * counters as NaN without touching them. The LUT23, direct-form and strip
  * kernels do not read the word, and their results on a workspace whose
  * counters were left set are not defined. Zero the workspace again before
- * any further call on it.
+ * any further call on it. 32-bit words 16380 and 16381 of the region may hold
+ * the address (low half first) of a 32-bit word the host can read, in pinned
+ * memory that outlives the workspace: such a kernel writes the error word's
+ * value there too, so that the host can notice without a copy. Zero: none.
  */
 #ifndef TERNEL_TQ1_H
 #define TERNEL_TQ1_H

@@ -33,7 +33,6 @@
 #include <atomic>
 #include <mutex>
 #include <set>
-#include <string>
 #include <utility>
 #include <type_traits>
 
@@ -72,6 +71,9 @@ constexpr int kThreads = 256;
 // error word (the host section keeps every kernel's counters below it).
 constexpr int kWorkspaceCounterBytes = 64 * 1024;
 constexpr int kWorkspaceErrorSlot = kWorkspaceCounterBytes / 4 - 1;
+// Slots 16380 and 16381 may hold the address of a 32-bit word that the host
+// reads (pinned memory), to which a give-up is written too; 0 for none.
+constexpr int kWorkspaceHostWordSlot = kWorkspaceErrorSlot - 3;
 
 // Phase timestamps (built only with -DTERNEL_TQ1_PROFILE, into a separate
 // library that bench.py --phase-profile loads): lane 0 of each wave of the
@@ -2839,8 +2841,14 @@ __global__ __launch_bounds__(kWideThreads) void wide_gemm_kernel(
                 __builtin_amdgcn_s_sleep(2);
             }
             s_published = published;
-            if (!published)
+            if (!published) {
                 __hip_atomic_fetch_or(counters + kWorkspaceErrorSlot, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint64_t address = counters[kWorkspaceHostWordSlot] |
+                                         (static_cast<uint64_t>(counters[kWorkspaceHostWordSlot + 1]) << 32);
+                if (address)
+                    __hip_atomic_store(reinterpret_cast<unsigned *>(address), 2u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_SYSTEM);
+            }
         }
         __syncthreads();
         TQ1_PHASE(wide_wave_id, 7);
@@ -3389,9 +3397,14 @@ int launch_strip(const uint32_t *packed, const void *x, void *y, const StripGeom
 bool uses_strip_gemv(int64_t M, int batch_tile, int k_split, int64_t rows, int64_t columns, bool allow_split = true) {
     if (M != 1 || batch_tile != 0 || k_split != 0 || rows < kStripMinRows) return false;
     StripGeometry geo;
-    const std::string saved = g_last_error;
+    char saved[sizeof(g_last_error)];  // a refusal here is not the caller's error
+    const bool had = g_last_error[0] != '\0';
+    if (had) memcpy(saved, g_last_error, sizeof(saved));
     const bool ok = plan_strip(rows, columns, &geo, allow_split) == TERNEL_TQ1_OK;
-    snprintf(g_last_error, sizeof(g_last_error), "%s", saved.c_str());
+    if (had)
+        memcpy(g_last_error, saved, sizeof(saved));
+    else
+        g_last_error[0] = '\0';
     return ok;
 }
 
@@ -3603,10 +3616,12 @@ int wide_blocks(int64_t M, int64_t tiles_n, int64_t groups, int64_t cus) {
     return nb == 8 && 10 * (cus - tiles) * cus > tiles * tiles * groups ? 4 : nb;
 }
 int device_cu_count() {
+    static std::atomic<int> known[64];  // per device, 0 until queried
     int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        return 256;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    if (dev >= 0 && dev < 64 && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
+    if (dev >= 0 && dev < 64) known[dev].store(cus, std::memory_order_relaxed);
     return cus;
 }
 

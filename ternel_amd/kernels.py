@@ -21,11 +21,19 @@ tensors in the activation dtype.
 Split-K workspaces: kernels that reduce K chunks inside the launch use arrival
 counters and piece slots that start at zero and are left at zero, so each
 (device, stream) gets one zero-filled workspace, reused.
+
+A small product takes 4-10 us on the GPU, so a call's host work is kept below
+that: what depends on sizes alone (shapes, the kernel, its workspace) is looked
+up per size, the raw stream is read without building a stream object, and a
+give-up is noticed from a host word (``_surface``). A module call takes 8.5 us
+of host time (3.5 of them the launch) where it took 15, and 9.5 where the wide
+form might run, which took 50.
 """
 
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import weakref
 from collections import OrderedDict
@@ -84,8 +92,7 @@ class MatmulConfig:
 
 GEMM_FORMS = {"auto": 0, "tile": 1, "direct": 2, "wide": 3}
 DIRECT_MAX_BATCH = 64
-# The automatic GEMM form may be the wide one above this many activation rows.
-WIDE_MIN_AUTO_BATCH = 32
+KERNEL_LUT23 = 100  # ternel_tq1_linear_kernel's answer for the matmul path
 
 
 @dataclass(frozen=True)
@@ -142,12 +149,52 @@ class GemmConfig:
         return name if self.k_split in (0, 1) else f"{name}_k{self.k_split}"
 
 
+def _device_index(device: torch.device) -> int:
+    return device.index if device.index is not None else torch.cuda.current_device()
+
+
+# The current stream's handle of a device, without the Stream object that
+# torch.cuda.current_stream builds (2 us).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(torch.device("cuda", index)).cuda_stream)
+
+
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(_device_index(device))
+
+
+@functools.lru_cache(maxsize=4096)
+def _packed_shape(rows: int, columns: int) -> torch.Size:
+    return torch.Size((math.ceil(rows / TILE_ROWS), columns // BLOCK_SIZE, BLOCK_WORDS, TILE_ROWS))
 
 
 def packed_shape(layout: PackedTensorLayout) -> tuple[int, int, int, int]:
-    return (math.ceil(layout.rows / TILE_ROWS), layout.groups_per_row, BLOCK_WORDS, TILE_ROWS)
+    return tuple(_packed_shape(layout.rows, layout.columns))
+
+
+# What the library answers for sizes alone, per device (the kernels are chosen
+# by its CU count).
+@functools.lru_cache(maxsize=4096)
+def _matmul_bytes(index: int, batch: int, rows: int, columns: int, batch_tile: int, k_split: int) -> int:
+    return _lib.lib().ternel_tq1_matmul_workspace_bytes(batch, rows, columns, batch_tile, k_split)
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_bytes(index: int, batch: int, rows: int, columns: int, form: int, k_split: int) -> int:
+    return _lib.lib().ternel_tq1_gemm_workspace_bytes(batch, rows, columns, form, k_split)
+
+
+@functools.lru_cache(maxsize=4096)
+def _linear_plan(index: int, batch: int, rows: int, columns: int, code: int) -> tuple[int, int]:
+    """(ternel_tq1_linear_kernel, workspace bytes) of a linear."""
+    handle = _lib.lib()
+    return (handle.ternel_tq1_linear_kernel(batch, rows, columns, code),
+            handle.ternel_tq1_linear_workspace_bytes(batch, rows, columns, code))
+
+
+@functools.lru_cache(maxsize=4096)
+def _swiglu_bytes(index: int, batch: int, rows: int, columns: int, code: int) -> int:
+    return _lib.lib().ternel_tq1_swiglu_workspace_bytes(batch, rows, columns, code)
 
 
 def pack_weights(blocks, *, layout: PackedTensorLayout, validate: bool = False) -> torch.Tensor:
@@ -188,7 +235,7 @@ def check_packed(packed: torch.Tensor, *, layout: PackedTensorLayout) -> torch.T
         raise FormatError("packed weights must be a torch tensor on the GPU")
     if packed.dtype not in (torch.int32, torch.uint32):
         raise FormatError(f"packed weights must be 32-bit words, got {packed.dtype}")
-    if tuple(packed.shape) != packed_shape(layout):
+    if packed.shape != _packed_shape(layout.rows, layout.columns):
         raise FormatError(f"packed weights of shape {tuple(packed.shape)} do not match {packed_shape(layout)}")
     if not packed.is_cuda:
         raise FormatError("packed weights must live on the GPU")
@@ -231,11 +278,6 @@ def _aligned_rows(x: torch.Tensor) -> torch.Tensor:
     return x
 
 
-def _workspace_key(device: torch.device) -> tuple[int, int]:
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    return index, torch.cuda.current_stream(torch.device("cuda", index)).cuda_stream
-
-
 def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
     """Zero-initialised split-K scratch, one per (device, stream), grown on demand.
 
@@ -245,23 +287,29 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
     stream run in order, so they can share its buffer; calls on two streams
     get two buffers and never race on each other's counters.
     """
+    global _FLAG_WORDS
     if nbytes == 0:
         return None
-    key = _workspace_key(device)
+    index = _device_index(device)
+    key = (index, _raw_stream(index))
     capturing = torch.cuda.is_current_stream_capturing()
     buf = _WORKSPACES.get(key)
     if capturing and (buf is None or buf.numel() < nbytes):
         # A capture stream (torch.cuda.graph captures on a side stream) borrows
         # the device's largest eager workspace: replays then share it with that
         # stream's eager calls, which must not run at the same time.
-        sized = [k for k, b in _WORKSPACES.items() if k[0] == key[0] and b.numel() >= nbytes]
+        sized = [k for k, b in _WORKSPACES.items() if k[0] == index and b.numel() >= nbytes]
         if not sized:
             raise RuntimeError("split-K workspace must be sized by an eager call before graph capture")
         key = max(sized, key=lambda k: _WORKSPACES[k].numel())
         buf = _WORKSPACES[key]
     if buf is None or buf.numel() < nbytes:
-        new = torch.zeros(max(nbytes, 1 << 22), dtype=torch.uint8, device=torch.device("cuda", key[0]))
-        torch.cuda.synchronize(key[0])
+        new = torch.empty(max(nbytes, 1 << 22), dtype=torch.uint8, device=torch.device("cuda", index))
+        if key not in _FLAGS:
+            _FLAGS[key] = _HostWord()
+            _FLAG_WORDS = tuple((k[0], f.word) for k, f in _FLAGS.items())
+        _reset(new, key)
+        torch.cuda.synchronize(index)
         if buf is not None and key in _CAPTURED:
             _RETIRED.append(buf)
         _WORKSPACES[key] = buf = new
@@ -270,66 +318,48 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
     return buf
 
 
-# Launches that may give up a bounded wait (the wide form's stream-K
-# reduction) leave an event per workspace; the next call on the device reads
-# the error word of every workspace whose event has completed -- no wait on
-# the caller's stream, a 4-byte copy on a side stream -- and raises
-# ``NativeError`` if it is set, after zeroing that workspace. (The kernels
-# themselves refuse a workspace whose word is set: they write the tiles that
-# would need its counters as NaN.) Graph replays are not watched; a caller
-# replaying graphs runs ``check_workspaces()`` at its own sync points.
-_WATCH: dict[tuple[int, int], torch.cuda.Event] = {}
-_SIDE: dict[int, torch.cuda.Stream] = {}
-_ERROR_WORD_OFFSET = 64 * 1024 - 4  # the last word of the 64 KiB counter region
+# A kernel whose bounded wait gives up (the wide form's stream-K reduction)
+# sets its workspace's error word and writes the same value to a pinned host
+# word whose address the workspace carries, so the next call on the device
+# notices by reading host memory. (An event per launch and a 4-byte copy on a
+# side stream at the next call, which this replaces, cost 30 us of host time a
+# call.) Graph replays report here too.
+class _HostWord:
+    def __init__(self) -> None:
+        self.tensor = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self.word = ctypes.c_int.from_address(self.tensor.data_ptr())
 
 
-def _key_of(buf: torch.Tensor) -> tuple[int, int] | None:
-    for key, b in _WORKSPACES.items():
-        if b is buf:
-            return key
-    return None
+_FLAGS: dict[tuple[int, int], _HostWord] = {}
+_FLAG_WORDS: tuple[tuple[int, ctypes.c_int], ...] = ()  # (device, host word) of each, replaced as one
+_HOST_WORD_OFFSET = 64 * 1024 - 16  # in the counter region, before the error word
 
 
-def _watch(ws: torch.Tensor | None, may_give_up: bool) -> None:
-    """After a launch: remember to read ``ws``'s error word once it is done."""
-    if ws is None or not may_give_up or torch.cuda.is_current_stream_capturing():
+def _reset(buf: torch.Tensor, key: tuple[int, int]) -> None:
+    """A workspace as it is handed out: zero but for its host word's address."""
+    flag = _FLAGS[key]
+    buf.zero_()
+    buf[_HOST_WORD_OFFSET:_HOST_WORD_OFFSET + 8].view(torch.int64).fill_(flag.tensor.data_ptr())
+    flag.word.value = 0
+
+
+def _surface(index: int) -> None:
+    """Before a launch: raise if a workspace of the device reported a wait that
+    gave up (zeroing it first, so the next call starts clean)."""
+    for device, word in _FLAG_WORDS:
+        if word.value and device == index:
+            break
+    else:
         return
-    key = _key_of(ws)
-    if key is None:
+    if torch.cuda.is_current_stream_capturing():
         return
-    event = torch.cuda.Event()
-    event.record(torch.cuda.current_stream(ws.device))
-    _WATCH[key] = event
-
-
-def _surface(device: torch.device) -> None:
-    """Before a launch: raise if a watched workspace of ``device`` reported a
-    wait that gave up (zeroing it first, so the next call starts clean)."""
-    if not _WATCH or torch.cuda.is_current_stream_capturing():
-        return
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    failed = {}
-    for key, event in list(_WATCH.items()):
-        if key[0] != index or not event.query():
-            continue
-        del _WATCH[key]
-        buf = _WORKSPACES[key]
-        side = _SIDE.get(index)
-        if side is None:
-            side = _SIDE[index] = torch.cuda.Stream(device=buf.device)
-        word = torch.empty(4, dtype=torch.uint8, pin_memory=True)
-        with torch.cuda.stream(side):
-            side.wait_event(event)
-            word.copy_(buf[_ERROR_WORD_OFFSET:_ERROR_WORD_OFFSET + 4], non_blocking=True)
-        side.synchronize()
-        value = int(word.view(torch.int32).item())
-        if value:
-            buf.zero_()
-            failed[key] = value
-    if failed:
-        torch.cuda.synchronize(index)
-        raise _lib.NativeError(f"a kernel's bounded wait for a published partial gave up: {failed}; "
-                               "its tiles were written as NaN and the workspace has been zeroed")
+    torch.cuda.synchronize(index)  # the launch that reported may still be running
+    failed = {k: f.word.value for k, f in list(_FLAGS.items()) if k[0] == index and f.word.value}
+    for key in failed:
+        _reset(_WORKSPACES[key], key)
+    torch.cuda.synchronize(index)
+    raise _lib.NativeError(f"a kernel's bounded wait for a published partial gave up: {failed}; "
+                           "its tiles were written as NaN and the workspace has been zeroed")
 
 
 def workspace_errors() -> dict[tuple[int, int], int]:
@@ -352,9 +382,8 @@ def check_workspaces() -> None:
     workspace is zeroed again first (its counters may be left set), so the
     next call starts clean."""
     failed = {key: word for key, word in workspace_errors().items() if word}
-    _WATCH.clear()
     for key in failed:
-        _WORKSPACES[key].zero_()
+        _reset(_WORKSPACES[key], key)
     if failed:
         torch.cuda.synchronize()
         raise _lib.NativeError(f"a kernel's bounded wait for a published partial gave up: {failed}")
@@ -373,15 +402,14 @@ def tq1_matmul_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTen
             f"k split {config.k_split} does not divide the tensor's {layout.groups_per_row} groups per row"
         )
     x = x.contiguous()
-    out = torch.empty((batch, layout.rows), dtype=x.dtype, device=x.device)
-    handle = _lib.lib()
-    need = handle.ternel_tq1_matmul_workspace_bytes(batch, layout.rows, layout.columns,
-                                                     config.batch_tile, config.k_split)
-    ws = workspace(x.device, need)
-    _lib.check(handle.ternel_tq1_matmul(
+    out = x.new_empty((batch, layout.rows))
+    index = x.get_device()
+    ws = workspace(x.device, _matmul_bytes(index, batch, layout.rows, layout.columns, config.batch_tile,
+                                           config.k_split))
+    _lib.check(_lib.lib().ternel_tq1_matmul(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns,
         _DTYPE_CODE[x.dtype], config.batch_tile, config.k_split,
-        ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream(x.device)))
+        ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _raw_stream(index)))
     return out
 
 
@@ -392,9 +420,10 @@ def tq1_gemm_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTenso
     fp16 activations run the form ``config`` names. bf16 ones run on bf16
     operands in small batches and the wide form above them, each row scaled by
     a power of two into fp16's range (exact: bf16's significand fits fp16's)
-    and the fp32 sums scaled back and rounded once to bf16. fp32 activations -- whose significand fp16 would not hold -- and bf16
-    ones with a fixed K split run through the LUT23 kernel, which computes in
-    fp32 from the activations as given."""
+    and the fp32 sums scaled back and rounded once to bf16. fp32 activations --
+    whose significand fp16 would not hold -- and bf16 ones with a fixed K split
+    run through the LUT23 kernel, which computes in fp32 from the activations
+    as given."""
     config = config or GemmConfig()
     check_packed(packed, layout=layout)
     batch = check_activations(x, layout=layout)
@@ -414,34 +443,48 @@ def tq1_gemm_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTenso
         raise FormatError(f"the direct-fragment form takes at most {DIRECT_MAX_BATCH} activation rows, got {batch}")
     form = GEMM_FORMS[form_name]
     x = _aligned_rows(x)
-    _surface(x.device)
-    out = torch.empty((batch, layout.rows), dtype=x.dtype, device=x.device)
-    handle = _lib.lib()
-    need = handle.ternel_tq1_gemm_workspace_bytes(batch, layout.rows, layout.columns, form, config.k_split)
-    ws = workspace(x.device, need)
-    _lib.check(handle.ternel_tq1_gemm(
+    index = x.get_device()
+    _surface(index)
+    out = x.new_empty((batch, layout.rows))
+    ws = workspace(x.device, _gemm_bytes(index, batch, layout.rows, layout.columns, form, config.k_split))
+    _lib.check(_lib.lib().ternel_tq1_gemm(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns,
         _DTYPE_CODE[x.dtype], form, config.k_split, ws.data_ptr() if ws is not None else None,
-        ws.numel() if ws is not None else 0, _stream(x.device)))
-    _watch(ws, form_name == "wide" or (form_name == "auto" and batch > WIDE_MIN_AUTO_BATCH))
+        ws.numel() if ws is not None else 0, _raw_stream(index)))
     return out
 
 
 def tq1_linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout) -> torch.Tensor:
     """The library's own dispatch (``ternel_tq1_linear``) for a 2-D ``x``."""
     check_packed(packed, layout=layout)
-    batch = check_activations(x, layout=layout)
-    x = _aligned_rows(x)
-    _surface(x.device)
-    out = torch.empty((batch, layout.rows), dtype=x.dtype, device=x.device)
-    handle = _lib.lib()
-    code = _DTYPE_CODE[x.dtype]
-    need = handle.ternel_tq1_linear_workspace_bytes(batch, layout.rows, layout.columns, code)
-    ws = workspace(x.device, need)
-    _lib.check(handle.ternel_tq1_linear(
+    check_activations(x, layout=layout)
+    return _linear(packed, _aligned_rows(x), layout)
+
+
+def linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout) -> torch.Tensor:
+    """The same for ``x`` with any leading dimensions, which the result keeps:
+    the modules' product (src/ternel_mlx/modules.py:425-457)."""
+    if x.shape[-1] != layout.columns:
+        raise FormatError(f"activation has {x.shape[-1]} columns, weight expects {layout.columns}")
+    flat = x if x.ndim == 2 else x.reshape(-1, layout.columns)
+    code = _DTYPE_CODE[flat.dtype]
+    if flat.shape[0] <= 0:
+        raise FormatError("activations have an empty batch dimension")
+    check_packed(packed, layout=layout)
+    check_activations(flat, layout=layout)
+    lut = _linear_plan(flat.get_device(), flat.shape[0], layout.rows, layout.columns, code)[0] == KERNEL_LUT23
+    out = _linear(packed, flat.contiguous() if lut else _aligned_rows(flat), layout)
+    return out if x.ndim == 2 else out.reshape(*x.shape[:-1], layout.rows)
+
+
+def _linear(packed: torch.Tensor, x: torch.Tensor, layout: PackedTensorLayout) -> torch.Tensor:
+    batch, code, index = x.shape[0], _DTYPE_CODE[x.dtype], x.get_device()
+    _surface(index)
+    out = x.new_empty((batch, layout.rows))
+    ws = workspace(x.device, _linear_plan(index, batch, layout.rows, layout.columns, code)[1])
+    _lib.check(_lib.lib().ternel_tq1_linear(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns, code,
-        ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream(x.device)))
-    _watch(ws, handle.ternel_tq1_linear_kernel(batch, layout.rows, layout.columns, code) == GEMM_FORMS["wide"])
+        ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _raw_stream(index)))
     return out
 
 
@@ -456,16 +499,14 @@ def tq1_swiglu_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTen
         raise FormatError(f"a SwiGLU weight interleaves gate and up rows, so its rows must be even, "
                           f"got {layout.rows}")
     x = _aligned_rows(x)
-    _surface(x.device)
-    out = torch.empty((batch, layout.rows // 2), dtype=x.dtype, device=x.device)
-    handle = _lib.lib()
+    index = x.get_device()
+    _surface(index)
+    out = x.new_empty((batch, layout.rows // 2))
     code = _DTYPE_CODE[x.dtype]
-    need = handle.ternel_tq1_swiglu_workspace_bytes(batch, layout.rows, layout.columns, code)
-    ws = workspace(x.device, need)
-    _lib.check(handle.ternel_tq1_swiglu(
+    ws = workspace(x.device, _swiglu_bytes(index, batch, layout.rows, layout.columns, code))
+    _lib.check(_lib.lib().ternel_tq1_swiglu(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns, code,
-        ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream(x.device)))
-    _watch(ws, handle.ternel_tq1_linear_kernel(batch, layout.rows, layout.columns, code) == GEMM_FORMS["wide"])
+        ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _raw_stream(index)))
     return out
 
 
@@ -476,8 +517,10 @@ def _gather_ids(indices: torch.Tensor, dtype: torch.dtype, device) -> torch.Tens
         raise FormatError(f"indices must be 1-D, got shape {tuple(indices.shape)}")
     if indices.numel() <= 0:
         raise FormatError("indices are empty")
-    if indices.dtype not in (torch.int8, torch.int16, torch.int32, torch.int64, torch.uint8, torch.uint32):
+    if indices.dtype not in (torch.int64, torch.int32, torch.int16, torch.int8, torch.uint8, torch.uint32):
         raise FormatError(f"indices must be an integer tensor, got {indices.dtype}")
+    if indices.dtype == torch.int64 and indices.device == device:
+        return indices.contiguous()
     return indices.to(device=device, dtype=torch.int64).contiguous()
 
 
@@ -488,10 +531,10 @@ def tq1_get_rows_words(packed: torch.Tensor, indices: torch.Tensor, *, layout: P
     (src/ternel_mlx/kernels.py:869-880)."""
     check_packed(packed, layout=layout)
     ids = _gather_ids(indices, dtype, packed.device)
-    out = torch.empty((ids.numel(), layout.columns), dtype=dtype, device=packed.device)
+    out = packed.new_empty((ids.numel(), layout.columns), dtype=dtype)
     _lib.check(_lib.lib().ternel_tq1_get_rows(
         packed.data_ptr(), layout.rows, layout.columns, ids.data_ptr(), ids.numel(), out.data_ptr(),
-        _DTYPE_CODE[dtype], _stream(packed.device)))
+        _DTYPE_CODE[dtype], _raw_stream(packed.get_device())))
     return out
 
 

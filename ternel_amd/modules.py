@@ -30,15 +30,12 @@ from torch import nn
 
 from .format import BLOCK_BYTES, FormatError, as_device_blocks
 from .kernels import (
-    GemmConfig,
-    MatmulConfig,
+    linear_words,
     pack_weights,
     packed_shape,
     tiled_from_words,
-    tq1_gemm_words,
     tq1_get_rows_canonical,
     tq1_get_rows_words,
-    tq1_matmul_words,
     tq1_swiglu_words,
     unpack_weights,
     words_from_tiled,
@@ -69,16 +66,9 @@ def select_kernel(layout: PackedTensorLayout, batch: int, dtype: torch.dtype) ->
 
 
 def matmul_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout) -> torch.Tensor:
-    """``x @ W.T`` for packed words ``W``, choosing the kernel by activation rows
-    and keeping the leading dimensions of ``x``."""
-    if x.shape[-1] != layout.columns:
-        raise FormatError(f"activation has {x.shape[-1]} columns, weight expects {layout.columns}")
-    flat = x.reshape(-1, layout.columns)
-    if select_kernel(layout, flat.shape[0], flat.dtype) == "gemm":
-        out = tq1_gemm_words(packed, flat, layout=layout, config=GemmConfig())
-    else:
-        out = tq1_matmul_words(packed, flat, layout=layout, config=MatmulConfig())
-    return out.reshape(*x.shape[:-1], layout.rows)
+    """``x @ W.T`` for packed words ``W``, the library choosing the kernel by
+    activation rows, keeping the leading dimensions of ``x``."""
+    return linear_words(packed, x, layout=layout)
 
 
 def packed_matmul(codes: torch.Tensor, scales: torch.Tensor, x: torch.Tensor, *,
@@ -275,7 +265,7 @@ class PackedLinear(_PackedWeight):
                 f"{self.layout.bits_per_weight:.3f} bits/weight")
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return matmul_words(self.packed, x, layout=self.layout)
+        return linear_words(self.packed, x, layout=self.layout)
 
 
 class PackedEmbedding(_PackedWeight):
@@ -321,12 +311,12 @@ class PackedEmbedding(_PackedWeight):
     def forward(self, indices: torch.Tensor) -> torch.Tensor:
         """Rows for ``indices`` of any shape and integer dtype; ids outside the
         table read as zeros (src/ternel_mlx/modules.py:527-545)."""
-        flat = indices.reshape(-1)
+        flat = indices if indices.ndim == 1 else indices.reshape(-1)
         if self.canonical_rows:
             rows = tq1_get_rows_canonical(self.row_blocks(), flat, layout=self.layout, dtype=self.dtype)
         else:
             rows = tq1_get_rows_words(self.packed, flat, layout=self.layout, dtype=self.dtype)
-        return rows.reshape(*indices.shape, self.layout.columns)
+        return rows if indices.ndim == 1 else rows.reshape(*indices.shape, self.layout.columns)
 
     def row_blocks(self) -> torch.Tensor:
         """The table as canonical ``(rows, G, 28)`` device blocks (``canonical_rows``),
@@ -345,7 +335,7 @@ class PackedEmbedding(_PackedWeight):
 
     def as_linear(self, x: torch.Tensor) -> torch.Tensor:
         """Tied output head: the embedding table used as a matmul."""
-        return matmul_words(self.packed, x, layout=self.layout)
+        return linear_words(self.packed, x, layout=self.layout)
 
 
 class PackedSwiGLU(nn.Module):
@@ -405,6 +395,8 @@ class PackedSwiGLU(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if x.shape[-1] != self.layout.columns:
             raise FormatError(f"activations have {x.shape[-1]} columns, expected {self.layout.columns}")
+        if x.ndim == 2:
+            return tq1_swiglu_words(self.packed, x, layout=self.layout)
         flat = x.reshape(-1, self.layout.columns)
         return tq1_swiglu_words(self.packed, flat, layout=self.layout).reshape(*x.shape[:-1], self.hidden)
 
