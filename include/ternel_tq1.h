@@ -231,11 +231,17 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
  *                          16 MiB of packed weights); WIDE up to M = 64;
  *                          above, WIDE when it has at least CUs/4 output
  *                          tiles or 15 (tile, group) steps per CU, TILE
- *                          otherwise (and for a fixed k_split > 1).
+ *                          otherwise (and for a fixed k_split > 1). With no
+ *                          k_split, larger batches on small matrices (under
+ *                          4 MiB up to M = 768; under 12 MiB, rows of at most
+ *                          64 groups, up to M = 384) run the DIRECT form's
+ *                          kernel on batch tiles of up to 64 rows in place of
+ *                          either.
  * bf16 activations (dtype TERNEL_TQ1_BF16) take form AUTO or WIDE and no fixed
  * k_split (size the workspace with form WIDE). Up to 32 rows (64 for matrices
- * under 24 MiB of packed weights) they run the DIRECT form's kernel on bf16
- * MFMAs, as they are; above, the WIDE form after a pre-pass that
+ * under 24 MiB of packed weights, 128 on long rows, 512 under 12 MiB and 768
+ * under 4 MiB) they run the DIRECT form's kernel on bf16 MFMAs, as they are;
+ * above, the WIDE form after a pre-pass that
  * scales each row by a power of two into fp16's range and converts it (exact:
  * bf16's 8-bit significand fits fp16's 11 bits; values more than 2^28 below
  * the row's largest lose bits), and the fp32 sums are scaled back and rounded
@@ -286,8 +292,9 @@ size_t ternel_tq1_linear_workspace_bytes(int64_t M, int64_t rows, int64_t column
 /*
  * The path ternel_tq1_linear takes for this shape: TERNEL_TQ1_KERNEL_LUT23
  * (ternel_tq1_matmul, with its automatic choice of kernel) or one of the
- * TERNEL_TQ1_GEMM_* forms of ternel_tq1_gemm (never AUTO; WIDE for every bf16
- * batch it takes); negative on a rejected shape or dtype. Host-only, touches no device. The counterpart of the
+ * TERNEL_TQ1_GEMM_* forms of ternel_tq1_gemm, as its automatic form names them
+ * (never AUTO; WIDE for every bf16 batch it takes); negative on a rejected
+ * shape or dtype. Host-only, touches no device. The counterpart of the
  * reference's select_gemm / select_lut23 decisions (src/ternel_mlx/modules.py
  * :320-423), exposed so that a dispatch sweep can be replayed through the rule.
  */

@@ -126,7 +126,8 @@ int fail(int code, const char *fmt, ...) {
 
 // ---------------------------------------------------------------------------
 // Scalar conversions. fp16 via _Float16 (v_cvt_f32_f16 keeps subnormals, inf
-// and NaN); bf16 by bit manipulation with round-to-nearest-even.
+// and NaN); bf16 widened by a shift, narrowed by gfx950's instruction (round to
+// nearest even, subnormals, inf and NaN kept).
 // ---------------------------------------------------------------------------
 struct bf16_t {
     uint16_t bits;
@@ -161,16 +162,8 @@ __device__ __forceinline__ _Float16 from_f32<_Float16>(float v) {
     return static_cast<_Float16>(v);
 }
 template <>
-__device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) {
-    uint32_t u = __float_as_uint(v);
-    bf16_t out;
-    if ((u & 0x7fffffffu) > 0x7f800000u) {
-        out.bits = static_cast<uint16_t>((u >> 16) | 0x0040u);  // quiet NaN, sign kept
-    } else {
-        u += 0x7fffu + ((u >> 16) & 1u);
-        out.bits = static_cast<uint16_t>(u >> 16);
-    }
-    return out;
+__device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) {  // v_cvt_pk_bf16_f32
+    return bf16_t{__builtin_bit_cast(uint16_t, static_cast<__bf16>(v))};
 }
 template <>
 __device__ __forceinline__ float from_f32<float>(float v) {
@@ -1697,7 +1690,8 @@ __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (
 
 // ---------------------------------------------------------------------------
 // trit_gemm_kernel: y = x @ W^T for small batches (M <= 32, or 64 with two
-// MFMA tiles) of fp16, bf16 and fp32 activations.
+// MFMA tiles) of fp16, bf16 and fp32 activations, and larger ones on small
+// matrices as tiles of that many rows.
 //
 // What bounds it: the decode. A wave turns 32 rows x one block into MFMA
 // operands while the words stream, so the loop is VALU and LDS issue, not
@@ -1864,7 +1858,7 @@ constexpr int trit_window(int value_bytes, int staged_rows) {
 template <typename T, int SR, bool MULTI>
 __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_kernel(
     const uint32_t *__restrict__ packed, const T *__restrict__ x, T *__restrict__ y, float *__restrict__ partial,
-    unsigned *__restrict__ counters, int M, int N, int G, int chunk_groups, int k_split, int flags) {
+    unsigned *__restrict__ counters, int M, int N, int G, int chunk_groups, int k_split, int tile_rows, int flags) {
     using Op = TritOperand<T>;
     constexpr int P = Op::kPlanes;
     constexpr int NB = SR > 32 ? 2 : 1;
@@ -1880,6 +1874,15 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
     __shared__ __align__(16) uint32_t pairs[tq1_bytes::kPairEntries];
     __shared__ unsigned s_last;
 
+    // Batch tile blockIdx.z: rows [z tile_rows, (z + 1) tile_rows) of x and y.
+    {
+        const int64_t m0 = static_cast<int64_t>(blockIdx.z) * tile_rows;
+        x += m0 * G * kBlockWeights;
+        y += m0 * ((flags & kTritGlu) ? N / 2 : N);
+        M = min(tile_rows, M - static_cast<int>(m0));
+    }
+    const int block = blockIdx.z * gridDim.x + blockIdx.x;  // of the partials and counters
+
     const int tid = threadIdx.x;
     if (tid < tq1_bytes::kPairEntries) pairs[tid] = tq1_bytes::pair_entry(tid, Op::kOne);
     const char *const tab = reinterpret_cast<const char *>(pairs);
@@ -1890,7 +1893,8 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
     const int g_begin = blockIdx.y * chunk_groups;
     const int cg = chunk_groups;
     const int64_t K = static_cast<int64_t>(G) * kBlockWeights;
-    const int direct_wave_id = (blockIdx.y * gridDim.x + blockIdx.x) * kDirectWaves + wave;
+    const int direct_wave_id =
+        ((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * kDirectWaves + wave;
     (void)direct_wave_id;
     TQ1_PHASE(direct_wave_id, 0);  // wave start
     TQ1_PHASE_XCC(direct_wave_id);
@@ -2084,9 +2088,9 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
         // Partials in quads: (chunk, wave, tile, quad) runs of 64 lanes x 16
         // bytes, the quads of real activation rows only.
         constexpr int kDeviceCoherent = 16;  // cache policy SC1
-        const int quads = NB == 1 ? (M + 7) >> 3 : 4;
+        const int quads = NB == 1 ? (tile_rows + 7) >> 3 : 4;
         const int wave_bytes = NB * quads * 1024;
-        const float *base = partial + static_cast<int64_t>(blockIdx.x) * k_split * (kDirectWaves * wave_bytes / 4) +
+        const float *base = partial + static_cast<int64_t>(block) * k_split * (kDirectWaves * wave_bytes / 4) +
                             wave * (wave_bytes / 4);
         const int chunk_bytes = kDirectWaves * wave_bytes;
         const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
@@ -2110,7 +2114,7 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
         asm volatile("" ::: "memory");
         TQ1_PHASE(direct_wave_id, 6);  // partial stored and acknowledged
         __syncthreads();
-        unsigned *counter = counters + blockIdx.x;
+        unsigned *counter = counters + block;
         if (tid == 0)
             s_last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
                      static_cast<unsigned>(k_split - 1);
@@ -3464,17 +3468,19 @@ constexpr int64_t kDirectMaxBatch = 64;
 // Auto split: at least this many workgroups (4 waves each) to fill 256 CUs twice.
 constexpr int64_t kDirectTargetWorkgroups = 512;
 // Fewer than this many workgroups of 8-group chunks: 4-group chunks.
-constexpr int64_t kDirectMinWorkgroups = 224;
+constexpr int64_t kDirectMinWorkgroups = 192;
 
 int direct_staged_rows(int64_t M) { return M <= 8 ? 8 : (M <= 16 ? 16 : (M <= 32 ? 32 : 64)); }
 
-// The trit kernel (trit_gemm_kernel): at most 64 rows of fp16 and bf16
-// activations, 32 of fp32, in one launch.
+// The trit kernel (trit_gemm_kernel): tiles of at most 64 rows of fp16 and
+// bf16 activations, 32 of fp32.
 struct TritPlan {
     int staged_rows;
     int k_split;
     int chunk_groups;
     int64_t row_blocks;
+    int64_t tile_rows;    // activation rows per batch tile
+    int64_t batch_tiles;  // in one launch
     int64_t launch_rows;  // activation rows per launch
     size_t partial_bytes;
 };
@@ -3485,46 +3491,77 @@ struct TritPlan {
 constexpr int64_t kTritPartialBytes = int64_t{64} << 20;
 constexpr int64_t kTritMatmulPartialBytes = int64_t{16} << 20;
 
-// batches: a batch past one launch's rows runs as several launches of nearly
-// equal size (ternel_tq1_matmul); otherwise it is refused.
-int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, TritPlan *plan, bool batches = false) {
+// batches: a batch past one tile runs as tiles of nearly equal size, in as
+// many launches as the counters and the partials' limit need; otherwise it is
+// refused.
+int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, TritPlan *plan, bool batches = false,
+              int64_t most_bytes = kTritPartialBytes) {
     const int64_t G = columns / kBlockWeights;
     const bool f32 = dtype == TERNEL_TQ1_F32;
     const int64_t most = f32 ? 32 : kDirectMaxBatch;
     if (M > most && !batches)
         return fail(TERNEL_TQ1_EINVAL, "the direct-fragment form takes at most %lld activation rows, got %lld",
                     static_cast<long long>(most), static_cast<long long>(M));
-    plan->launch_rows = ceil_div(M, ceil_div(M, most));
-    const int64_t m = plan->launch_rows;
+    const int64_t tiles = ceil_div(M, most);
+    const int64_t m = plan->tile_rows = ceil_div(M, tiles);
     plan->staged_rows = direct_staged_rows(m);
     plan->row_blocks = ceil_div(rows, kDirectRows);
     const int64_t quads = plan->staged_rows > 32 ? 8 : ceil_div(m, 8);
-    const int64_t split_bytes = plan->row_blocks * kDirectWaves * quads * 1024;
-    const int64_t most_bytes = batches ? kTritMatmulPartialBytes : kTritPartialBytes;
+    const int64_t split_bytes = plan->row_blocks * kDirectWaves * quads * 1024;  // one chunk of one tile
+    const int64_t blocks = plan->row_blocks * tiles;
     if (k_split < 0) return fail(TERNEL_TQ1_EINVAL, "k split must be positive, got %d", k_split);
     if (k_split == 0) {
         // The smallest split into chunks of a multiple of `granule` groups
         // that reaches the workgroup target, else the largest such split.
         // Chunks of 8 amortise a workgroup's start and its share of the
-        // reduction best where they still give about one workgroup per CU
-        // (M=8, us, 8 / 4 groups: out_proj, 240 workgroups, 8.7 / 8.9; QKV,
-        // 320, 9.9 / 10.5), chunks of 4 where they do not (4096 square, 128:
-        // 7.8 / 7.0; k_proj, 40: 7.2 / 6.2; 2 groups: 8.3, 7.9) and at 17-32
-        // rows, whose window is 4 groups (QKV M=32 13.8 / 13.5).
+        // reduction best where they still give most CUs a workgroup (us, 8 /
+        // 4 groups: out_proj M=8, 240 workgroups, 8.7 / 9.1, M=32 11.9 / 13.1;
+        // 1500 x 17408, 204, M=8 10.4 / 12.2), chunks of 4 where they do not
+        // (4096 square M=8, 128: 7.9 / 7.2; k_proj, 40: 7.2 / 6.3; 2 groups:
+        // 8.5, 8.0).
+        auto usable = [&](int64_t k, int64_t granule) {
+            return G % k == 0 && (G / k) % granule == 0 &&
+                   (k == 1 || (k * split_bytes <= most_bytes && plan->row_blocks <= kUsableCounters));
+        };
         auto widest = [&](int64_t granule) {
             int best = 0;
             for (int64_t k = 1; k <= G; ++k) {
-                if (G % k || (G / k) % granule) continue;
-                if (k > 1 && (k * split_bytes > most_bytes || plan->row_blocks > kUsableCounters)) break;
+                if (!usable(k, granule)) continue;
                 best = static_cast<int>(k);
-                if (plan->row_blocks * k >= kDirectTargetWorkgroups) break;
+                if (blocks * k >= kDirectTargetWorkgroups) break;
             }
             return best;
         };
-        int best = plan->staged_rows == 32 ? 0 : widest(8);
-        if (plan->row_blocks * best < kDirectMinWorkgroups) best = std::max(best, widest(4));
+        // 33-64 rows a tile: two workgroups per CU, whose loop the LDS bounds,
+        // so a second workgroup on a CU adds its groups' time and a third
+        // waits for a slot. The split of least estimated time, in us, fitted
+        // to sweeps of every split (seven shapes, M=64-384, within 10 %
+        // but for chunks too short to matter): a start, 0.82 per group for a
+        // CU's only workgroup or 0.66 for each of several, 8 per further round
+        // of two, 3 for a reduction.
+        auto fastest = [&]() {
+            const int64_t cus = device_cu_count();
+            int best = 0;
+            double least = 0;
+            for (int64_t k = 1; k <= G; ++k) {
+                if (!usable(k, 4)) continue;
+                const int64_t n = blocks * k, per_cu = ceil_div(n, cus), rounds = ceil_div(n, 2 * cus);
+                const double us = (k > 1 ? 8.0 : 5.0) +
+                                  static_cast<double>(G / k) * (per_cu == 1 ? 0.82 : 0.66 * static_cast<double>(per_cu)) +
+                                  (per_cu > 1 ? 1.5 : 0.0) + 8.0 * static_cast<double>(rounds - 1);
+                if (!best || us <= least) {
+                    best = static_cast<int>(k);
+                    least = us;
+                }
+            }
+            return best;
+        };
+        // (fp32 past 8 rows stages 4 or 2 groups at a time: QKV M=24 in chunks of
+        // 8 21.7 us, of 4 19.5; M=16 17.8 / 15.6.)
+        int best = plan->staged_rows > 32 ? fastest() : widest(f32 && plan->staged_rows >= 16 ? 4 : 8);
+        if (plan->staged_rows <= 32 && blocks * best < kDirectMinWorkgroups) best = std::max(best, widest(4));
         if (!best) {
-            best = largest_divisor_split(G, plan->row_blocks, kDirectTargetWorkgroups);
+            best = largest_divisor_split(G, blocks, kDirectTargetWorkgroups);
             if (best * split_bytes > most_bytes || plan->row_blocks > kUsableCounters) best = 1;
         }
         k_split = best;
@@ -3538,7 +3575,12 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
                     static_cast<long long>(plan->row_blocks), kUsableCounters);
     plan->k_split = k_split;
     plan->chunk_groups = static_cast<int>(G / k_split);
-    plan->partial_bytes = k_split > 1 ? static_cast<size_t>(k_split) * split_bytes : 0;
+    // Tiles per launch: what the counters, the partials and the grid hold.
+    int64_t fit = 65535;
+    if (k_split > 1) fit = std::min(kUsableCounters / plan->row_blocks, std::max<int64_t>(most_bytes / (k_split * split_bytes), 1));
+    plan->batch_tiles = std::min(tiles, fit);
+    plan->launch_rows = plan->batch_tiles * plan->tile_rows;
+    plan->partial_bytes = k_split > 1 ? static_cast<size_t>(plan->batch_tiles) * k_split * split_bytes : 0;
     return TERNEL_TQ1_OK;
 }
 
@@ -3547,15 +3589,16 @@ size_t trit_workspace_bytes(const TritPlan &plan) { return plan.k_split > 1 ? kP
 template <typename T, int SR>
 void launch_trit_kernel(const uint32_t *packed, const T *x, T *y, int64_t M, int64_t rows, int G, const TritPlan &plan,
                         float *partial, unsigned *counters, int flags, hipStream_t stream) {
-    const dim3 grid(static_cast<unsigned>(plan.row_blocks), static_cast<unsigned>(plan.k_split));
+    const dim3 grid(static_cast<unsigned>(plan.row_blocks), static_cast<unsigned>(plan.k_split),
+                    static_cast<unsigned>(ceil_div(M, plan.tile_rows)));
     if (plan.chunk_groups > trit_window(sizeof(T), SR))
         hipLaunchKernelGGL((trit_gemm_kernel<T, SR, true>), grid, dim3(kDirectThreads), 0, stream, packed, x, y, partial,
                            counters, static_cast<int>(M), static_cast<int>(rows), G, plan.chunk_groups, plan.k_split,
-                           flags);
+                           static_cast<int>(plan.tile_rows), flags);
     else
         hipLaunchKernelGGL((trit_gemm_kernel<T, SR, false>), grid, dim3(kDirectThreads), 0, stream, packed, x, y, partial,
                            counters, static_cast<int>(M), static_cast<int>(rows), G, plan.chunk_groups, plan.k_split,
-                           flags);
+                           static_cast<int>(plan.tile_rows), flags);
 }
 
 template <typename T>
@@ -3790,14 +3833,38 @@ int linear_gemm_form(int64_t M, int64_t rows, int64_t columns, int dtype) {
     return dtype == TERNEL_TQ1_BF16 ? TERNEL_TQ1_GEMM_WIDE : TERNEL_TQ1_GEMM_AUTO;
 }
 
-// The trit kernel runs the direct form (fp16), and in the wide form's place the
-// bf16 batches it is faster for.
-bool gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int form) {
-    if (form == TERNEL_TQ1_GEMM_DIRECT) return true;
-    if (dtype != TERNEL_TQ1_BF16 || form != TERNEL_TQ1_GEMM_WIDE) return false;
+// The trit kernel runs the direct form (fp16), and batches of the automatic
+// forms that it is faster for: bf16 (asked for as WIDE) up to 32 rows, and
+// tiles of up to 64 rows above that (fp16 where the direct form ends). Small
+// matrices give the wide form's 256-row tiles too few CUs or too long a
+// reduction, and the tile form waits for each group's loads. Measured on MI355X
+// (us, trit / best other fp16 form; the bf16 wide form is 2-8 us slower than
+// the fp16 one for its scaling pass):
+//   under 4 MB: 4096 square M=128 17 / 26, M=768 44 / 47; k_proj M=128 16 / 27,
+//   M=768 26 / 30, M=1024 34 / 33; 3000 x 3072 M=768 35 / 35;
+//   under 12 MB: out_proj M=128 22 / 29, M=384 39 / 44, M=512 58 / 54; QKV M=203
+//   34 / 41, M=384 52 / 52; 12288 x 2048 M=128 17 / 29, M=384 37 / 37, bf16 M=512
+//   40 / 42; but on long rows 1500 x 17408 M=128 30 / 29, M=203 42 / 34, where
+//   bf16 (which the tile form does not take) runs M=128 31 / 98, M=512 68 / 78;
+//   larger: bf16 M=64 gate/up 31 / 35, M=100 47 / 45; down M=100 49 / 58, M=203
+//   86 / 77.
+bool trit_beats_wide(int64_t M, int64_t rows, int64_t columns, int dtype) {
+    const int64_t G = columns / kBlockWeights, bytes = rows * G * kBlockBytes;
+    const bool bf16 = dtype == TERNEL_TQ1_BF16;
+    if (bytes < 4 << 20) return M <= 768;
+    if (bytes < 12 << 20) return bf16 ? M <= 512 : (G <= 64 && M <= 384);
+    return bf16 && bytes < kTritBf16MatrixBytes && M <= (G > 64 ? 128 : 64);
+}
+
+// `form` as asked for, `resolved` by resolve_gemm_form.
+bool gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int form, int resolved, int k_split) {
+    if (resolved == TERNEL_TQ1_GEMM_DIRECT) return true;
+    if (dtype == TERNEL_TQ1_F16)
+        return form == TERNEL_TQ1_GEMM_AUTO && k_split == 0 && columns <= kWideMaxColumns &&
+               trit_beats_wide(M, rows, columns, dtype);
+    if (dtype != TERNEL_TQ1_BF16 || resolved != TERNEL_TQ1_GEMM_WIDE) return false;
     WidePlan wide;  // what the wide form refuses is left for it to refuse
-    return (M <= kAutoDirectMaxBatch ||
-            (M <= kDirectMaxBatch && rows * (columns / kBlockWeights) * kBlockBytes < kTritBf16MatrixBytes)) &&
+    return (M <= kAutoDirectMaxBatch || trit_beats_wide(M, rows, columns, dtype)) &&
            plan_wide(M, rows, columns, 0, &wide) == TERNEL_TQ1_OK;
 }
 
@@ -4126,10 +4193,10 @@ size_t ternel_tq1_matmul_workspace_bytes(int64_t M, int64_t rows, int64_t column
     size_t need = plan.counter_bytes + plan.partial_bytes;
     TritPlan trit;  // the workspace of whichever kernel runs (unaligned activations take the LUT23 kernel)
     if (matmul_uses_trit(M, rows, columns, TERNEL_TQ1_F32, batch_tile, k_split) &&
-        plan_trit(M, rows, columns, TERNEL_TQ1_F32, 0, &trit, true) == TERNEL_TQ1_OK)
+        plan_trit(M, rows, columns, TERNEL_TQ1_F32, 0, &trit, true, kTritMatmulPartialBytes) == TERNEL_TQ1_OK)
         need = std::max(need, trit_workspace_bytes(trit));
     if (matmul_uses_trit(M, rows, columns, TERNEL_TQ1_F16, batch_tile, k_split) &&
-        plan_trit(M, rows, columns, TERNEL_TQ1_F16, 0, &trit, true) == TERNEL_TQ1_OK)
+        plan_trit(M, rows, columns, TERNEL_TQ1_F16, 0, &trit, true, kTritMatmulPartialBytes) == TERNEL_TQ1_OK)
         need = std::max(need, trit_workspace_bytes(trit));
     return need;
 }
@@ -4161,7 +4228,7 @@ int ternel_tq1_matmul(const uint32_t *packed, const void *x, void *y, int64_t M,
     }
     if (matmul_uses_trit(M, rows, columns, dtype, batch_tile, k_split) && !(reinterpret_cast<uintptr_t>(x) & 15u)) {
         TritPlan trit;
-        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true)) != TERNEL_TQ1_OK) return rc;
+        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true, kTritMatmulPartialBytes)) != TERNEL_TQ1_OK) return rc;
         if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
         if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
         const size_t need = trit_workspace_bytes(trit);
@@ -4216,7 +4283,7 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
     }
     if (matmul_uses_trit(M, rows, columns, dtype, batch_tile, k_split) && !(reinterpret_cast<uintptr_t>(x) & 15u)) {
         TritPlan trit;  // its partials fit the scratch
-        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true)) != TERNEL_TQ1_OK) return rc;
+        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true, kTritMatmulPartialBytes)) != TERNEL_TQ1_OK) return rc;
         if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
         if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
         hipStream_t s = static_cast<hipStream_t>(stream);
@@ -4251,7 +4318,12 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
 
 size_t ternel_tq1_gemm_workspace_bytes(int64_t M, int64_t rows, int64_t columns, int form, int k_split) {
     if (check_geometry(M, rows, columns) != TERNEL_TQ1_OK) return 0;
+    const int asked = form;
     form = resolve_gemm_form(M, rows, columns, form, k_split);
+    if (form != TERNEL_TQ1_GEMM_DIRECT && gemm_uses_trit(M, rows, columns, TERNEL_TQ1_F16, asked, form, k_split)) {
+        TritPlan trit;
+        return plan_trit(M, rows, columns, TERNEL_TQ1_F16, 0, &trit, true) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
+    }
     if (form == TERNEL_TQ1_GEMM_DIRECT) {
         TritPlan trit;
         return plan_trit(M, rows, columns, TERNEL_TQ1_F16, k_split, &trit) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
@@ -4261,8 +4333,8 @@ size_t ternel_tq1_gemm_workspace_bytes(int64_t M, int64_t rows, int64_t columns,
         if (plan_wide(M, rows, columns, k_split, &wide) != TERNEL_TQ1_OK) return 0;
         TritPlan trit;
         size_t small = 0;  // what a bf16 batch of this size uses
-        if (gemm_uses_trit(M, rows, columns, TERNEL_TQ1_BF16, form) &&
-            plan_trit(M, rows, columns, TERNEL_TQ1_BF16, 0, &trit) == TERNEL_TQ1_OK)
+        if (gemm_uses_trit(M, rows, columns, TERNEL_TQ1_BF16, form, form, 0) &&
+            plan_trit(M, rows, columns, TERNEL_TQ1_BF16, 0, &trit, true) == TERNEL_TQ1_OK)
             small = trit_workspace_bytes(trit);
         return std::max(kPartialOffset + wide.partial_bytes + wide.xp_bytes, small);
     }
@@ -4290,11 +4362,12 @@ int ternel_tq1_gemm(const uint32_t *packed, const void *x, void *y, int64_t M, i
         if (k_split > 1) return fail(TERNEL_TQ1_EINVAL, "the wide form takes no fixed K split, got %d", k_split);
         form = TERNEL_TQ1_GEMM_WIDE;
     }
+    const int asked = form;
     form = resolve_gemm_form(M, rows, columns, form, k_split);
-    if (gemm_uses_trit(M, rows, columns, dtype, form)) {
+    if (gemm_uses_trit(M, rows, columns, dtype, asked, form, k_split)) {
         TritPlan trit;
-        if ((rc = plan_trit(M, rows, columns, dtype, form == TERNEL_TQ1_GEMM_WIDE ? 0 : k_split, &trit)) != TERNEL_TQ1_OK)
-            return rc;
+        const bool direct = form == TERNEL_TQ1_GEMM_DIRECT;
+        if ((rc = plan_trit(M, rows, columns, dtype, direct ? k_split : 0, &trit, !direct)) != TERNEL_TQ1_OK) return rc;
         if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
         if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
         if (reinterpret_cast<uintptr_t>(x) & 15u) return fail(TERNEL_TQ1_EINVAL, "activations must be 16-byte aligned");
@@ -4380,8 +4453,8 @@ int ternel_tq1_linear_kernel(int64_t M, int64_t rows, int64_t columns, int dtype
 
 // Whether the fused SwiGLU's GEMM is the trit kernel.
 static bool swiglu_gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype) {
-    return gemm_uses_trit(M, rows, columns, dtype,
-                          resolve_gemm_form(M, rows, columns, linear_gemm_form(M, rows, columns, dtype), 0));
+    const int form = linear_gemm_form(M, rows, columns, dtype);
+    return gemm_uses_trit(M, rows, columns, dtype, form, resolve_gemm_form(M, rows, columns, form, 0), 0);
 }
 
 size_t ternel_tq1_swiglu_workspace_bytes(int64_t M, int64_t rows, int64_t columns, int dtype) {
@@ -4391,12 +4464,12 @@ size_t ternel_tq1_swiglu_workspace_bytes(int64_t M, int64_t rows, int64_t column
         const size_t lut = ternel_tq1_matmul_workspace_bytes(
             M, rows, columns, uses_strip_gemv(M, 0, 0, rows, columns, false) ? 0 : 1, 0);
         return matmul_uses_trit(M, rows, columns, dtype, 0, 0) &&
-                       plan_trit(M, rows, columns, dtype, 0, &trit, true) == TERNEL_TQ1_OK
+                       plan_trit(M, rows, columns, dtype, 0, &trit, true, kTritMatmulPartialBytes) == TERNEL_TQ1_OK
                    ? std::max(lut, trit_workspace_bytes(trit))
                    : lut;
     }
     if (swiglu_gemm_uses_trit(M, rows, columns, dtype))
-        return plan_trit(M, rows, columns, dtype, 0, &trit) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
+        return plan_trit(M, rows, columns, dtype, 0, &trit, true) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
     if (resolve_gemm_form(M, rows, columns, linear_gemm_form(M, rows, columns, dtype), 0) == TERNEL_TQ1_GEMM_WIDE)
         return ternel_tq1_gemm_workspace_bytes(M, rows, columns, TERNEL_TQ1_GEMM_WIDE, 0);
     return swiglu_pairs_offset(M, rows, columns, dtype) + static_cast<size_t>(M) * rows * sizeof(_Float16);
@@ -4432,7 +4505,9 @@ int ternel_tq1_swiglu(const uint32_t *packed, const void *x, void *z, int64_t M,
         lut && matmul_uses_trit(M, rows, columns, dtype, 0, 0) && !(reinterpret_cast<uintptr_t>(x) & 15u);
     if (matmul_trit || (!lut && swiglu_gemm_uses_trit(M, rows, columns, dtype))) {
         TritPlan trit;
-        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, matmul_trit)) != TERNEL_TQ1_OK) return rc;
+        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true,
+                            matmul_trit ? kTritMatmulPartialBytes : kTritPartialBytes)) != TERNEL_TQ1_OK)
+            return rc;
         if (reinterpret_cast<uintptr_t>(x) & 15u) return fail(TERNEL_TQ1_EINVAL, "activations must be 16-byte aligned");
         const size_t need = trit_workspace_bytes(trit);
         if (need && (!ws || ws_bytes < need))

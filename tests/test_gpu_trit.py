@@ -45,6 +45,9 @@ def bound(x: np.ndarray, blocks: np.ndarray, want: np.ndarray, dtype: torch.dtyp
 SHAPES = ((130, 128), (300, 640), (257, 1152), (96, 2176), (1024, 5120))
 CASES = [(dtype, rows, columns, batch) for dtype in (torch.float16, torch.bfloat16)
          for rows, columns in SHAPES for batch in (5, 8, 9, 17, 32, 33, 64)]
+# tiles of 64 rows and the remainder of a batch past them, split and unsplit
+CASES += [(dtype, rows, columns, batch) for dtype in (torch.float16, torch.bfloat16)
+          for rows, columns, batch in ((257, 1152, 65), (1024, 5120, 130), (300, 640, 203), (4100, 1024, 193))]
 # fp32: matrices large enough for the trit kernel at each tile width, and batches of several launches
 CASES += [(torch.float32, 5121, 4608, 8), (torch.float32, 2562, 4608, 15), (torch.float32, 300, 640, 77),
           (torch.float32, 257, 1152, 130), (torch.float32, 130, 128, 65)]
@@ -66,8 +69,8 @@ def test_small_batches_match_the_oracle(dtype, rows, columns, batch) -> None:
 # the trit kernel's tiles, then the wide form's (fp16 takes it from 64 tiles of
 # 256 rows on); an output width that no 16-byte store divides, and one it does
 SWIGLU = [(dtype, 1030, 1152, batch) for dtype in (torch.float16, torch.bfloat16) for batch in (2, 7, 30, 64)]
-SWIGLU += [(torch.bfloat16, 1030, 1152, 70), (torch.bfloat16, 1030, 1152, 300), (torch.bfloat16, 1024, 1152, 300),
-           (torch.float16, 16390, 256, 70), (torch.float16, 16400, 256, 300)]
+SWIGLU += [(torch.bfloat16, 1030, 1152, 70), (torch.bfloat16, 1030, 1152, 800), (torch.bfloat16, 1024, 1152, 800),
+           (torch.bfloat16, 60006, 1024, 70), (torch.float16, 60000, 1024, 70), (torch.float16, 16390, 256, 800)]
 
 
 @pytest.mark.parametrize(("dtype", "rows", "columns", "batch"), SWIGLU)
@@ -108,7 +111,7 @@ def test_non_finite_values_follow_the_entry_point(dtype) -> None:
 def test_a_swiglu_reduction_that_gives_up_writes_nan() -> None:
     """The wide form's bounded wait driven to give up from the host: every
     output is the fused value or NaN, some are NaN, and the error word is set."""
-    rows, columns, batch = 1030, 5120, 300
+    rows, columns, batch = 1030, 5120, 800
     packed, lay = pack(random_blocks(rows, columns, seed=5)), layout(rows, columns)
     x = to_dev(np.random.default_rng(5).normal(0.0, 0.3, size=(batch, columns)).astype(np.float32)).to(torch.bfloat16)
     want = tq1_swiglu_words(packed, x, layout=lay)
