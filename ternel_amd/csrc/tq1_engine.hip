@@ -3556,9 +3556,12 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
             }
             return best;
         };
-        // (fp32 past 8 rows stages 4 or 2 groups at a time: QKV M=24 in chunks of
-        // 8 21.7 us, of 4 19.5; M=16 17.8 / 15.6.)
+        // At 17-32 rows, whose window is 4 groups, chunks of 4 where they reach
+        // the target (QKV M=32, 640 workgroups against 320 of 8: 12.8 / 12.9).
+        // fp32 past 8 rows stages 4 or 2 groups at a time: chunks of 4 (QKV
+        // M=24 19.5 us against 21.7 in chunks of 8, M=16 15.6 / 17.8).
         int best = plan->staged_rows > 32 ? fastest() : widest(f32 && plan->staged_rows >= 16 ? 4 : 8);
+        if (plan->staged_rows == 32 && blocks * widest(4) >= kDirectTargetWorkgroups) best = widest(4);
         if (plan->staged_rows <= 32 && blocks * best < kDirectMinWorkgroups) best = std::max(best, widest(4));
         if (!best) {
             best = largest_divisor_split(G, blocks, kDirectTargetWorkgroups);
