@@ -1702,7 +1702,7 @@ __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (
 // (t - 1) * scale weights together and took only fp16 (bf16 ran the wide form
 // after a scaling pass, fp32 the LUT23 kernel): fp16 M=8 17.9 / 20.3 / 12.8 ->
 // 14.1 / 14.3 / 9.9, M=32 20.6 / 23.6 / 15.5 -> 18.1 / 21.3 / 13.3; bf16 M=8
-// 27.2 / 34.8 / 24.6 -> 14.1 / 14.3 / 9.9; fp32 QKV M=24 41.9 -> 19.9.
+// 27.2 / 34.8 / 24.6 -> 14.1 / 14.3 / 9.9; fp32 QKV M=24 41.7 -> 20.7.
 //
 // Weights never touch LDS: lane l of a wave decodes half l / 32 of the block
 // of weight row l % 32 straight into an operand of v_mfma_f32_32x32x16, in the
@@ -1995,11 +1995,17 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
     auto group = [&](int slot, const uint32_t (&w)[5], auto with_decode) __attribute__((always_inline)) {
         constexpr bool kDecode = decltype(with_decode)::value;
         const uint32_t u[4] = {w[0], w[1], w[2], w[3]};
-        float16v sum[NB];
+        // fp32's lower terms are summed by themselves: beside the upper ones
+        // each of their additions would round at the sum's full magnitude.
+        // Errors against fp64, one sum / two (the LUT23 kernel's): 5839 x 15872,
+        // M=11 1.57e-7 / 1.14e-7 (1.52e-7), QKV M=24 1.23e-7 / 0.78e-7
+        // (1.26e-7); the registers cost QKV M=24 18.7 -> 20.7 us (41.7), M=14 of
+        // 20799 x 2176 21.0 -> 21.4 (44.3).
+        float16v sum[NB], low[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sum[nb][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) sum[nb][r] = low[nb][r] = 0.0f;
         WindowSplits s;
 #pragma unroll
         for (int st = 0; st < 8; ++st) {
@@ -2012,7 +2018,10 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
 #pragma unroll
             for (int p = P - 1; p >= 0; --p)
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) sum[nb] = Op::mfma(b[p][nb], wt, sum[nb]);
+                for (int nb = 0; nb < NB; ++nb) {
+                    float16v &into = p == 0 ? sum[nb] : low[nb];
+                    into = Op::mfma(b[p][nb], wt, into);
+                }
             if constexpr (kDecode) {
                 // window w's dwords end at 5w + 4: after the stage that reads it
                 if (st == 0) s = window_splits(u, 0);
@@ -2036,13 +2045,17 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int r = 0; r < RQ * 4; ++r) acc[nb][r] = fmaf(scale, sum[nb][r], acc[nb][r]);
+            for (int r = 0; r < RQ * 4; ++r)
+                acc[nb][r] = fmaf(scale, P == 1 ? sum[nb][r] : sum[nb][r] + low[nb][r], acc[nb][r]);
         // All 16 sums stay live until the fmas above have waited for the last
         // MFMA: the compiler would reuse the registers of the unused ones at
         // once, and its hazard checks do not see the decode's inline asm
         // write them while the MFMA still does.
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) keep_live(acc[nb][0], sum[nb]);
+        for (int nb = 0; nb < NB; ++nb) {
+            keep_live(acc[nb][0], sum[nb]);
+            if constexpr (P > 1) keep_live(acc[nb][0], low[nb]);
+        }
         if constexpr (kDecode) finish_decode(w);
     };
 
