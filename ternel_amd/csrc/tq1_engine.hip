@@ -1908,7 +1908,8 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
     const uint32_t wother = wrow + (upper ? 0 : 6) * kTileRows * 4;
     uint32_t ring[4][5];  // words of group v in ring[v % 4]: 3h .. 3h + 3 and the other end word
     auto load_words = [&](uint32_t (&w)[5], int v) __attribute__((always_inline)) {
-        const char *const p = reinterpret_cast<const char *>(tile_words) + min(v, cg - 1) * (kTileGroupWords * 4);
+        const char *const p = reinterpret_cast<const char *>(tile_words) +
+                              static_cast<int64_t>(min(v, cg - 1)) * (kTileGroupWords * 4);  // past 2 GiB on long rows
 #pragma unroll
         for (int j = 0; j < 4; ++j) w[j] = *reinterpret_cast<const uint32_t *>(p + wfirst + j * (kTileRows * 4));
         w[4] = *reinterpret_cast<const uint32_t *>(p + wother);

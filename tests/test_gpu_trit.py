@@ -20,7 +20,7 @@ import torch
 from oracle import tq1_oracle as O
 from tests.gpu_util import layout, pack, random_blocks, to_dev
 from ternel_amd import _lib
-from ternel_amd.kernels import tq1_linear_words, tq1_matmul_words, tq1_swiglu_words
+from ternel_amd.kernels import GemmConfig, tq1_gemm_words, tq1_linear_words, tq1_matmul_words, tq1_swiglu_words
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +131,20 @@ def test_a_swiglu_reduction_that_gives_up_writes_nan() -> None:
     nan = torch.isnan(out)
     assert word.value == 2 and bool(nan.any())
     assert torch.equal(out[~nan], want[~nan])
+
+
+def test_a_row_of_more_than_2_gib_of_packed_words() -> None:
+    """One K chunk whose last groups lie past 2^31 bytes of the tile's words:
+    blocks of scale 0 but for two at the far end, trits all -1, so an output is
+    minus those groups' activations, times their scales, exactly."""
+    rows, groups = 64, 2 ** 31 // 1792 + 11
+    columns = groups * 128
+    packed = torch.zeros((1, groups, 7, 64), dtype=torch.int32, device="cuda")
+    packed[0, groups - 1, 0, :] = 0x3C00  # word 0: the scale (1.0) and code bytes 0 and 1
+    packed[0, groups - 9, 0, :] = 0x4000  # 2.0
+    x = torch.zeros((2, columns), dtype=torch.float16, device="cuda")
+    x[0, (groups - 1) * 128:] = 1.0
+    x[1, (groups - 9) * 128:(groups - 8) * 128] = 0.5
+    got = tq1_gemm_words(packed, x, layout=layout(rows, columns), config=GemmConfig(form="direct", k_split=1))
+    want = torch.tensor([[-128.0], [-128.0]], dtype=torch.float16, device="cuda").expand(2, rows)
+    assert torch.equal(got, want)
