@@ -262,8 +262,9 @@ def check_activations(x: torch.Tensor, *, layout: PackedTensorLayout) -> int:
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 # Workspaces that a graph may still address: replaced by a larger one after
 # their stream was captured, so never freed (a replay would otherwise write
-# counters and partials into memory the caching allocator has reused).
-_RETIRED: list[torch.Tensor] = []
+# counters and partials into memory the caching allocator has reused). Each
+# carries the host word of its (device, stream), as its successor does.
+_RETIRED: list[tuple[tuple[int, int], torch.Tensor]] = []
 _CAPTURED: set[tuple[int, int]] = set()
 
 
@@ -304,14 +305,16 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
         key = max(sized, key=lambda k: _WORKSPACES[k].numel())
         buf = _WORKSPACES[key]
     if buf is None or buf.numel() < nbytes:
-        new = torch.empty(max(nbytes, 1 << 22), dtype=torch.uint8, device=torch.device("cuda", index))
+        new = _new_buffer(index, max(nbytes, 1 << 22))
         if key not in _FLAGS:
             _FLAGS[key] = _HostWord()
             _FLAG_WORDS = tuple((k[0], f.word) for k, f in _FLAGS.items())
-        _reset(new, key)
+        # The host word stays as it is: a give-up on the old buffer that no call
+        # has raised yet is raised by the next one.
+        _clear(new, key)
         torch.cuda.synchronize(index)
         if buf is not None and key in _CAPTURED:
-            _RETIRED.append(buf)
+            _RETIRED.append((key, buf))
         _WORKSPACES[key] = buf = new
     if capturing:
         _CAPTURED.add(key)
@@ -323,7 +326,10 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
 # word whose address the workspace carries, so the next call on the device
 # notices by reading host memory. (An event per launch and a 4-byte copy on a
 # side stream at the next call, which this replaces, cost 30 us of host time a
-# call.) Graph replays report here too.
+# call.) Graph replays report here too, also on workspaces that have been
+# replaced since their capture: a report clears every buffer of its stream, so
+# that no replay is left on one whose error word is set (such a launch writes
+# NaN without a report of its own).
 class _HostWord:
     def __init__(self) -> None:
         self.tensor = torch.zeros(1, dtype=torch.int32, pin_memory=True)
@@ -335,12 +341,33 @@ _FLAG_WORDS: tuple[tuple[int, ctypes.c_int], ...] = ()  # (device, host word) of
 _HOST_WORD_OFFSET = 64 * 1024 - 16  # in the counter region, before the error word
 
 
-def _reset(buf: torch.Tensor, key: tuple[int, int]) -> None:
+def _new_buffer(index: int, nbytes: int) -> torch.Tensor:
+    return torch.empty(nbytes, dtype=torch.uint8, device=torch.device("cuda", index))
+
+
+def _clear(buf: torch.Tensor, key: tuple[int, int]) -> None:
     """A workspace as it is handed out: zero but for its host word's address."""
-    flag = _FLAGS[key]
     buf.zero_()
-    buf[_HOST_WORD_OFFSET:_HOST_WORD_OFFSET + 8].view(torch.int64).fill_(flag.tensor.data_ptr())
-    flag.word.value = 0
+    buf[_HOST_WORD_OFFSET:_HOST_WORD_OFFSET + 8].view(torch.int64).fill_(_FLAGS[key].tensor.data_ptr())
+
+
+def _buffers() -> list[tuple[tuple[int, int], torch.Tensor]]:
+    """Every workspace a launch or a replay may use, with its (device, stream)."""
+    return [*_WORKSPACES.items(), *_RETIRED]
+
+
+def _reset(keys) -> None:
+    """Clears every buffer of these (device, stream) pairs, once all work on
+    their devices is done, and then their host words."""
+    for index in {key[0] for key in keys}:
+        torch.cuda.synchronize(index)
+    for key, buf in _buffers():
+        if key in keys:
+            _clear(buf, key)
+    for key in keys:
+        _FLAGS[key].word.value = 0
+    for index in {key[0] for key in keys}:
+        torch.cuda.synchronize(index)
 
 
 def _surface(index: int) -> None:
@@ -355,25 +382,24 @@ def _surface(index: int) -> None:
         return
     torch.cuda.synchronize(index)  # the launch that reported may still be running
     failed = {k: f.word.value for k, f in list(_FLAGS.items()) if k[0] == index and f.word.value}
-    for key in failed:
-        _reset(_WORKSPACES[key], key)
-    torch.cuda.synchronize(index)
+    _reset(failed)
     raise _lib.NativeError(f"a kernel's bounded wait for a published partial gave up: {failed}; "
                            "its tiles were written as NaN and the workspace has been zeroed")
 
 
 def workspace_errors() -> dict[tuple[int, int], int]:
-    """The error word of every workspace (synchronises each one's stream): a
-    nonzero word names the kernels whose bounded wait for another workgroup's
-    partial gave up (2 = the wide GEMM's stream-K reduction; the LUT23 and
-    direct-form fix-ups never wait)."""
+    """The error word of every (device, stream), over its workspace and those a
+    graph may still replay on (synchronises each one's stream): a nonzero word
+    names the kernels whose bounded wait for another workgroup's partial gave
+    up (2 = the wide GEMM's stream-K reduction; the LUT23 and direct-form
+    fix-ups never wait)."""
     handle = _lib.lib()
     words = {}
-    for (index, stream), buf in _WORKSPACES.items():
+    for (index, stream), buf in _buffers():
         word = ctypes.c_int(0)
         with torch.cuda.device(index):
             _lib.check(handle.ternel_tq1_workspace_error(buf.data_ptr(), buf.numel(), ctypes.byref(word), stream))
-        words[(index, stream)] = word.value
+        words[(index, stream)] = words.get((index, stream), 0) | word.value
     return words
 
 
@@ -382,10 +408,8 @@ def check_workspaces() -> None:
     workspace is zeroed again first (its counters may be left set), so the
     next call starts clean."""
     failed = {key: word for key, word in workspace_errors().items() if word}
-    for key in failed:
-        _reset(_WORKSPACES[key], key)
     if failed:
-        torch.cuda.synchronize()
+        _reset(failed)
         raise _lib.NativeError(f"a kernel's bounded wait for a published partial gave up: {failed}")
 
 

@@ -200,3 +200,48 @@ def test_workspace_error_entry_refuses_a_workspace_without_an_error_word() -> No
     word = ctypes.c_int(0)
     buf = torch.zeros(1024, dtype=torch.uint8, device=dev())
     assert handle.ternel_tq1_workspace_error(buf.data_ptr(), 1024, ctypes.byref(word), None) == _lib.TERNEL_TQ1_EINVAL
+
+
+def test_replays_on_a_replaced_workspace_report_and_recover(monkeypatch) -> None:
+    """Two graphs captured on one workspace, one with a limit that makes every
+    bounded wait give up, then the workspace replaced by a larger one: each
+    replay that gives up is raised by the next call, which clears the replaced
+    workspace too, so the other graph's replays are exact."""
+    from ternel_amd import kernels
+
+    for name, value in (("_WORKSPACES", {}), ("_RETIRED", []), ("_CAPTURED", set()), ("_FLAGS", {}),
+                        ("_FLAG_WORDS", ())):
+        monkeypatch.setattr(kernels, name, value)
+    packed, xt, lay, config, want = _wide_case()
+    handle = _lib.lib()
+    graphs, outs = [], []
+    for limit in (-1, None):
+        graph = torch.cuda.CUDAGraph()
+        old = handle.ternel_tq1_set_spin_limit(limit) if limit is not None else None
+        try:
+            with torch.cuda.graph(graph):
+                out = tq1_gemm_words(packed, xt, layout=lay, config=config)
+        finally:
+            if old is not None:
+                handle.ternel_tq1_set_spin_limit(old)
+        graphs.append(graph)
+        outs.append(out)
+    tq1_gemm_words(packed, xt.repeat(4, 1), layout=lay, config=config)  # a larger workspace
+    assert len(kernels._RETIRED) == 1
+    for _ in range(3):
+        graphs[0].replay()
+        torch.cuda.synchronize()
+        _nan_tiles_and_exact_elsewhere(outs[0].cpu(), want)
+        assert any(w & 2 for w in workspace_errors().values())
+        with pytest.raises(_lib.NativeError, match="bounded wait"):
+            tq1_gemm_words(packed, xt, layout=lay, config=config)
+        assert not any(workspace_errors().values())
+        outs[1].zero_()
+        graphs[1].replay()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[1].cpu(), want)
+        assert torch.equal(tq1_gemm_words(packed, xt, layout=lay, config=config).cpu(), want)
+    graphs[0].replay()
+    with pytest.raises(_lib.NativeError, match="bounded wait"):
+        check_workspaces()
+    assert not any(workspace_errors().values())
