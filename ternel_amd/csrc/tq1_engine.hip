@@ -23,6 +23,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <math.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -1843,6 +1844,7 @@ struct TritHalf {
     }
 };
 
+constexpr int kTritReduceBatch = 17;  // K chunks the reduction loads at once, at most
 constexpr int kTritGlu = 1;         // write SiLU(row 2r) * (row 2r + 1)
 constexpr int kTritIeeeScales = 2;  // zero trits of a non-finite scale are NaN
 
@@ -1891,7 +1893,7 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
     const bool upper = lane >= 32;
     const int row0 = blockIdx.x * kDirectRows + wave * 32;
     const int g_begin = blockIdx.y * chunk_groups;
-    const int cg = chunk_groups;
+    const int cg = min(chunk_groups, G - g_begin);  // the last chunk may be shorter
     const int64_t K = static_cast<int64_t>(G) * kBlockWeights;
     const int direct_wave_id =
         ((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * kDirectWaves + wave;
@@ -2180,7 +2182,7 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
         else if (k_split <= 10)
             reduce(std::integral_constant<int, 10>{});
         else
-            reduce(std::integral_constant<int, 17>{});
+            reduce(std::integral_constant<int, kTritReduceBatch>{});
         if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         TQ1_PHASE(direct_wave_id, 8);  // fix-up sums done
     }
@@ -3491,7 +3493,7 @@ int direct_staged_rows(int64_t M) { return M <= 8 ? 8 : (M <= 16 ? 16 : (M <= 32
 struct TritPlan {
     int staged_rows;
     int k_split;
-    int chunk_groups;
+    int chunk_groups;  // of every chunk but the last, which may be shorter
     int64_t row_blocks;
     int64_t tile_rows;    // activation rows per batch tile
     int64_t batch_tiles;  // in one launch
@@ -3504,6 +3506,11 @@ struct TritPlan {
 // workspace-free twin.
 constexpr int64_t kTritPartialBytes = int64_t{64} << 20;
 constexpr int64_t kTritMatmulPartialBytes = int64_t{16} << 20;
+
+// Equal K chunks up to this many times the workgroups that chunks of any size
+// would need; unequal ones below this share of their estimated time.
+constexpr int64_t kTritEqualSplitSlack = 3;
+constexpr double kTritUnequalGain = 0.85;
 
 // batches: a batch past one tile runs as tiles of nearly equal size, in as
 // many launches as the counters and the partials' limit need; otherwise it is
@@ -3533,18 +3540,31 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
         // 1500 x 17408, 204, M=8 10.4 / 12.2), chunks of 4 where they do not
         // (4096 square M=8, 128: 7.9 / 7.2; k_proj, 40: 7.2 / 6.3; 2 groups:
         // 8.5, 8.0).
-        auto usable = [&](int64_t k, int64_t granule) {
-            return G % k == 0 && (G / k) % granule == 0 &&
-                   (k == 1 || (k * split_bytes <= most_bytes && plan->row_blocks <= kUsableCounters));
+        //
+        // Equal chunks where the group count has a split that fits; otherwise
+        // the last chunk is shorter. A prime count has only splits of one and
+        // of all, four times a prime only chunks of 4 (which may not fit the
+        // partials' limit). us, equal chunks alone / now: 4096 x 8576 fp32 M=9
+        // 71.7 / 14.0, 1024 x 8576 fp16 M=2 30.4 / 7.4, 4096 x 16768 bf16 M=32
+        // 80.9 / 17.5, 16749 x 9728 (76 groups) fp32 M=10 83.5 / 43.6.
+        auto chunk_of = [&](int64_t k, int64_t granule, bool equal) -> int64_t {  // groups; 0: no such split
+            if (k > 1 && (k * split_bytes > most_bytes || plan->row_blocks > kUsableCounters)) return 0;
+            if (equal) return G % k == 0 && (G / k) % granule == 0 ? G / k : 0;
+            const int64_t chunk = ceil_div(ceil_div(G, k), granule) * granule;
+            return ceil_div(G, chunk) == k ? chunk : 0;
         };
-        auto widest = [&](int64_t granule) {
+        auto search = [&](int64_t granule, bool equal) {
             int best = 0;
             for (int64_t k = 1; k <= G; ++k) {
-                if (!usable(k, granule)) continue;
+                if (!chunk_of(k, granule, equal)) continue;
                 best = static_cast<int>(k);
                 if (blocks * k >= kDirectTargetWorkgroups) break;
             }
             return best;
+        };
+        auto widest = [&](int64_t granule) {
+            const int equal = search(granule, true), any = search(granule, false);
+            return equal >= any && equal <= kTritEqualSplitSlack * any ? equal : any;
         };
         // 33-64 rows a tile: two workgroups per CU, whose loop the LDS bounds,
         // so a second workgroup on a CU adds its groups' time and a third
@@ -3557,15 +3577,19 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
             const int64_t cus = device_cu_count();
             int best = 0;
             double least = 0;
-            for (int64_t k = 1; k <= G; ++k) {
-                if (!usable(k, 4)) continue;
-                const int64_t n = blocks * k, per_cu = ceil_div(n, cus), rounds = ceil_div(n, 2 * cus);
-                const double us = (k > 1 ? 8.0 : 5.0) +
-                                  static_cast<double>(G / k) * (per_cu == 1 ? 0.82 : 0.66 * static_cast<double>(per_cu)) +
-                                  (per_cu > 1 ? 1.5 : 0.0) + 8.0 * static_cast<double>(rounds - 1);
-                if (!best || us <= least) {
-                    best = static_cast<int>(k);
-                    least = us;
+            for (const bool equal : {true, false}) {
+                const double most_us = best ? kTritUnequalGain * least : HUGE_VAL;
+                for (int64_t k = 1; k <= G; ++k) {
+                    const int64_t chunk = chunk_of(k, 4, equal);
+                    if (!chunk) continue;
+                    const int64_t n = blocks * k, per_cu = ceil_div(n, cus), rounds = ceil_div(n, 2 * cus);
+                    const double us = (k > 1 ? 8.0 : 5.0) +
+                                      static_cast<double>(chunk) * (per_cu == 1 ? 0.82 : 0.66 * static_cast<double>(per_cu)) +
+                                      (per_cu > 1 ? 1.5 : 0.0) + 8.0 * static_cast<double>(rounds - 1);
+                    if (us < most_us && (!best || us <= least)) {
+                        best = static_cast<int>(k);
+                        least = us;
+                    }
                 }
             }
             return best;
@@ -3576,22 +3600,26 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
         // M=24 19.5 us against 21.7 in chunks of 8, M=16 15.6 / 17.8).
         int best = plan->staged_rows > 32 ? fastest() : widest(f32 && plan->staged_rows >= 16 ? 4 : 8);
         if (plan->staged_rows == 32 && blocks * widest(4) >= kDirectTargetWorkgroups) best = widest(4);
-        if (plan->staged_rows <= 32 && blocks * best < kDirectMinWorkgroups) best = std::max(best, widest(4));
-        if (!best) {
-            best = largest_divisor_split(G, blocks, kDirectTargetWorkgroups);
-            if (best * split_bytes > most_bytes || plan->row_blocks > kUsableCounters) best = 1;
-        }
-        k_split = best;
-    }
-    if (G % k_split)
+        // More chunks of 4 than the reduction loads in one batch pay only where
+        // next to no workgroups are (us, chunks of 4 / 8: 2048 x 10752 M=3 11.0
+        // / 9.5, 768 x 17408 9.4 / 8.9, but 128 x 12800 7.1 / 7.6).
+        if (plan->staged_rows <= 32 && blocks * best < kDirectMinWorkgroups &&
+            (widest(4) <= kTritReduceBatch || blocks <= 4))
+            best = std::max(best, widest(4));
+        k_split = best;  // (a split of one always qualifies)
+        // (the same chunk whichever way `best` was found: equal where it can be)
+        plan->chunk_groups = static_cast<int>(std::min(G, G % best == 0 ? G / best : chunk_of(best, 4, false)));
+    } else if (G % k_split) {
         return fail(TERNEL_TQ1_EINVAL, "k split %d does not divide the tensor's %lld groups per row", k_split,
                     static_cast<long long>(G));
+    } else {
+        plan->chunk_groups = static_cast<int>(G / k_split);
+    }
     if (k_split > 65535) return fail(TERNEL_TQ1_EINVAL, "K too large for one launch");
     if (k_split > 1 && plan->row_blocks > kUsableCounters)
         return fail(TERNEL_TQ1_EINVAL, "%lld row blocks exceed the %d split-K counters",
                     static_cast<long long>(plan->row_blocks), kUsableCounters);
     plan->k_split = k_split;
-    plan->chunk_groups = static_cast<int>(G / k_split);
     // Tiles per launch: what the counters, the partials and the grid hold.
     int64_t fit = 65535;
     if (k_split > 1) fit = std::min(kUsableCounters / plan->row_blocks, std::max<int64_t>(most_bytes / (k_split * split_bytes), 1));

@@ -49,3 +49,31 @@ def test_fp32_activations_take_the_lut_kernel_and_bf16_the_wide_form() -> None:
 def test_the_sweep_covers_every_regime() -> None:
     chosen = {NAMES[_lib.lib().ternel_tq1_linear_kernel(r["M"], r["N"], r["K"], _lib.DTYPE_F16)] for r in SWEEP["rows"]}
     assert chosen == {"lut23", "direct", "wide", "tile"}
+
+
+def direct_split(M: int, rows: int, groups: int) -> int:
+    """K chunks of the direct form, from the partials its workspace holds (a
+    quad of sums per lane of four waves, per 8 activation rows and 128 rows)."""
+    need = _lib.lib().ternel_tq1_gemm_workspace_bytes(M, rows, groups * 128, 2, 0)
+    quads = 8 if M > 32 else -(-M // 8)
+    return max(1, (need - 65536) // (-(-rows // 128) * 4 * quads * 1024)) if need else 1
+
+
+@pytest.mark.parametrize("M", (8, 16, 32, 64))
+@pytest.mark.parametrize("rows", (256, 1024, 4096, 17408))
+def test_every_group_count_splits_over_the_chip(M, rows) -> None:
+    """Prime and almost prime group counts as well: about a workgroup per CU (at
+    64 rows, half of that, where a split would cost more), or chunks of at most
+    12 groups."""
+    blocks = -(-rows // 128)
+    for groups in range(1, 141):
+        k = direct_split(M, rows, groups)
+        assert 1 <= k <= groups
+        assert blocks * k >= (192 if M <= 32 else 128) or -(-groups // k) <= 12, (groups, k)
+
+
+def test_the_27b_widths_split_into_equal_chunks() -> None:
+    for M, rows, groups, k in ((8, 17408, 40, 5), (8, 8192, 40, 5), (8, 5120, 136, 17), (8, 5120, 48, 6),
+                               (8, 34816, 40, 5), (32, 8192, 40, 10), (32, 5120, 48, 6), (8, 1024, 40, 10),
+                               (8, 4096, 32, 8)):
+        assert direct_split(M, rows, groups) == k, (M, rows, groups)

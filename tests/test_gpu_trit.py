@@ -148,3 +148,32 @@ def test_a_row_of_more_than_2_gib_of_packed_words() -> None:
     got = tq1_gemm_words(packed, x, layout=layout(rows, columns), config=GemmConfig(form="direct", k_split=1))
     want = torch.tensor([[-128.0], [-128.0]], dtype=torch.float16, device="cuda").expand(2, rows)
     assert torch.equal(got, want)
+
+
+# group counts that no chunk of 4 or 8 divides: K chunks with a shorter last one, of one group (5,
+# 9, 37, 73), two (74) and three (67), at each tile width, over batch tiles and through the fused SwiGLU
+ODD_GROUPS = [(dtype, rows, groups, batch) for rows, groups in ((1024, 37), (1030, 67), (300, 5), (386, 74))
+              for dtype, batches in ((torch.float16, (2, 3, 8, 16, 32, 64, 130)), (torch.bfloat16, (3, 8, 32, 50)),
+                                     (torch.float32, (40, 70))) for batch in batches]
+ODD_GROUPS += [(torch.float32, 4096, 67, 9), (torch.float32, 4096, 37, 24), (torch.float32, 2560, 73, 16)]
+
+
+@pytest.mark.parametrize(("dtype", "rows", "groups", "batch"), ODD_GROUPS)
+def test_group_counts_without_divisors_match_the_oracle(dtype, rows, groups, batch) -> None:
+    print(f"trit: {dtype} rows={rows} groups={groups} batch={batch}", flush=True)
+    columns = groups * 128
+    blocks = random_blocks(rows, columns, seed=rows + groups + batch)
+    packed, lay = pack(blocks), layout(rows, columns)
+    x = activations(batch, columns, dtype, seed=batch)
+    got = tq1_linear_words(packed, x, layout=lay)
+    assert torch.equal(got, tq1_linear_words(packed, x, layout=lay))
+    sample = np.unique(np.r_[0:64, rows - 70:rows, np.random.default_rng(batch).integers(0, rows, 200)])
+    x64 = x.double().cpu().numpy()
+    want = O.oracle_matmul(blocks[sample], x64, rows=len(sample), columns=columns)
+    assert (np.abs(got.double().cpu().numpy()[:, sample] - want) <= bound(x64, blocks[sample], want, dtype)).all()
+    z = tq1_swiglu_words(packed, x[:, :].mul(0.01), layout=lay).float()
+    both = tq1_linear_words(packed, x[:, :].mul(0.01), layout=lay).float()
+    gate, up = both[:, 0::2], both[:, 1::2]
+    silu = (gate / (1.0 + torch.exp(-gate)) * up).to(dtype).float()
+    finite = torch.isfinite(silu)
+    assert bool(((z - silu).abs() <= silu.abs() * 4 * ROUNDOFF[dtype] + 2.0 ** -24)[finite].all())
