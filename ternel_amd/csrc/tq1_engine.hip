@@ -3510,7 +3510,7 @@ constexpr int64_t kTritMatmulPartialBytes = int64_t{16} << 20;
 // Equal K chunks up to this many times the workgroups that chunks of any size
 // would need; unequal ones below this share of their estimated time.
 constexpr int64_t kTritEqualSplitSlack = 3;
-constexpr double kTritUnequalGain = 0.85;
+constexpr double kTritUnequalGain = 0.95;
 
 // batches: a batch past one tile runs as tiles of nearly equal size, in as
 // many launches as the counters and the partials' limit need; otherwise it is
@@ -3568,11 +3568,13 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
         };
         // 33-64 rows a tile: two workgroups per CU, whose loop the LDS bounds,
         // so a second workgroup on a CU adds its groups' time and a third
-        // waits for a slot. The split of least estimated time, in us, fitted
-        // to sweeps of every split (seven shapes, M=64-384, within 10 %
-        // but for chunks too short to matter): a start, 0.82 per group for a
-        // CU's only workgroup or 0.66 for each of several, 8 per further round
-        // of two, 3 for a reduction.
+        // waits for a slot; the last arriver of a tile adds the chunks alone.
+        // The split of least estimated time, in us, fitted to 686 calls
+        // (matrices under 12 MiB, M=33-768; half of them within 4.6 %, nine in
+        // ten within 12.7 %): a start, 0.55 per chunk of a reduction, per group
+        // 0.93 for a CU's only workgroup and 1.07 for two, and a further round
+        // of two. (Without the reduction's term 5449 x 5632 M=91 took 11 chunks
+        // of 4, 37.4 us, against 24.5.)
         auto fastest = [&]() {
             const int64_t cus = device_cu_count();
             int best = 0;
@@ -3583,9 +3585,10 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
                     const int64_t chunk = chunk_of(k, 4, equal);
                     if (!chunk) continue;
                     const int64_t n = blocks * k, per_cu = ceil_div(n, cus), rounds = ceil_div(n, 2 * cus);
-                    const double us = (k > 1 ? 8.0 : 5.0) +
-                                      static_cast<double>(chunk) * (per_cu == 1 ? 0.82 : 0.66 * static_cast<double>(per_cu)) +
-                                      (per_cu > 1 ? 1.5 : 0.0) + 8.0 * static_cast<double>(rounds - 1);
+                    const double groups = static_cast<double>(chunk);
+                    const double us = (k > 1 ? 6.3 + 0.55 * static_cast<double>(k) : 2.6) +
+                                      (per_cu == 1 ? 0.93 * groups : 5.0 + 1.07 * groups) +
+                                      static_cast<double>(rounds - 1) * (8.7 + 0.58 * groups);
                     if (us < most_us && (!best || us <= least)) {
                         best = static_cast<int>(k);
                         least = us;
