@@ -4274,21 +4274,19 @@ int ternel_tq1_matmul(const uint32_t *packed, const void *x, void *y, int64_t M,
                 return launch_strip<float>(packed, x, y, geo, s, false, ws);
         }
     }
+    LutPlan plan;  // what the LUT23 kernel refuses is refused for either kernel
+    if ((rc = plan_lut(M, rows, columns, batch_tile, k_split, &plan)) != TERNEL_TQ1_OK) return rc;
+    if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
+    if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
     if (matmul_uses_trit(M, rows, columns, dtype, batch_tile, k_split) && !(reinterpret_cast<uintptr_t>(x) & 15u)) {
         TritPlan trit;
         if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true, kTritMatmulPartialBytes)) != TERNEL_TQ1_OK) return rc;
-        if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
-        if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
         const size_t need = trit_workspace_bytes(trit);
         if (need && (!ws || ws_bytes < need))
             return fail(TERNEL_TQ1_EINVAL, "workspace of %zu bytes is smaller than the %zu the split needs", ws_bytes,
                         need);
         return launch_trit(packed, x, y, M, rows, columns, dtype, trit, ws, static_cast<hipStream_t>(stream), 0);
     }
-    LutPlan plan;
-    if ((rc = plan_lut(M, rows, columns, batch_tile, k_split, &plan)) != TERNEL_TQ1_OK) return rc;
-    if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
-    if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
     const size_t need = plan.counter_bytes + plan.partial_bytes;
     if (need && (!ws || ws_bytes < need))
         return fail(TERNEL_TQ1_EINVAL, "workspace of %zu bytes is smaller than the %zu the split needs", ws_bytes,
@@ -4329,16 +4327,6 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
                 return launch_strip<float>(packed, x, y, geo, s, false, ws);
         }
     }
-    if (matmul_uses_trit(M, rows, columns, dtype, batch_tile, k_split) && !(reinterpret_cast<uintptr_t>(x) & 15u)) {
-        TritPlan trit;  // its partials fit the scratch
-        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true, kTritMatmulPartialBytes)) != TERNEL_TQ1_OK) return rc;
-        if ((rc = check_packed_pointer(packed)) != TERNEL_TQ1_OK) return rc;
-        if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
-        hipStream_t s = static_cast<hipStream_t>(stream);
-        void *ws = nullptr;
-        if (trit.k_split > 1 && (rc = noalloc_scratch(s, &ws)) != TERNEL_TQ1_OK) return rc;
-        return launch_trit(packed, x, y, M, rows, columns, dtype, trit, ws, s, 0);
-    }
     LutPlan plan;
     if ((rc = plan_lut(M, rows, columns, batch_tile, k_split, &plan, kNoAllocPartialBytes)) != TERNEL_TQ1_OK)
         return rc;
@@ -4353,6 +4341,12 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
     if (!x || !y) return fail(TERNEL_TQ1_EINVAL, "null pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
     void *ws = nullptr;
+    if (matmul_uses_trit(M, rows, columns, dtype, batch_tile, k_split) && !(reinterpret_cast<uintptr_t>(x) & 15u)) {
+        TritPlan trit;  // its partials fit the scratch
+        if ((rc = plan_trit(M, rows, columns, dtype, 0, &trit, true, kTritMatmulPartialBytes)) != TERNEL_TQ1_OK) return rc;
+        if (trit.k_split > 1 && (rc = noalloc_scratch(s, &ws)) != TERNEL_TQ1_OK) return rc;
+        return launch_trit(packed, x, y, M, rows, columns, dtype, trit, ws, s, 0);
+    }
     if (plan.k_split > 1 && (rc = noalloc_scratch(s, &ws)) != TERNEL_TQ1_OK) return rc;
     switch (dtype) {
         case TERNEL_TQ1_F16:
@@ -4549,6 +4543,8 @@ int ternel_tq1_swiglu(const uint32_t *packed, const void *x, void *z, int64_t M,
     }
     // The trit kernel writes SiLU(g) * u itself.
     const bool lut = linear_uses_lut(M, rows, columns, dtype);
+    LutPlan plan;
+    if (lut && (rc = plan_lut(M, rows, columns, 1, 0, &plan)) != TERNEL_TQ1_OK) return rc;
     const bool matmul_trit =
         lut && matmul_uses_trit(M, rows, columns, dtype, 0, 0) && !(reinterpret_cast<uintptr_t>(x) & 15u);
     if (matmul_trit || (!lut && swiglu_gemm_uses_trit(M, rows, columns, dtype))) {
@@ -4564,9 +4560,7 @@ int ternel_tq1_swiglu(const uint32_t *packed, const void *x, void *z, int64_t M,
         return launch_trit(packed, x, z, M, rows, columns, dtype, trit, ws, s,
                            kTritGlu | (matmul_trit ? 0 : kTritIeeeScales));
     }
-    if (linear_uses_lut(M, rows, columns, dtype)) {
-        LutPlan plan;
-        if ((rc = plan_lut(M, rows, columns, 1, 0, &plan)) != TERNEL_TQ1_OK) return rc;
+    if (lut) {
         const size_t need = plan.counter_bytes + plan.partial_bytes;
         if (need && (!ws || ws_bytes < need))
             return fail(TERNEL_TQ1_EINVAL, "workspace of %zu bytes is smaller than the %zu the split needs", ws_bytes,

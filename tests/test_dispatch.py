@@ -77,3 +77,21 @@ def test_the_27b_widths_split_into_equal_chunks() -> None:
                                (8, 34816, 40, 5), (32, 8192, 40, 10), (32, 5120, 48, 6), (8, 1024, 40, 10),
                                (8, 4096, 32, 8)):
         assert direct_split(M, rows, groups) == k, (M, rows, groups)
+
+
+def test_what_the_matmul_path_refuses_it_refuses_for_every_kernel() -> None:
+    """More K chunks than a LUT23 launch takes, in a batch that the trit kernel
+    would run: refused before any launch, with and without a workspace."""
+    handle = _lib.lib()
+    columns = (65536 * 4 + 1) * 128
+    aligned = 1 << 20  # never read: the call is refused first
+    for M in (4, 8, 64):
+        assert handle.ternel_tq1_matmul_workspace_bytes(M, 256, columns, 0, 0) == 0
+        for rc in (handle.ternel_tq1_matmul(aligned, aligned, aligned, M, 512, columns, _lib.DTYPE_F16, 0, 0, None, 0, None),
+                   handle.ternel_tq1_matmul_noalloc(aligned, aligned, aligned, M, 512, columns, _lib.DTYPE_F16, 0, 0,
+                                                    None)):
+            assert rc == _lib.TERNEL_TQ1_EINVAL
+            assert "K too large for one launch" in _lib.last_error()
+        assert handle.ternel_tq1_swiglu(aligned, aligned, aligned, M, 512, columns, _lib.DTYPE_F32, None, 0,
+                                        None) == _lib.TERNEL_TQ1_EINVAL
+        assert "K too large for one launch" in _lib.last_error()
