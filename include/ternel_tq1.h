@@ -302,6 +302,15 @@ size_t ternel_tq1_linear_workspace_bytes(int64_t M, int64_t rows, int64_t column
 int ternel_tq1_linear_kernel(int64_t M, int64_t rows, int64_t columns, int dtype);
 
 /*
+ * The kernel ternel_tq1_linear launches for this shape and 16-byte aligned x:
+ * the strip form or the LUT23 kernel, the trit kernel (the DIRECT form's), or
+ * the TILE or WIDE form's. Negative on a rejected shape or dtype; host-only.
+ */
+#define TERNEL_TQ1_KERNEL_TRIT 101
+#define TERNEL_TQ1_KERNEL_STRIP 102
+int ternel_tq1_linear_launches(int64_t M, int64_t rows, int64_t columns, int dtype);
+
+/*
  * A SwiGLU MLP's gate and up projections as one packed weight, with the
  * elementwise step fused: z[m][r] = SiLU(g) * u, where g and u are rows 2r and
  * 2r + 1 of x @ W^T (the packed weight's rows alternate gate, up -- see

@@ -4493,6 +4493,18 @@ int ternel_tq1_linear_kernel(int64_t M, int64_t rows, int64_t columns, int dtype
     return resolve_gemm_form(M, rows, columns, linear_gemm_form(M, rows, columns, dtype), 0);
 }
 
+int ternel_tq1_linear_launches(int64_t M, int64_t rows, int64_t columns, int dtype) {
+    const int path = ternel_tq1_linear_kernel(M, rows, columns, dtype);
+    if (path < 0) return path;
+    if (path == TERNEL_TQ1_KERNEL_LUT23) {
+        if (uses_strip_gemv(M, 0, 0, rows, columns)) return TERNEL_TQ1_KERNEL_STRIP;
+        return matmul_uses_trit(M, rows, columns, dtype, 0, 0) ? TERNEL_TQ1_KERNEL_TRIT : path;
+    }
+    return gemm_uses_trit(M, rows, columns, dtype, linear_gemm_form(M, rows, columns, dtype), path, 0)
+               ? TERNEL_TQ1_KERNEL_TRIT
+               : path;
+}
+
 // Whether the fused SwiGLU's GEMM is the trit kernel.
 static bool swiglu_gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype) {
     const int form = linear_gemm_form(M, rows, columns, dtype);

@@ -93,6 +93,8 @@ class MatmulConfig:
 GEMM_FORMS = {"auto": 0, "tile": 1, "direct": 2, "wide": 3}
 DIRECT_MAX_BATCH = 64
 KERNEL_LUT23 = 100  # ternel_tq1_linear_kernel's answer for the matmul path
+# ternel_tq1_linear_launches' answers
+KERNEL_NAMES = {KERNEL_LUT23: "lut23", 101: "trit", 102: "strip", 1: "tile", 3: "wide"}
 
 
 @dataclass(frozen=True)
@@ -483,6 +485,15 @@ def tq1_linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTen
     check_packed(packed, layout=layout)
     check_activations(x, layout=layout)
     return _linear(packed, _aligned_rows(x), layout)
+
+
+def linear_kernel(layout: PackedTensorLayout, batch: int, dtype: torch.dtype) -> str:
+    """The kernel that a module's product of ``batch`` activation rows launches
+    (``select_kernel`` names the path that chooses it)."""
+    code = _lib.lib().ternel_tq1_linear_launches(batch, layout.rows, layout.columns, _DTYPE_CODE[dtype])
+    if code < 0:
+        raise FormatError(_lib.last_error())
+    return KERNEL_NAMES[code]
 
 
 def linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout) -> torch.Tensor:

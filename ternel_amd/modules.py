@@ -55,7 +55,8 @@ _KERNEL_NAMES = {100: "lut23", 1: "gemm", 2: "gemm", 3: "gemm"}
 
 
 def select_kernel(layout: PackedTensorLayout, batch: int, dtype: torch.dtype) -> str:
-    """``"lut23"`` or ``"gemm"`` for ``batch`` activation rows: the library's own choice."""
+    """``"lut23"`` or ``"gemm"`` for ``batch`` activation rows: the entry point of the
+    library's own choice (``kernels.linear_kernel`` names the kernel that runs)."""
     from . import _lib
     from .kernels import _DTYPE_CODE
 

@@ -14,6 +14,7 @@ import torch
 
 from tests.conftest import GOLDEN
 from ternel_amd import _lib
+from ternel_amd.kernels import linear_kernel
 from ternel_amd.layout import PackedTensorLayout
 from ternel_amd.modules import select_kernel
 
@@ -95,3 +96,27 @@ def test_what_the_matmul_path_refuses_it_refuses_for_every_kernel() -> None:
         assert handle.ternel_tq1_swiglu(aligned, aligned, aligned, M, 512, columns, _lib.DTYPE_F32, None, 0,
                                         None) == _lib.TERNEL_TQ1_EINVAL
         assert "K too large for one launch" in _lib.last_error()
+
+
+def test_the_reported_kernel_is_one_the_path_can_launch() -> None:
+    handle = _lib.lib()
+    seen = set()
+    for dtype, code in ((torch.float16, _lib.DTYPE_F16), (torch.bfloat16, _lib.DTYPE_BF16), (torch.float32, _lib.DTYPE_F32)):
+        for rows, columns in ((48, 5120), (1024, 5120), (4096, 4096), (5120, 17408), (8192, 5120), (17408, 5120)):
+            layout = PackedTensorLayout.for_tensor(rows, columns)
+            for M in (1, 2, 3, 4, 6, 8, 24, 33, 64, 100, 128, 400, 600, 2048):
+                name = linear_kernel(layout, M, dtype)
+                seen.add(name)
+                path = handle.ternel_tq1_linear_kernel(M, rows, columns, code)
+                if path == 100:
+                    assert name in ("lut23", "strip", "trit")
+                    assert name != "strip" or M == 1
+                elif path == 2:
+                    assert name == "trit"
+                else:
+                    assert name in ("trit", NAMES[path])
+                # the workspace that the launch needs tells the trit kernel's split from the wide form's
+                if name == "wide":
+                    assert handle.ternel_tq1_linear_workspace_bytes(M, rows, columns, code) > 65536
+    assert seen == {"lut23", "strip", "trit", "wide", "tile"}
+    assert handle.ternel_tq1_linear_launches(0, 64, 128, 0) == _lib.TERNEL_TQ1_EINVAL
