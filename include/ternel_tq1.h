@@ -177,7 +177,7 @@ int ternel_tq1_tiled_from_words(const uint32_t *packed, int64_t rows, int64_t co
  * region alone, left empty by every call.
  * Batches (M > 1) with both left automatic run the DIRECT form's kernel of
  * ternel_tq1_gemm where it is faster (most matrices from M = 3; fp32, as three
- * bf16 terms per value, exactly, from about M = 4-10 by matrix size), with
+ * bf16 terms per value, exactly, from about M = 5-64 by matrix size), with
  * the same arithmetic per block: acc = fma(scale, sum of +-x, acc) in fp32. x
  * that is not 16-byte aligned takes the LUT23 kernel.
  * ws: at least ternel_tq1_matmul_workspace_bytes(...) bytes (0 when the split

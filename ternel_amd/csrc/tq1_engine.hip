@@ -3601,14 +3601,31 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
         // the target (QKV M=32, 640 workgroups against 320 of 8: 12.8 / 12.9).
         // fp32 past 8 rows stages 4 or 2 groups at a time: chunks of 4 (QKV
         // M=24 19.5 us against 21.7 in chunks of 8, M=16 15.6 / 17.8).
-        int best = plan->staged_rows > 32 ? fastest() : widest(f32 && plan->staged_rows >= 16 ? 4 : 8);
-        if (plan->staged_rows == 32 && blocks * widest(4) >= kDirectTargetWorkgroups) best = widest(4);
+        // (Short rows that only 4 divides take equal chunks of 4: 9052 x 2560 M=6
+        // 7.8 us, 8.2 in 8 + 8 + 4.)
+        const bool fours = (f32 && plan->staged_rows >= 16) || (G % 8 == 4 && G <= 40);
+        int best = plan->staged_rows > 32 ? fastest() : widest(fours ? 4 : 8);
+        if (plan->staged_rows == 32 && G % 4 == 0 && blocks * widest(4) >= kDirectTargetWorkgroups) best = widest(4);
         // More chunks of 4 than the reduction loads in one batch pay only where
         // next to no workgroups are (us, chunks of 4 / 8: 2048 x 10752 M=3 11.0
         // / 9.5, 768 x 17408 9.4 / 8.9, but 128 x 12800 7.1 / 7.6).
         if (plan->staged_rows <= 32 && blocks * best < kDirectMinWorkgroups &&
             (widest(4) <= kTritReduceBatch || blocks <= 4))
             best = std::max(best, widest(4));
+        // Other equal chunks where they do better: a few groups on a few rows in
+        // chunks of one or two, that many workgroups at once (129 x 1280 M=6 4.6
+        // us, 5.4 in 4 + 4 + 2); fewer chunks that all but reach the target
+        // (12649 x 7040 M=4, 495 workgroups, 12.5, 13.2 with 693); a few groups
+        // on many rows in few chunks or one (22035 x 1152 M=16 7.9, 9.3 in 8 +
+        // 1; 16892 x 1280 fp32 M=23 19.7 in 5 + 5, 23.6 in 4 + 4 + 2).
+        if (plan->staged_rows <= 32 && G % 4) {
+            const int divisor = largest_divisor_split(G, blocks, kDirectTargetWorkgroups);
+            if (chunk_of(divisor, 1, true) &&
+                (divisor > best ? divisor <= kTritReduceBatch
+                                : 8 * blocks * divisor >= 7 * kDirectTargetWorkgroups ||
+                                      (G <= 12 && 4 * blocks >= kDirectTargetWorkgroups)))
+                best = divisor;
+        }
         k_split = best;  // (a split of one always qualifies)
         // (the same chunk whichever way `best` was found: equal where it can be)
         plan->chunk_groups = static_cast<int>(std::min(G, G % best == 0 ? G / best : chunk_of(best, 4, false)));
@@ -3889,7 +3906,9 @@ int linear_gemm_form(int64_t M, int64_t rows, int64_t columns, int dtype) {
 // (us, trit / best other fp16 form; the bf16 wide form is 2-8 us slower than
 // the fp16 one for its scaling pass):
 //   under 4 MB: 4096 square M=128 17 / 26, M=768 44 / 47; k_proj M=128 16 / 27,
-//   M=768 26 / 30, M=1024 34 / 33; 3000 x 3072 M=768 35 / 35;
+//   M=768 26 / 30, M=1024 34 / 33; 3000 x 3072 M=768 35 / 35; short rows under
+//   64 KB the tile form's one short launch: 57 x 1152 M=90 10.8 / 10.1, 110 x 1664 M=81
+//   11.8 / 11.0;
 //   under 12 MB: out_proj M=128 22 / 29, M=384 39 / 44, M=512 58 / 54; QKV M=203
 //   34 / 41, M=384 52 / 52; 12288 x 2048 M=128 17 / 29, M=384 37 / 37, bf16 M=512
 //   40 / 42; but on long rows 1500 x 17408 M=128 30 / 29, M=203 42 / 34, where
@@ -3899,7 +3918,7 @@ int linear_gemm_form(int64_t M, int64_t rows, int64_t columns, int dtype) {
 bool trit_beats_wide(int64_t M, int64_t rows, int64_t columns, int dtype) {
     const int64_t G = columns / kBlockWeights, bytes = rows * G * kBlockBytes;
     const bool bf16 = dtype == TERNEL_TQ1_BF16;
-    if (bytes < 4 << 20) return M <= 768;
+    if (bytes < 4 << 20) return M <= 768 && (bf16 || G >= 16 || bytes >= 64 << 10);
     if (bytes < 12 << 20) return bf16 ? M <= 512 : (G <= 64 && M <= 384);
     return bf16 && bytes < kTritBf16MatrixBytes && M <= (G > 64 ? 128 : 64);
 }
@@ -3918,22 +3937,38 @@ bool gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int for
 
 // ternel_tq1_matmul's batches with the configuration left automatic: the trit
 // kernel decodes a weight once per batch where the LUT23 kernel looks it up
-// once per vector. Measured on MI355X (us, LUT23 / trit):
-//   fp16 and bf16, M=2: gate/up 13.3 / 12.5, 4096 square 7.4 / 7.0, k_proj
-//   6.7 / 6.1, but QKV 8.8 / 9.4, out_proj 8.1 / 8.8 (matrices of 4-12 MB);
-//   M=3: gate/up 16.0 / 12.1, QKV 9.8 / 9.4, out_proj 9.2 / 8.7, 4096 square
-//   7.7 / 7.0; a 48-row matrix (one row block) 5.2 / 5.4 at M=3, 5.7 / 5.5 at 8.
-//   fp32 (three MFMAs per K slice): gate/up M=4 19.2 / 19.4, M=6 25.9 / 20.0;
-//   QKV M=4 10.9 / 13.9, M=6 14.7 / 13.8; out_proj M=6 12.2 / 11.6; 4096
-//   square M=8 9.8 / 10.7; k_proj M=8 8.1 / 10.3. The LUT23 kernel's time per
-//   vector grows with the matrix and the trit kernel's fixed cost does not, so
-//   the line is a product of both.
+// once per vector, and starts slower. From sweeps of both kernels on MI355X
+// (cold weights; 64-17408 rows, 9-136 groups per row; us, LUT23 / trit):
+//   fp16 and bf16, M=2: within 10 % of each other where the trit kernel is not
+//   kept busy or the LUT23 kernel streams well (gate/up 13.3 / 12.5, 4096
+//   square 8.1 / 7.7, k_proj 6.7 / 6.1; but 512 x 10752 6.9 / 7.9, QKV 8.8 /
+//   9.4, out_proj 8.1 / 8.8, 17408 x 10752 22.0 / 24.7);
+//   M=3: gate/up 16.0 / 12.1, QKV 9.8 / 9.4, out_proj 9.2 / 8.7, 320 x 5120
+//   6.3 / 6.0, but 256 x 10752 6.5 / 7.7; a 48-row matrix 5.2 / 5.4 at M=3,
+//   5.7 / 5.5 at 8.
+//   fp32 (three MFMAs per K slice, which cost twice as much at 17-32 rows a
+//   tile): the LUT23 kernel's time grows with the product of vectors, rows and
+//   groups, the trit kernel's less than in proportion to the groups: 8192 x 5120
+//   M=6 14.7 / 13.8, 4096 x 5120 M=9 11.7 / 11.7, 2048 x 5120 M=16 10.9 / 11.0,
+//   M=24 14.1 / 15.1, M=32 17.6 / 16.0, 949 x 8192 M=32 14.6 / 16.1, M=48 20.1 /
+//   18.5; 219 x 5120 M=64 9.0 / 14.1; short rows 2862 x 1408 M=35 14.1 / 17.5. An odd group count leaves the LUT23 kernel
+//   chunks of one, whose reduction outweighs all that past 32 (2048 x 4736 M=4
+//   13.1 / 9.5, M=12 18.6 / 10.7, 64 x 4736 M=9 9.7 / 9.0), and for fp16 and bf16
+//   as well (1447 x 10368 M=2 19.1 / 10.4, 145 x 5248 M=4 9.7 / 7.6).
+constexpr int64_t kTritF32Work = 2'600'000, kTritF32WideWork = 4'800'000, kTritF32ShortWork = 5'400'000;
 bool matmul_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int batch_tile, int k_split) {
     if (batch_tile != 0 || k_split != 0 || M < 2) return false;
-    const int64_t bytes = rows * (columns / kBlockWeights) * kBlockBytes;
-    if (dtype == TERNEL_TQ1_F32) return M >= 4 && (M - 2) * (bytes + (1 << 19)) >= 30 << 20;
-    if (rows <= kDirectRows) return M >= 8;
-    return M >= 3 || bytes < 4 << 20 || bytes >= 12 << 20;
+    const int64_t G = columns / kBlockWeights, bytes = rows * G * kBlockBytes;
+    const bool lut_singles = G % 2 && G > 32;
+    if (dtype == TERNEL_TQ1_F32) {
+        if (lut_singles) return M >= (rows > kDirectRows ? 4 : 9);
+        const int64_t work = M <= 16 ? kTritF32Work : (G <= 16 ? kTritF32ShortWork : kTritF32WideWork);
+        return M >= 5 && M * rows >= work / (G + 40);
+    }
+    if (lut_singles && rows > kDirectRows) return true;
+    if (rows <= 2 * kDirectRows) return M >= (rows <= kDirectRows ? 8 : 5);
+    if (M == 2) return (rows >= 5 * kDirectRows && bytes < 3 << 20) || (bytes >= 12 << 20 && G <= 64);
+    return true;
 }
 
 int check_packed_pointer(const void *packed) {

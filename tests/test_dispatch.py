@@ -120,3 +120,34 @@ def test_the_reported_kernel_is_one_the_path_can_launch() -> None:
                     assert handle.ternel_tq1_linear_workspace_bytes(M, rows, columns, code) > 65536
     assert seen == {"lut23", "strip", "trit", "wide", "tile"}
     assert handle.ternel_tq1_linear_launches(0, 64, 128, 0) == _lib.TERNEL_TQ1_EINVAL
+
+
+# Both sides of the lines between the LUT23 and the trit kernel (and, fp16 above 64 rows, the tile
+# form) as measured on an MI355X: the kernel that was the faster one, or within 5 % of it.
+LINES = [
+    # fp16 and bf16 batches of the matmul path: 2 rows, then 3 and 4
+    (torch.float16, 17408, 5120, 2, "trit"), (torch.float16, 17408, 10752, 2, "lut23"),
+    (torch.float16, 8192, 5120, 2, "lut23"), (torch.float16, 5120, 6144, 2, "lut23"),
+    (torch.bfloat16, 1024, 5120, 2, "trit"), (torch.bfloat16, 512, 10752, 2, "lut23"),
+    (torch.float16, 256, 10752, 3, "lut23"), (torch.float16, 320, 5120, 3, "trit"),
+    (torch.bfloat16, 160, 7168, 4, "lut23"), (torch.float16, 48, 5120, 4, "lut23"),
+    # fp32: too few rows or groups, then enough, at each tile width; odd group counts
+    (torch.float32, 17408, 5120, 4, "lut23"), (torch.float32, 17408, 5120, 6, "trit"),
+    (torch.float32, 4096, 5120, 6, "lut23"), (torch.float32, 8192, 5120, 9, "trit"),
+    (torch.float32, 2048, 3072, 16, "lut23"), (torch.float32, 4096, 5120, 16, "trit"),
+    (torch.float32, 949, 5120, 24, "lut23"), (torch.float32, 8192, 5120, 24, "trit"),
+    (torch.float32, 219, 1152, 61, "lut23"), (torch.float32, 512, 8192, 48, "lut23"),
+    (torch.float32, 2048, 8192, 48, "trit"), (torch.float32, 1024, 1664, 64, "lut23"),
+    (torch.float32, 2048, 4736, 4, "trit"), (torch.float32, 2048, 5120, 4, "lut23"),
+    (torch.float32, 64, 4736, 9, "trit"), (torch.float32, 64, 4736, 4, "lut23"),
+    (torch.float32, 136, 2688, 47, "lut23"), (torch.float32, 2862, 1408, 35, "lut23"),
+    (torch.float16, 1447, 10368, 2, "trit"), (torch.bfloat16, 145, 5248, 4, "trit"),
+    # fp16 above the direct form: short rows under 64 KiB keep the tile form
+    (torch.float16, 57, 1152, 90, "tile"), (torch.float16, 54, 3584, 375, "trit"), (torch.float16, 1024, 5120, 128, "trit"),
+    (torch.bfloat16, 57, 1152, 90, "trit"),
+]
+
+
+@pytest.mark.parametrize(("dtype", "rows", "columns", "batch", "kernel"), LINES)
+def test_each_side_of_a_line_runs_its_faster_kernel(dtype, rows, columns, batch, kernel) -> None:
+    assert linear_kernel(PackedTensorLayout.for_tensor(rows, columns), batch, dtype) == kernel
