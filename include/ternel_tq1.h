@@ -238,11 +238,11 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
  *                          kernel on batch tiles of up to 64 rows in place of
  *                          either.
  * bf16 activations (dtype TERNEL_TQ1_BF16) take form AUTO or WIDE and no fixed
- * k_split (size the workspace with form WIDE). Up to 32 rows (64 for matrices
- * under 24 MiB of packed weights, 128 on long rows, 512 under 12 MiB and 768
- * under 4 MiB) they run the DIRECT form's kernel on bf16 MFMAs, as they are;
- * above, the WIDE form after a pre-pass that
- * scales each row by a power of two into fp16's range and converts it (exact:
+ * k_split (size the workspace with form WIDE for either). With AUTO, up to 32
+ * rows (64 for matrices under 24 MiB of packed weights, 128 on long rows, 512
+ * under 12 MiB and 768 under 4 MiB) they run the DIRECT form's kernel on bf16
+ * MFMAs, as they are; above, and for any batch with WIDE, the WIDE form after
+ * a pre-pass that scales each row by a power of two into fp16's range and converts it (exact:
  * bf16's 8-bit significand fits fp16's 11 bits; values more than 2^28 below
  * the row's largest lose bits), and the fp32 sums are scaled back and rounded
  * once to bf16; inf and NaN propagate as in the reference. F32 is refused.

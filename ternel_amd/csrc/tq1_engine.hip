@@ -3892,14 +3892,15 @@ bool linear_uses_lut(int64_t M, int64_t rows, int64_t columns, int dtype) {
     return M <= (bytes < kLinearSmallMatrixBytes ? kLinearLutMaxBatchSmall : kLinearLutMaxBatch);
 }
 
-// The GEMM form of the library's dispatch for a batch that does not take the
-// LUT23 kernel: bf16 activations run the wide form.
+// The GEMM form whose workspace a batch of the library's dispatch needs, where
+// it does not take the matmul path: bf16 activations run the wide form, or the
+// trit kernel on that form's workspace (gemm_uses_trit).
 int linear_gemm_form(int64_t M, int64_t rows, int64_t columns, int dtype) {
     return dtype == TERNEL_TQ1_BF16 ? TERNEL_TQ1_GEMM_WIDE : TERNEL_TQ1_GEMM_AUTO;
 }
 
 // The trit kernel runs the direct form (fp16), and batches of the automatic
-// forms that it is faster for: bf16 (asked for as WIDE) up to 32 rows, and
+// forms that it is faster for (never a form asked for by name): bf16 up to 32 rows, and
 // tiles of up to 64 rows above that (fp16 where the direct form ends). Small
 // matrices give the wide form's 256-row tiles too few CUs or too long a
 // reduction, and the tile form waits for each group's loads. Measured on MI355X
@@ -3923,12 +3924,12 @@ bool trit_beats_wide(int64_t M, int64_t rows, int64_t columns, int dtype) {
     return bf16 && bytes < kTritBf16MatrixBytes && M <= (G > 64 ? 128 : 64);
 }
 
-// `form` as asked for, `resolved` by resolve_gemm_form.
+// `form` as asked for, `resolved` by resolve_gemm_form (WIDE for bf16).
 bool gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int form, int resolved, int k_split) {
     if (resolved == TERNEL_TQ1_GEMM_DIRECT) return true;
+    if (form != TERNEL_TQ1_GEMM_AUTO) return false;
     if (dtype == TERNEL_TQ1_F16)
-        return form == TERNEL_TQ1_GEMM_AUTO && k_split == 0 && columns <= kWideMaxColumns &&
-               trit_beats_wide(M, rows, columns, dtype);
+        return k_split == 0 && columns <= kWideMaxColumns && trit_beats_wide(M, rows, columns, dtype);
     if (dtype != TERNEL_TQ1_BF16 || resolved != TERNEL_TQ1_GEMM_WIDE) return false;
     WidePlan wide;  // what the wide form refuses is left for it to refuse
     return (M <= kAutoDirectMaxBatch || trit_beats_wide(M, rows, columns, dtype)) &&
@@ -4410,7 +4411,7 @@ size_t ternel_tq1_gemm_workspace_bytes(int64_t M, int64_t rows, int64_t columns,
         if (plan_wide(M, rows, columns, k_split, &wide) != TERNEL_TQ1_OK) return 0;
         TritPlan trit;
         size_t small = 0;  // what a bf16 batch of this size uses
-        if (gemm_uses_trit(M, rows, columns, TERNEL_TQ1_BF16, form, form, 0) &&
+        if (gemm_uses_trit(M, rows, columns, TERNEL_TQ1_BF16, TERNEL_TQ1_GEMM_AUTO, form, 0) &&
             plan_trit(M, rows, columns, TERNEL_TQ1_BF16, 0, &trit, true) == TERNEL_TQ1_OK)
             small = trit_workspace_bytes(trit);
         return std::max(kPartialOffset + wide.partial_bytes + wide.xp_bytes, small);
@@ -4437,10 +4438,9 @@ int ternel_tq1_gemm(const uint32_t *packed, const void *x, void *y, int64_t M, i
             return fail(TERNEL_TQ1_EINVAL, "bf16 activations run the wide form (form %d or %d), got %d",
                         TERNEL_TQ1_GEMM_AUTO, TERNEL_TQ1_GEMM_WIDE, form);
         if (k_split > 1) return fail(TERNEL_TQ1_EINVAL, "the wide form takes no fixed K split, got %d", k_split);
-        form = TERNEL_TQ1_GEMM_WIDE;
     }
     const int asked = form;
-    form = resolve_gemm_form(M, rows, columns, form, k_split);
+    form = dtype == TERNEL_TQ1_BF16 ? TERNEL_TQ1_GEMM_WIDE : resolve_gemm_form(M, rows, columns, form, k_split);
     if (gemm_uses_trit(M, rows, columns, dtype, asked, form, k_split)) {
         TritPlan trit;
         const bool direct = form == TERNEL_TQ1_GEMM_DIRECT;
@@ -4507,8 +4507,7 @@ int ternel_tq1_linear(const uint32_t *packed, const void *x, void *y, int64_t M,
                       int dtype, void *ws, size_t ws_bytes, void *stream) {
     if (linear_uses_lut(M, rows, columns, dtype))
         return ternel_tq1_matmul(packed, x, y, M, rows, columns, dtype, 0, 0, ws, ws_bytes, stream);
-    return ternel_tq1_gemm(packed, x, y, M, rows, columns, dtype, linear_gemm_form(M, rows, columns, dtype), 0, ws,
-                           ws_bytes, stream);
+    return ternel_tq1_gemm(packed, x, y, M, rows, columns, dtype, TERNEL_TQ1_GEMM_AUTO, 0, ws, ws_bytes, stream);
 }
 
 // Where the GEMM path's fp16 gate/up output sits in the workspace: after the
@@ -4535,15 +4534,13 @@ int ternel_tq1_linear_launches(int64_t M, int64_t rows, int64_t columns, int dty
         if (uses_strip_gemv(M, 0, 0, rows, columns)) return TERNEL_TQ1_KERNEL_STRIP;
         return matmul_uses_trit(M, rows, columns, dtype, 0, 0) ? TERNEL_TQ1_KERNEL_TRIT : path;
     }
-    return gemm_uses_trit(M, rows, columns, dtype, linear_gemm_form(M, rows, columns, dtype), path, 0)
-               ? TERNEL_TQ1_KERNEL_TRIT
-               : path;
+    return gemm_uses_trit(M, rows, columns, dtype, TERNEL_TQ1_GEMM_AUTO, path, 0) ? TERNEL_TQ1_KERNEL_TRIT : path;
 }
 
 // Whether the fused SwiGLU's GEMM is the trit kernel.
 static bool swiglu_gemm_uses_trit(int64_t M, int64_t rows, int64_t columns, int dtype) {
-    const int form = linear_gemm_form(M, rows, columns, dtype);
-    return gemm_uses_trit(M, rows, columns, dtype, form, resolve_gemm_form(M, rows, columns, form, 0), 0);
+    const int form = resolve_gemm_form(M, rows, columns, linear_gemm_form(M, rows, columns, dtype), 0);
+    return gemm_uses_trit(M, rows, columns, dtype, TERNEL_TQ1_GEMM_AUTO, form, 0);
 }
 
 size_t ternel_tq1_swiglu_workspace_bytes(int64_t M, int64_t rows, int64_t columns, int dtype) {

@@ -443,10 +443,10 @@ def tq1_gemm_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTenso
                    config: GemmConfig | None = None) -> torch.Tensor:
     """``x @ W.T`` on the MFMA kernels (reference tq1_gemm, kernels.py:1287-1357).
 
-    fp16 activations run the form ``config`` names. bf16 ones run on bf16
-    operands in small batches and the wide form above them, each row scaled by
-    a power of two into fp16's range (exact: bf16's significand fits fp16's)
-    and the fp32 sums scaled back and rounded once to bf16. fp32 activations --
+    fp16 activations run the form ``config`` names. bf16 ones run the wide form,
+    each row scaled by a power of two into fp16's range (exact: bf16's
+    significand fits fp16's) and the fp32 sums scaled back and rounded once to
+    bf16; with ``"auto"`` small batches run on bf16 operands instead. fp32 activations --
     whose significand fp16 would not hold -- and bf16 ones with a fixed K split
     run through the LUT23 kernel, which computes in fp32 from the activations
     as given."""
@@ -462,7 +462,7 @@ def tq1_gemm_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTenso
     if x.dtype == torch.bfloat16:
         if config.form not in ("auto", "wide"):
             raise FormatError(f"bf16 activations run the wide GEMM form, not {config.form!r}")
-        form_name = "wide"
+        form_name = config.form
     else:
         form_name = config.form_for(batch)
     if form_name == "direct" and batch > DIRECT_MAX_BATCH:
@@ -472,7 +472,8 @@ def tq1_gemm_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTenso
     index = x.get_device()
     _surface(index)
     out = x.new_empty((batch, layout.rows))
-    ws = workspace(x.device, _gemm_bytes(index, batch, layout.rows, layout.columns, form, config.k_split))
+    sized = GEMM_FORMS["wide"] if x.dtype == torch.bfloat16 else form
+    ws = workspace(x.device, _gemm_bytes(index, batch, layout.rows, layout.columns, sized, config.k_split))
     _lib.check(_lib.lib().ternel_tq1_gemm(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns,
         _DTYPE_CODE[x.dtype], form, config.k_split, ws.data_ptr() if ws is not None else None,

@@ -151,3 +151,15 @@ LINES = [
 @pytest.mark.parametrize(("dtype", "rows", "columns", "batch", "kernel"), LINES)
 def test_each_side_of_a_line_runs_its_faster_kernel(dtype, rows, columns, batch, kernel) -> None:
     assert linear_kernel(PackedTensorLayout.for_tensor(rows, columns), batch, dtype) == kernel
+
+
+def test_a_form_asked_for_by_name_is_the_one_that_runs() -> None:
+    """bf16, a shape the trit kernel runs unsplit and so without a workspace: the
+    wide form always needs one, and is refused for the lack of it."""
+    handle = _lib.lib()
+    rows, columns = 256, 128
+    assert linear_kernel(PackedTensorLayout.for_tensor(rows, columns), 8, torch.bfloat16) == "trit"
+    aligned = 1 << 20  # never read
+    rc = handle.ternel_tq1_gemm(aligned, aligned, aligned, 8, rows, columns, _lib.DTYPE_BF16, 3, 0, None, 0, None)
+    assert rc == _lib.TERNEL_TQ1_EINVAL
+    assert "workspace of 0 bytes" in _lib.last_error()

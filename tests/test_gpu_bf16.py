@@ -1,6 +1,7 @@
-"""bf16 activations on the matrix cores (the wide form after scale_rows_kernel).
+"""bf16 activations on the matrix cores: the wide form after scale_rows_kernel
+(by name, and large batches), and the trit kernel on bf16 operands (smaller ones).
 
-Each activation row is scaled by a power of two into fp16's range (exact for
+For the wide form each activation row is scaled by a power of two into fp16's range (exact for
 bf16 values: their 8-bit significand fits fp16's 11 bits) and the fp32 sums
 are scaled back and rounded once to bf16. Pinned against the fp64 oracle with
 the reference's bf16 tolerance (src/ternel_mlx/kernel_gate.py:113, 1e-2) on
@@ -19,8 +20,8 @@ import torch
 from oracle import tq1_oracle as O
 from tests.gpu_util import dev, layout, pack, random_blocks, to_dev
 from ternel_amd import _lib, synthetic
-from ternel_amd.kernels import (GemmConfig, MatmulConfig, pack_weights, tq1_gemm_words, tq1_linear_words,
-                                tq1_matmul_words, tq1_swiglu_words)
+from ternel_amd.kernels import (GemmConfig, MatmulConfig, linear_kernel, pack_weights, tq1_gemm_words,
+                                tq1_linear_words, tq1_matmul_words, tq1_swiglu_words)
 from ternel_amd.format import FormatError
 from ternel_amd.layout import PackedTensorLayout
 
@@ -133,6 +134,89 @@ def test_bf16_fused_swiglu_on_the_matrix_cores() -> None:
     diff = (z.float() - want.float()).abs()
     tol = want.float().abs().clamp_min(2.0 ** -126) * 2.0 ** -7
     assert bool((diff <= tol).all())
+
+
+# The wide form by name (M=8 in one 32-row block, 64 in two, 80 and 300 in the permuted copy's wider
+# tiles) beside "auto", which runs these on bf16 operands up to M=300 (linear_kernel): rows beyond
+# fp16's range, inf and NaN, exact integers.
+FORMS = [(form, batch) for form in ("wide", "auto") for batch in (8, 64, 80, 300)]
+
+
+@pytest.mark.parametrize(("form", "batch"), FORMS)
+def test_each_form_keeps_rows_beyond_fp16_range_and_non_finite_values(form, batch) -> None:
+    rows, columns = 512, 2048
+    assert linear_kernel(layout(rows, columns), batch, torch.bfloat16) == "trit"
+    blocks = random_blocks(rows, columns, seed=19 + batch)
+    rng = np.random.default_rng(batch)
+    x = rng.normal(0.0, 1.0, size=(batch, columns))
+    x[0] *= 2.0 ** 100
+    x[1] *= 2.0 ** -100
+    x[2] *= 2.0 ** rng.integers(-20, 21, size=columns)
+    x[3, 5], x[4, 700], x[5, 9], x[6, 3] = np.inf, -np.inf, np.nan, 3e38
+    xb = to_dev(x.astype(np.float32)).to(torch.bfloat16)
+    got = tq1_gemm_words(pack(blocks), xb, layout=layout(rows, columns), config=GemmConfig(form=form)).float().cpu().numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = O.oracle_matmul(blocks, bf16_host(xb), rows=rows, columns=columns)
+    for r in range(batch):
+        result = O.compare(got[r:r + 1], want[r:r + 1])
+        assert result["pattern_mismatches"] == 0, r
+        if np.isfinite(want[r]).all():
+            assert result["normalised_max_abs_error"] < BF16_TOLERANCE, r
+
+
+@pytest.mark.parametrize(("form", "batch"), FORMS)
+def test_each_form_is_exact_on_integers(form, batch) -> None:
+    rows, columns = 300, 1024
+    rng = np.random.default_rng(batch)
+    trits = rng.integers(0, 3, size=(rows * 8, 128), dtype=np.uint8)
+    trits[:, 8:] = 1
+    scales = np.tile(np.array([0x00, 0x3C], dtype=np.uint8), (rows * 8, 1))  # fp16 1.0
+    blocks = O.encode_tq1_blocks(scales, trits).reshape(rows, 8, 28)
+    x = rng.integers(-3, 4, size=(batch, columns)).astype(np.float32)
+    got = tq1_gemm_words(pack(blocks), to_dev(x).to(torch.bfloat16), layout=layout(rows, columns),
+                         config=GemmConfig(form=form))
+    want = O.oracle_matmul(blocks, x.astype(np.float64), rows=rows, columns=columns)
+    np.testing.assert_array_equal(got.float().cpu().numpy(), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("batch", (33, 64))
+def test_two_block_tiles_match_the_oracle_through_the_dispatch(batch) -> None:
+    """A matrix past 24 MiB: the dispatch takes the wide form in tiles of two
+    32-row blocks, its activations scaled but not permuted; linear and SwiGLU."""
+    rows, columns = 34816, 5120
+    lay = PackedTensorLayout.for_tensor(rows, columns)
+    assert linear_kernel(lay, batch, torch.bfloat16) == "wide"
+    blocks = synthetic.device_blocks(rows, columns, seed=synthetic.SEED_BASE + 17)
+    packed = pack_weights(blocks, layout=lay)
+    x = synthetic.device_activations(batch, columns, seed=13, sigma=0.5).to(torch.bfloat16)
+    x[1] *= 2.0 ** 60
+    x[2] *= 2.0 ** -60
+    y = tq1_linear_words(packed, x, layout=lay)
+    sample = np.sort(np.random.default_rng(batch).choice(rows // 2, size=96, replace=False))
+    pairs = np.stack([2 * sample, 2 * sample + 1], axis=1).reshape(-1)
+    want = O.oracle_matmul(blocks[torch.from_numpy(pairs).cuda()].cpu().numpy(), bf16_host(x), rows=len(pairs),
+                           columns=columns)
+    got = y.float().cpu().numpy()[:, pairs]
+    for r in range(batch):
+        assert O.compare(got[r:r + 1], want[r:r + 1])["normalised_max_abs_error"] < BF16_TOLERANCE, r
+    gate, up = y.float()[:, 0::2], y.float()[:, 1::2]
+    silu = (gate / (1.0 + torch.exp(-gate)) * up).to(torch.bfloat16).float()
+    diff = (tq1_swiglu_words(packed, x, layout=lay).float() - silu).abs()
+    assert bool((diff <= silu.abs() * 2.0 ** -7 + 2.0 ** -126)[torch.isfinite(silu)].all())
+
+
+def test_the_lut23_kernel_agrees_with_bf16_operands() -> None:
+    """The trit kernel against the LUT23 kernel (a fixed batch tile, so that
+    it is the one that runs): one bf16 step apart, or fp32 reassociation."""
+    rows, columns, batch = 1024, 2560, 64
+    blocks = random_blocks(rows, columns, seed=31)
+    packed = pack(blocks)
+    xb = to_dev(np.random.default_rng(31).normal(0.0, 1.0, size=(batch, columns)).astype(np.float32)).to(torch.bfloat16)
+    got = tq1_linear_words(packed, xb, layout=layout(rows, columns)).float().cpu().numpy()
+    lut = tq1_matmul_words(packed, xb, layout=layout(rows, columns), config=MatmulConfig(batch_tile=1)).float().cpu().numpy()
+    want = O.oracle_matmul(blocks, bf16_host(xb), rows=rows, columns=columns)
+    step = np.exp2(np.floor(np.log2(np.maximum(np.abs(lut), 2.0 ** -126))) - 7)
+    assert (np.abs(got - lut) <= step + 1e-5 * np.abs(want).max(axis=1, keepdims=True)).all()
 
 
 def test_bf16_takes_no_other_mfma_form() -> None:
