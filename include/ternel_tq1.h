@@ -228,7 +228,8 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
  *                          with an ordered in-launch reduction (k_split must
  *                          be 0/1; columns < 2^22);
  *   TERNEL_TQ1_GEMM_AUTO   DIRECT for M <= 32 (M <= 64 for matrices under
- *                          16 MiB of packed weights); WIDE up to M = 64;
+ *                          16 MiB of packed weights, 48 with a k_split
+ *                          given); WIDE up to M = 64;
  *                          above, WIDE when it has at least CUs/4 output
  *                          tiles or 15 (tile, group) steps per CU, TILE
  *                          otherwise (and for a fixed k_split > 1). With no

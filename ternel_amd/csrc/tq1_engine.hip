@@ -3850,6 +3850,7 @@ int launch_wide(const uint32_t *packed, const void *x, void *y, const WidePlan &
 // 32 rows and rows too long for the wide form's 32-bit buffer offsets.
 constexpr int64_t kAutoDirectMaxBatch = 32;
 constexpr int64_t kAutoDirectMaxBatchSmall = 64;
+constexpr int64_t kAutoDirectMaxBatchSmallSplit = 48;  // with a k_split given, which the direct form would be held to
 constexpr int64_t kAutoSmallMatrixBytes = 16ll << 20;
 constexpr int64_t kAutoWideMaxBatch = 64;
 constexpr int64_t kTritBf16MatrixBytes = 24ll << 20;
@@ -3858,7 +3859,8 @@ int device_cu_count();
 int resolve_gemm_form(int64_t M, int64_t rows, int64_t columns, int form, int k_split) {
     if (form != TERNEL_TQ1_GEMM_AUTO) return form;
     const bool small = rows * (columns / kBlockWeights) * kBlockBytes < kAutoSmallMatrixBytes;
-    if (M <= kAutoDirectMaxBatch || (small && M <= kAutoDirectMaxBatchSmall)) return TERNEL_TQ1_GEMM_DIRECT;
+    const int64_t small_max = k_split == 0 ? kAutoDirectMaxBatchSmall : kAutoDirectMaxBatchSmallSplit;
+    if (M <= kAutoDirectMaxBatch || (small && M <= small_max)) return TERNEL_TQ1_GEMM_DIRECT;
     const bool wide_ok = k_split <= 1 && columns <= kWideMaxColumns;
     if (M <= kAutoWideMaxBatch && wide_ok) return TERNEL_TQ1_GEMM_WIDE;
     if (k_split > 1 || columns > kWideMaxColumns) return TERNEL_TQ1_GEMM_TILE;

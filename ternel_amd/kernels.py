@@ -108,10 +108,11 @@ class GemmConfig:
     ``"wide"`` decodes into the operand registers of 256-row output tiles (32
     to 256 activation rows wide) split stream-K over the CUs (prefill; K split
     0 or 1), ``"auto"`` takes ``"direct"`` up to 32 rows (64 for matrices under
-    16 MiB of packed weights), ``"wide"`` up to 64 and, above, ``"wide"`` when
-    it has enough tiles (CUs/4) or work per CU (15 steps) for its stream-K
-    reduction to pay, ``"tile"`` otherwise (and, above 32 rows, whenever a K
-    split above 1 is fixed).
+    16 MiB of packed weights, 48 with a K split given), ``"wide"`` up to 64 and,
+    above, ``"wide"`` when it has enough tiles (CUs/4) or work per CU (15 steps)
+    for its stream-K reduction to pay, ``"tile"`` otherwise (and, above 32 rows,
+    whenever a K split above 1 is fixed); with no K split, up to several hundred
+    rows of a matrix under 12 MiB run the direct form's kernel in batch tiles.
 
     The reference's tiling fields (``batch_block`` .. ``safe_clamp``) are
     accepted by keyword so its configurations construct unchanged; they tile

@@ -163,3 +163,17 @@ def test_a_form_asked_for_by_name_is_the_one_that_runs() -> None:
     rc = handle.ternel_tq1_gemm(aligned, aligned, aligned, 8, rows, columns, _lib.DTYPE_BF16, 3, 0, None, 0, None)
     assert rc == _lib.TERNEL_TQ1_EINVAL
     assert "workspace of 0 bytes" in _lib.last_error()
+
+
+def test_a_given_split_moves_no_batch_to_the_direct_form() -> None:
+    """AUTO with a k_split at 49-64 rows on a small matrix: one K chunk runs the
+    wide form (whose workspace holds more than partials), several the tile
+    form; without one the direct form, up to 48 rows in any case."""
+    size = _lib.lib().ternel_tq1_gemm_workspace_bytes
+    rows, columns = 4096, 4096
+    for M in (49, 56, 64):
+        assert size(M, rows, columns, 0, 0) == size(M, rows, columns, 2, 0)
+        assert size(M, rows, columns, 0, 1) == size(M, rows, columns, 3, 1)
+        assert size(M, rows, columns, 0, 4) == size(M, rows, columns, 1, 4)
+    for k_split in (0, 1, 4):
+        assert size(48, rows, columns, 0, k_split) == size(48, rows, columns, 2, k_split)
