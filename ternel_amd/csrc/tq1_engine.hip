@@ -1716,7 +1716,8 @@ __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (
 // every activation type with no conversion of the weights or activations:
 //   fp16, bf16  the activations as they are (products with -1/0/+1 exact);
 //   fp32        each value as three bf16 terms (its significand's upper,
-//               middle and lower 8 bits: exact), three MFMAs per K slice.
+//               middle and lower 8 bits, the lower ones scaled up so that
+//               none is lost: exact), three MFMAs per K slice.
 // The weights are the MFMA's second operand, so a lane's 16 sums belong to one
 // weight row -- its own: the scale is a per-lane scalar, an output row's
 // stores are contiguous, and only the sums of real activation rows are
@@ -1739,9 +1740,14 @@ __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
+// kOne: the bits a trit of +1 has in the operand, 1 / kScale. In fp32 half of 1,
+// so that the middle terms below, kept at 2^8 times their value, sum to no more
+// than the values do; 2^-8 of it is kOne without kLowerBit.
 template <typename T>
 struct TritOperand {  // bf16 and (as three bf16 terms) fp32
-    static constexpr uint32_t kOne = 0x3f80u;
+    static constexpr uint32_t kOne = sizeof(T) == 4 ? 0x3f00u : 0x3f80u;
+    static constexpr float kScale = sizeof(T) == 4 ? 2.0f : 1.0f;
+    static constexpr uint32_t kLowerBit = 0x0400u;
     static constexpr int kPlanes = sizeof(T) == 4 ? 3 : 1;
     static __device__ __forceinline__ float16v mfma(u32x4 a, u32x4 b, float16v c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
@@ -1751,6 +1757,7 @@ struct TritOperand {  // bf16 and (as three bf16 terms) fp32
 template <>
 struct TritOperand<_Float16> {
     static constexpr uint32_t kOne = 0x3c00u;
+    static constexpr float kScale = 1.0f;
     static constexpr int kPlanes = 1;
     static __device__ __forceinline__ float16v mfma(u32x4 a, u32x4 b, float16v c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0,
@@ -1758,9 +1765,11 @@ struct TritOperand<_Float16> {
     }
 };
 
-// An fp32 value as three bf16 terms, bits in the upper half of each: hi + mid
-// + lo == v exactly (the subtractions are exact: each term takes the leading
-// 8 significand bits left). inf and NaN go in hi alone.
+// An fp32 value as three bf16 terms, bits in the upper half of each: hi + 2^-8
+// mid + 2^-16 lo == v exactly for every finite v (each term takes the leading 8
+// significand bits left, the subtractions and the powers of two are exact, and
+// 2^-149, the last bit of a subnormal, is 2^-133 in lo, bf16's own last bit).
+// inf and NaN go in hi alone.
 __device__ __forceinline__ void split_bf16x3(float v, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
     const uint32_t u = __float_as_uint(v);
     if ((u & 0x7f800000u) == 0x7f800000u) {
@@ -1769,9 +1778,9 @@ __device__ __forceinline__ void split_bf16x3(float v, uint32_t &hi, uint32_t &mi
         return;
     }
     hi = u & 0xffff0000u;
-    const float r = v - __uint_as_float(hi);
+    const float r = (v - __uint_as_float(hi)) * 256.0f;
     mid = __float_as_uint(r) & 0xffff0000u;
-    lo = __float_as_uint(r - __uint_as_float(mid));
+    lo = __float_as_uint((r - __uint_as_float(mid)) * 256.0f);
 }
 
 // Keeps every register of `sum` allocated until `after` has been computed.
@@ -1971,7 +1980,7 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
     // The scale of words w, with the operand of a non-finite one rewritten.
     auto finish_decode = [&](const uint32_t (&w)[5]) __attribute__((always_inline)) {
         const uint32_t bits = (upper ? w[4] : w[0]) & 0xffffu;
-        scale = half_bits_to_float(bits);
+        scale = half_bits_to_float(bits) * Op::kScale;
         if constexpr (sizeof(T) == 2) {
             const bool bad = (bits & 0x7c00u) == 0x7c00u;
             if (__builtin_expect((flags & kTritIeeeScales) && __any(bad), 0)) {
@@ -2019,12 +2028,16 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
                 for (int nb = 0; nb < NB; ++nb) b[p][nb] = frag(slot, p, nb, st);
             const u32x4 wt = {half.dword(4 * st), half.dword(4 * st + 1), half.dword(4 * st + 2), half.dword(4 * st + 3)};
 #pragma unroll
-            for (int p = P - 1; p >= 0; --p)
+            for (int p = P - 1; p >= 0; --p) {
+                u32x4 w_p = wt;
+                if constexpr (P == 3)  // the last terms weigh 2^-8 of the middle ones
+                    if (p == 2) w_p = wt & ~(Op::kLowerBit * 0x10001u);
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
                     float16v &into = p == 0 ? sum[nb] : low[nb];
-                    into = Op::mfma(b[p][nb], wt, into);
+                    into = Op::mfma(b[p][nb], w_p, into);
                 }
+            }
             if constexpr (kDecode) {
                 // window w's dwords end at 5w + 4: after the stage that reads it
                 if (st == 0) s = window_splits(u, 0);
@@ -2049,7 +2062,7 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
             for (int r = 0; r < RQ * 4; ++r)
-                acc[nb][r] = fmaf(scale, P == 1 ? sum[nb][r] : sum[nb][r] + low[nb][r], acc[nb][r]);
+                acc[nb][r] = fmaf(scale, P == 1 ? sum[nb][r] : fmaf(low[nb][r], 0x1p-8f, sum[nb][r]), acc[nb][r]);
         // All 16 sums stay live until the fmas above have waited for the last
         // MFMA: the compiler would reuse the registers of the unused ones at
         // once, and its hazard checks do not see the decode's inline asm

@@ -20,7 +20,8 @@ import torch
 from oracle import tq1_oracle as O
 from tests.gpu_util import layout, pack, random_blocks, to_dev
 from ternel_amd import _lib
-from ternel_amd.kernels import GemmConfig, tq1_gemm_words, tq1_linear_words, tq1_matmul_words, tq1_swiglu_words
+from ternel_amd.kernels import (GemmConfig, linear_kernel, tq1_gemm_words, tq1_linear_words, tq1_matmul_words,
+                                tq1_swiglu_words)
 
 pytestmark = pytest.mark.gpu
 
@@ -177,3 +178,24 @@ def test_group_counts_without_divisors_match_the_oracle(dtype, rows, groups, bat
     silu = (gate / (1.0 + torch.exp(-gate)) * up).to(dtype).float()
     finite = torch.isfinite(silu)
     assert bool(((z - silu).abs() <= silu.abs() * 4 * ROUNDOFF[dtype] + 2.0 ** -24)[finite].all())
+
+
+# fp32 activations down to the last bits of the subnormals and up to near the largest value (group sums
+# of random signs stay finite): the three bf16 terms hold every finite value exactly, so the bound is
+# the summation one, with the spacing of the subnormals once per rounding
+@pytest.mark.parametrize("exponent", (-148, -140, -130, -126, -120, -110, -60, 110))
+@pytest.mark.parametrize(("rows", "columns", "batch"), ((8192, 1152, 7), (4100, 4608, 16), (4100, 4608, 24)))
+def test_fp32_values_of_any_magnitude_match_the_oracle(rows, columns, batch, exponent) -> None:
+    print(f"trit: fp32 rows={rows} columns={columns} batch={batch} 2^{exponent}", flush=True)
+    lay = layout(rows, columns)
+    assert linear_kernel(lay, batch, torch.float32) == "trit"
+    blocks = random_blocks(rows, columns, seed=rows + batch)
+    rng = np.random.default_rng(1000 + batch - exponent)
+    x = to_dev((rng.normal(0.0, 1.0, size=(batch, columns)) * 2.0 ** exponent).astype(np.float32))
+    got = tq1_linear_words(pack(blocks), x, layout=lay)
+    sample = np.unique(np.r_[0:64, rows - 70:rows, rng.integers(0, rows, 200)])
+    x64 = x.double().cpu().numpy()
+    want = O.oracle_matmul(blocks[sample], x64, rows=len(sample), columns=columns)
+    weights = O.dense_weights(blocks[sample], rows=len(sample), columns=columns)
+    sums = (128 + columns // 128) * 2.0 ** -23 * (np.abs(x64) @ np.abs(weights).T) + (columns // 64) * 2.0 ** -149
+    assert (np.abs(got.double().cpu().numpy()[:, sample] - want) <= sums).all()
