@@ -1703,7 +1703,7 @@ __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (
 // (t - 1) * scale weights together and took only fp16 (bf16 ran the wide form
 // after a scaling pass, fp32 the LUT23 kernel): fp16 M=8 17.9 / 20.3 / 12.8 ->
 // 14.1 / 14.3 / 9.9, M=32 20.6 / 23.6 / 15.5 -> 18.1 / 21.3 / 13.3; bf16 M=8
-// 27.2 / 34.8 / 24.6 -> 14.1 / 14.3 / 9.9; fp32 QKV M=24 41.7 -> 20.7.
+// 27.2 / 34.8 / 24.6 -> 14.1 / 14.3 / 9.9; fp32 QKV M=24 41.7 -> 20.5.
 //
 // Weights never touch LDS: lane l of a wave decodes half l / 32 of the block
 // of weight row l % 32 straight into an operand of v_mfma_f32_32x32x16, in the
@@ -1929,11 +1929,17 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
     // Activations of the window at group w0 (rows past M and groups past the
     // chunk re-read the last), as physical 16-byte chunks; written to LDS in
     // the K order as 4-value units.
+    // fp32's widest tiles index their chunks anew for each window: kept across the
+    // loop, those addresses put 25 registers into scratch (QKV M=24 20.9 us
+    // against 20.5, two waves per SIMD 22.2).
+    constexpr bool kReindex = MULTI && P == 3 && SR == 32;
     uint4 xc[kChunks];
     auto load_x = [&](int w0) __attribute__((always_inline)) {
+        int t = tid;
+        if constexpr (kReindex) asm volatile("" : "+v"(t));
 #pragma unroll
         for (int k = 0; k < kChunks; ++k) {
-            const int j = tid + k * kDirectThreads;
+            const int j = t + k * kDirectThreads;
             const int r = j / kRowChunks, q = r / SR, m = r - q * SR;
             xc[k] = *reinterpret_cast<const uint4 *>(x + static_cast<int64_t>(min(m, M - 1)) * K +
                                                      static_cast<int64_t>(g_begin + min(w0 + q, cg - 1)) * kBlockWeights +
@@ -1942,9 +1948,11 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
     };
     auto target_unit = [](int u) { return u < 15 ? u : (u < 30 ? u + 1 : (u == 30 ? 15 : 31)); };
     auto store_x = [&]() __attribute__((always_inline)) {
+        int t = tid;
+        if constexpr (kReindex) asm volatile("" : "+v"(t));
 #pragma unroll
         for (int k = 0; k < kChunks; ++k) {
-            const int j = tid + k * kDirectThreads;
+            const int j = t + k * kDirectThreads;
             const int r = j / kRowChunks, c = j % kRowChunks;
             uint16_t *row = xs + r * kDirectStride;
             if constexpr (P == 1) {
@@ -2011,8 +2019,8 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
         // each of their additions would round at the sum's full magnitude.
         // Errors against fp64, one sum / two (the LUT23 kernel's): 5839 x 15872,
         // M=11 1.57e-7 / 1.14e-7 (1.52e-7), QKV M=24 1.23e-7 / 0.78e-7
-        // (1.26e-7); the registers cost QKV M=24 18.7 -> 20.7 us (41.7), M=14 of
-        // 20799 x 2176 21.0 -> 21.4 (44.3).
+        // (1.26e-7). The second sum and the last terms' own operand cost QKV
+        // M=24 18.7 -> 20.5 us (LUT23 41.7).
         float16v sum[NB], low[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
