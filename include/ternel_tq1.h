@@ -242,7 +242,9 @@ int ternel_tq1_matmul_noalloc(const uint32_t *packed, const void *x, void *y, in
  * k_split (size the workspace with form WIDE for either). With AUTO, up to 32
  * rows (64 for matrices under 24 MiB of packed weights, 128 on long rows, 512
  * under 12 MiB and 768 under 4 MiB) they run the DIRECT form's kernel on bf16
- * MFMAs, as they are; above, and for any batch with WIDE, the WIDE form after
+ * MFMAs, as they are (a block's sum of 128 activations stays within range
+ * wherever its product with the scale does; the running sum over blocks is
+ * fp32); above, and for any batch with WIDE, the WIDE form after
  * a pre-pass that scales each row by a power of two into fp16's range and converts it (exact:
  * bf16's 8-bit significand fits fp16's 11 bits; values more than 2^28 below
  * the row's largest lose bits), and the fp32 sums are scaled back and rounded

@@ -1740,13 +1740,15 @@ __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// kOne: the bits a trit of +1 has in the operand, 1 / kScale. In fp32 half of 1,
-// so that the middle terms below, kept at 2^8 times their value, sum to no more
-// than the values do; 2^-8 of it is kOne without kLowerBit.
+// kOne: the bits a trit of +1 has in the operand, 1 / kScale. In bf16 2^-8, so
+// that no sum of 128 finite values overflows where scale * sum does not (products
+// stay exact: the smallest is 2^-141). In fp32 half of 1, so that the middle
+// terms below, kept at 2^8 times their value, sum to no more than the values do;
+// 2^-8 of it is kOne without kLowerBit.
 template <typename T>
 struct TritOperand {  // bf16 and (as three bf16 terms) fp32
-    static constexpr uint32_t kOne = sizeof(T) == 4 ? 0x3f00u : 0x3f80u;
-    static constexpr float kScale = sizeof(T) == 4 ? 2.0f : 1.0f;
+    static constexpr uint32_t kOne = sizeof(T) == 4 ? 0x3f00u : 0x3b80u;
+    static constexpr float kScale = sizeof(T) == 4 ? 2.0f : 256.0f;
     static constexpr uint32_t kLowerBit = 0x0400u;
     static constexpr int kPlanes = sizeof(T) == 4 ? 3 : 1;
     static __device__ __forceinline__ float16v mfma(u32x4 a, u32x4 b, float16v c) {

@@ -165,6 +165,25 @@ def test_each_form_keeps_rows_beyond_fp16_range_and_non_finite_values(form, batc
 
 
 @pytest.mark.parametrize(("form", "batch"), FORMS)
+def test_each_form_stays_finite_near_the_largest_values(form, batch) -> None:
+    """Sums of a group's activations beyond fp32's range whose products with the
+    block scales are within it: 128 values of 2^124 and all trits +1."""
+    rows, columns = 300, 1024
+    rng = np.random.default_rng(batch)
+    trits = np.full((rows * 8, 128), 2, dtype=np.uint8)
+    trits[:, 40:] = rng.integers(0, 3, size=(rows * 8, 88), dtype=np.uint8)
+    scales = (2.0 ** -9 * rng.choice((-1.0, 1.0), size=(rows * 8, 1))).astype(np.float16).view(np.uint8)
+    blocks = O.encode_tq1_blocks(scales, trits).reshape(rows, 8, 28)
+    x = rng.uniform(1.0, 2.0, size=(batch, columns)) * 2.0 ** 124
+    xb = to_dev(x.astype(np.float32)).to(torch.bfloat16)
+    got = tq1_gemm_words(pack(blocks), xb, layout=layout(rows, columns), config=GemmConfig(form=form)).float().cpu().numpy()
+    want = O.oracle_matmul(blocks, bf16_host(xb), rows=rows, columns=columns)
+    assert np.isfinite(want.astype(np.float32)).all() and (np.abs(want) < 2.0 ** 127).all()
+    assert np.isfinite(got).all()
+    assert O.compare(got, want)["normalised_max_abs_error"] < BF16_TOLERANCE
+
+
+@pytest.mark.parametrize(("form", "batch"), FORMS)
 def test_each_form_is_exact_on_integers(form, batch) -> None:
     rows, columns = 300, 1024
     rng = np.random.default_rng(batch)
