@@ -175,29 +175,39 @@ def packed_shape(layout: PackedTensorLayout) -> tuple[int, int, int, int]:
     return tuple(_packed_shape(layout.rows, layout.columns))
 
 
-# What the library answers for sizes alone, per device (the kernels are chosen
-# by its CU count).
-@functools.lru_cache(maxsize=4096)
-def _matmul_bytes(index: int, batch: int, rows: int, columns: int, batch_tile: int, k_split: int) -> int:
-    return _lib.lib().ternel_tq1_matmul_workspace_bytes(batch, rows, columns, batch_tile, k_split)
+# What the library answers for sizes alone. It chooses kernels by the CU count of
+# the current device, which need not be the one the tensors are on, so that is
+# part of the key.
+_plan_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 @functools.lru_cache(maxsize=4096)
-def _gemm_bytes(index: int, batch: int, rows: int, columns: int, form: int, k_split: int) -> int:
-    return _lib.lib().ternel_tq1_gemm_workspace_bytes(batch, rows, columns, form, k_split)
+def _answer(device: int, name: str, *sizes: int) -> int:
+    return getattr(_lib.lib(), name)(*sizes)
+
+
+def _matmul_bytes(batch: int, rows: int, columns: int, batch_tile: int, k_split: int) -> int:
+    return _answer(_plan_device(), "ternel_tq1_matmul_workspace_bytes", batch, rows, columns, batch_tile, k_split)
+
+
+def _gemm_bytes(batch: int, rows: int, columns: int, form: int, k_split: int) -> int:
+    return _answer(_plan_device(), "ternel_tq1_gemm_workspace_bytes", batch, rows, columns, form, k_split)
 
 
 @functools.lru_cache(maxsize=4096)
-def _linear_plan(index: int, batch: int, rows: int, columns: int, code: int) -> tuple[int, int]:
-    """(ternel_tq1_linear_kernel, workspace bytes) of a linear."""
+def _linear_answers(device: int, batch: int, rows: int, columns: int, code: int) -> tuple[bool, int]:
     handle = _lib.lib()
-    return (handle.ternel_tq1_linear_kernel(batch, rows, columns, code),
+    return (handle.ternel_tq1_linear_kernel(batch, rows, columns, code) == KERNEL_LUT23,
             handle.ternel_tq1_linear_workspace_bytes(batch, rows, columns, code))
 
 
-@functools.lru_cache(maxsize=4096)
-def _swiglu_bytes(index: int, batch: int, rows: int, columns: int, code: int) -> int:
-    return _lib.lib().ternel_tq1_swiglu_workspace_bytes(batch, rows, columns, code)
+def _linear_plan(batch: int, rows: int, columns: int, code: int) -> tuple[bool, int]:
+    """(whether a linear takes the matmul path, its workspace bytes)"""
+    return _linear_answers(_plan_device(), batch, rows, columns, code)
+
+
+def _swiglu_bytes(batch: int, rows: int, columns: int, code: int) -> int:
+    return _answer(_plan_device(), "ternel_tq1_swiglu_workspace_bytes", batch, rows, columns, code)
 
 
 def pack_weights(blocks, *, layout: PackedTensorLayout, validate: bool = False) -> torch.Tensor:
@@ -431,8 +441,7 @@ def tq1_matmul_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTen
     x = x.contiguous()
     out = x.new_empty((batch, layout.rows))
     index = x.get_device()
-    ws = workspace(x.device, _matmul_bytes(index, batch, layout.rows, layout.columns, config.batch_tile,
-                                           config.k_split))
+    ws = workspace(x.device, _matmul_bytes(batch, layout.rows, layout.columns, config.batch_tile, config.k_split))
     _lib.check(_lib.lib().ternel_tq1_matmul(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns,
         _DTYPE_CODE[x.dtype], config.batch_tile, config.k_split,
@@ -474,19 +483,12 @@ def tq1_gemm_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTenso
     _surface(index)
     out = x.new_empty((batch, layout.rows))
     sized = GEMM_FORMS["wide"] if x.dtype == torch.bfloat16 else form
-    ws = workspace(x.device, _gemm_bytes(index, batch, layout.rows, layout.columns, sized, config.k_split))
+    ws = workspace(x.device, _gemm_bytes(batch, layout.rows, layout.columns, sized, config.k_split))
     _lib.check(_lib.lib().ternel_tq1_gemm(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns,
         _DTYPE_CODE[x.dtype], form, config.k_split, ws.data_ptr() if ws is not None else None,
         ws.numel() if ws is not None else 0, _raw_stream(index)))
     return out
-
-
-def tq1_linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout) -> torch.Tensor:
-    """The library's own dispatch (``ternel_tq1_linear``) for a 2-D ``x``."""
-    check_packed(packed, layout=layout)
-    check_activations(x, layout=layout)
-    return _linear(packed, _aligned_rows(x), layout)
 
 
 def linear_kernel(layout: PackedTensorLayout, batch: int, dtype: torch.dtype) -> str:
@@ -496,6 +498,14 @@ def linear_kernel(layout: PackedTensorLayout, batch: int, dtype: torch.dtype) ->
     if code < 0:
         raise FormatError(_lib.last_error())
     return KERNEL_NAMES[code]
+
+
+def tq1_linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout) -> torch.Tensor:
+    """The library's own dispatch (``ternel_tq1_linear``) for a 2-D ``x``."""
+    check_packed(packed, layout=layout)
+    batch = check_activations(x, layout=layout)
+    need = _linear_plan(batch, layout.rows, layout.columns, _DTYPE_CODE[x.dtype])[1]
+    return _linear(packed, _aligned_rows(x), layout, need)
 
 
 def linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout) -> torch.Tensor:
@@ -509,16 +519,16 @@ def linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorL
         raise FormatError("activations have an empty batch dimension")
     check_packed(packed, layout=layout)
     check_activations(flat, layout=layout)
-    lut = _linear_plan(flat.get_device(), flat.shape[0], layout.rows, layout.columns, code)[0] == KERNEL_LUT23
-    out = _linear(packed, flat.contiguous() if lut else _aligned_rows(flat), layout)
+    lut, need = _linear_plan(flat.shape[0], layout.rows, layout.columns, code)
+    out = _linear(packed, flat.contiguous() if lut else _aligned_rows(flat), layout, need)
     return out if x.ndim == 2 else out.reshape(*x.shape[:-1], layout.rows)
 
 
-def _linear(packed: torch.Tensor, x: torch.Tensor, layout: PackedTensorLayout) -> torch.Tensor:
+def _linear(packed: torch.Tensor, x: torch.Tensor, layout: PackedTensorLayout, need: int) -> torch.Tensor:
     batch, code, index = x.shape[0], _DTYPE_CODE[x.dtype], x.get_device()
     _surface(index)
     out = x.new_empty((batch, layout.rows))
-    ws = workspace(x.device, _linear_plan(index, batch, layout.rows, layout.columns, code)[1])
+    ws = workspace(x.device, need)
     _lib.check(_lib.lib().ternel_tq1_linear(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns, code,
         ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _raw_stream(index)))
@@ -540,7 +550,7 @@ def tq1_swiglu_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTen
     _surface(index)
     out = x.new_empty((batch, layout.rows // 2))
     code = _DTYPE_CODE[x.dtype]
-    ws = workspace(x.device, _swiglu_bytes(index, batch, layout.rows, layout.columns, code))
+    ws = workspace(x.device, _swiglu_bytes(batch, layout.rows, layout.columns, code))
     _lib.check(_lib.lib().ternel_tq1_swiglu(
         packed.data_ptr(), x.data_ptr(), out.data_ptr(), batch, layout.rows, layout.columns, code,
         ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _raw_stream(index)))

@@ -94,3 +94,31 @@ def test_a_report_is_kept_while_a_stream_captures(host) -> None:
     host.capturing = False
     with pytest.raises(_lib.NativeError):
         kernels._surface(0)
+
+
+def test_sizes_are_kept_per_device_that_plans_the_launch(monkeypatch) -> None:
+    """The library plans on the current device: an answer given there is not
+    used for a call made while another one is current."""
+
+    class Library:
+        def __getattr__(self, name):
+            return lambda *sizes: 1000 * device + len(sizes)
+
+    device = 0
+    monkeypatch.setattr(_lib, "lib", lambda: Library())
+    monkeypatch.setattr(kernels, "_plan_device", lambda: device)
+    caches = (kernels._answer, kernels._linear_answers)
+    for cache in caches:
+        cache.cache_clear()
+    try:
+        calls = (lambda: kernels._matmul_bytes(2, 64, 128, 0, 0), lambda: kernels._gemm_bytes(2, 64, 128, 0, 0),
+                 lambda: kernels._linear_plan(2, 64, 128, 0)[1],
+                 lambda: kernels._swiglu_bytes(2, 64, 128, 0))
+        first = [call() for call in calls]
+        device = 1
+        assert [call() for call in calls] == [1000 + value for value in first]
+        device = 0
+        assert [call() for call in calls] == first
+    finally:
+        for cache in caches:
+            cache.cache_clear()
