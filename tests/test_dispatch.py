@@ -177,3 +177,26 @@ def test_a_given_split_moves_no_batch_to_the_direct_form() -> None:
         assert size(M, rows, columns, 0, 4) == size(M, rows, columns, 1, 4)
     for k_split in (0, 1, 4):
         assert size(48, rows, columns, 0, k_split) == size(48, rows, columns, 2, k_split)
+
+
+KERNEL_SWEEP = json.loads((GOLDEN / "kernel_sweep_mi355x.json").read_text())
+# Where another kernel was more than 15 % faster: the tile form splits K only by divisors of the group
+# count (67 and 74 here), as does the LUT23 kernel's automatic choice in chunks of 1 or 2 groups.
+SLOWER = {(4096, 8576, 100), (4096, 8576, 203), (4096, 8576, 384), (2048, 9472, 203), (2048, 9472, 384), (2048, 9472, 768),
+          (1024, 16768, 1), (2048, 9472, 2)}
+
+
+@pytest.mark.parametrize("row", KERNEL_SWEEP["rows"], ids=lambda r: f"{r['N']}x{r['K']}-{r['dtype']}-M{r['M']}")
+def test_the_dispatch_runs_the_kernel_of_the_sweep(row) -> None:
+    """The kernel that was timed is the one that runs, within 15 % of any other."""
+    layout = PackedTensorLayout.for_tensor(row["N"], row["K"])
+    assert linear_kernel(layout, row["M"], getattr(torch, row["dtype"])) == row["runs"]
+    others = [us for name, us in row["us"].items() if name != "dispatch"]
+    if (row["N"], row["K"], row["M"]) not in SLOWER or row["dtype"] != "float16":
+        assert row["us"]["dispatch"] <= 1.15 * min(others, default=row["us"]["dispatch"]), row["us"]
+
+
+def test_the_kernel_sweep_covers_every_kernel_of_every_type() -> None:
+    runs = {(row["dtype"], row["runs"]) for row in KERNEL_SWEEP["rows"]}
+    assert runs == {(t, k) for t in ("float16", "bfloat16") for k in ("strip", "lut23", "trit", "wide")} | \
+        {("float16", "tile")} | {("float32", k) for k in ("strip", "lut23", "trit")}
