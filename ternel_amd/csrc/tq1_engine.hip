@@ -16,8 +16,13 @@
 //   validate_kernel    fail-closed byte scan of canonical blocks
 //   decode_kernel      bit-exact trit decode of canonical blocks (test entry)
 //   interleave_kernel / deinterleave_kernel   canonical <-> packed
-//   lut_gemv_kernel    LUT23 product, M = 1 decode GEMV and small batches,
-//                      with a fused, ordered split-K fix-up
+//   lut_gemv_kernel    LUT23 product, M = 1 and small batches, with a fused,
+//                      ordered split-K fix-up
+//   strip_gemv_kernel  the same product at M = 1 as one strip of rows per CU
+//   trit_gemm_kernel   trits as MFMA operands: small batches of every type, and
+//                      larger ones on small matrices in tiles of up to 64 rows
+//   wide_gemm_kernel   256-row tiles, weights decoded into operand registers,
+//                      stream-K over the CUs: larger batches and prefill
 //   mfma_gemm_kernel   trits -> fp16 LDS tiles -> v_mfma_f32_32x32x16_f16
 //   get_rows_kernel    packed embedding-row gather
 
@@ -3817,7 +3822,11 @@ int launch_wide_nb(const uint32_t *packed, const _Float16 *xp, void *y, float *p
                    const float *row_inv, const WidePlan &plan, const WideGeometry &geo, hipStream_t stream) {
     const int wgs = plan.workgroups;
     switch (plan.nb) {
-        case 1: return launch_wide_kernel<1, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
+        case 1:  // (no SwiGLU: the trit kernel takes those batches)
+            if constexpr (GLU)
+                return fail(TERNEL_TQ1_EINVAL, "the wide form's SwiGLU takes more than 32 activation rows");
+            else
+                return launch_wide_kernel<1, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
         case 2: return launch_wide_kernel<2, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
         case 4: return launch_wide_kernel<4, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
         default: return launch_wide_kernel<8, BF, GLU>(packed, xp, y, partial, counters, row_inv, geo, wgs, stream);
@@ -3857,19 +3866,19 @@ int launch_wide(const uint32_t *packed, const void *x, void *y, const WidePlan &
                : launch_wide_nb<false, false>(packed, xp, y, partial, counters, nullptr, plan, geo, stream);
 }
 
-// Automatic choice, from a sweep of every form over the 27B linears on MI355X
-// (the fixture tests/golden/dispatch_sweep_mi355x.json replays it): the direct
-// form up to 32 activation rows (gate/up, down M=24-32: 19.9-23.6 us against
-// the wide form's 24.1-28.0; QKV, O 15.0-16.3 against 20.8-21.5), and up to
-// 48 for matrices under 16 MiB of packed weights (QKV M=40-48: 22.2-23.0
-// against 24.3-24.5; O 25.2-27.0 against 27.0-27.3); the wide form otherwise
-// up to 64 rows (gate/up, down M=40-64: 28.9-33.6 against the two-tile direct
-// form's 31.2-37.5; QKV and O at M=64 within 5 %); above, the wide form when
+// Automatic choice, from a sweep of every form on MI355X (the fixture
+// tests/golden/kernel_sweep_mi355x.json replays it; fp16, us): the direct form
+// up to 32 activation rows (gate/up, down M=24-32: 16.6-20.4 against the wide
+// form's 24.7-28.3; QKV, out_proj 12.0-13.0 against 20.0-21.2), and up to 64
+// for matrices under 16 MiB of packed weights (QKV M=48-64 19.1 against 24.5,
+// out_proj 16.7 against 24.6-25.0); the wide form otherwise up to 64 rows
+// (gate/up M=48-64 29.0-29.5 against the direct form's 29.6-30.1; down 33.4-34.0
+// against 30.2-30.6 the other way); above, the wide form when
 // stream-K has enough tiles or enough work per CU to amortise its reduction --
 // at least CUs/4 tiles (a tile's partials come from at most ~4 contributors)
 // or 15 (tile, group) steps per CU -- and the fixed-split tile form otherwise
-// (QKV 5120->8192 M=128: 31.6 us against 38.8; gate/up 5120->17408 M=128: 44.6
-// against 58.1 the other way). The tile form also serves a fixed K split above
+// (down M=100 49.1 against 53.1; gate/up M=100 42.7 against 56.1 the other
+// way). The tile form also serves a fixed K split above
 // 32 rows and rows too long for the wide form's 32-bit buffer offsets.
 constexpr int64_t kAutoDirectMaxBatch = 32;
 constexpr int64_t kAutoDirectMaxBatchSmall = 64;
@@ -3899,18 +3908,16 @@ int resolve_gemm_form(int64_t M, int64_t rows, int64_t columns, int form, int k_
     return 4 * tiles >= cus || tiles * groups >= min_steps * cus ? TERNEL_TQ1_GEMM_WIDE : TERNEL_TQ1_GEMM_TILE;
 }
 
-// The dispatch rule of packed_matmul, retuned for MI355X by the same sweep: the
-// LUT23 kernel up to 3 activation rows -- 4 for matrices under 16 MiB of
-// packed weights, where the MFMA forms' fixed costs weigh more (O 8192->5120
-// M=4: 11.5 us against the direct form's 13.1, M=5 13.7 against 13.0; gate/up
-// M=4: the direct form 16.2 us against 18.9) -- the MFMA kernels above it
-// (fp16 only).
+// The dispatch rule of packed_matmul: the matmul path for fp32 (the GEMM forms
+// take 16-bit activations) and up to 3 activation rows, 4 for matrices under
+// 16 MiB of packed weights; the GEMM path above. Either may run the trit kernel
+// (matmul_uses_trit, gemm_uses_trit), so the line no longer decides between
+// kernels: it was drawn between the LUT23 kernel and the direct form before it
+// (O 8192->5120 M=4 11.5 us / 13.1), and now is where the arithmetic of a
+// non-finite scale changes (scale * sum below, (t - 1) * scale above).
 constexpr int64_t kLinearLutMaxBatch = 3;
 constexpr int64_t kLinearLutMaxBatchSmall = 4;
 constexpr int64_t kLinearSmallMatrixBytes = 16ll << 20;
-// bf16 activations above the same batch run the wide form (scale_rows_kernel
-// then wide_gemm_kernel<NB, true>); fp32 ones always run the LUT23 kernel:
-// their 24-bit significands do not fit the matrix cores' fp16 operands.
 bool linear_uses_lut(int64_t M, int64_t rows, int64_t columns, int dtype) {
     if (dtype == TERNEL_TQ1_F32) return true;
     const int64_t bytes = rows * (columns / kBlockWeights) * kBlockBytes;

@@ -428,7 +428,9 @@ def check_workspaces() -> None:
 
 def tq1_matmul_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout,
                      config: MatmulConfig | None = None) -> torch.Tensor:
-    """``x @ W.T`` through the LUT23 kernel; ``(batch, rows)`` in ``x.dtype``.
+    """``x @ W.T`` on the matmul path: the LUT23 kernel, or with ``config`` left
+    automatic the strip form (one vector) or the trit kernel where they are
+    faster; ``(batch, rows)`` in ``x.dtype``.
     A ``k_split`` that does not divide the group count is refused, as the
     reference refuses it (src/ternel_mlx/kernels.py:1240-1246)."""
     config = config or MatmulConfig()
@@ -509,8 +511,8 @@ def tq1_linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTen
 
 
 def linear_words(packed: torch.Tensor, x: torch.Tensor, *, layout: PackedTensorLayout) -> torch.Tensor:
-    """The same for ``x`` with any leading dimensions, which the result keeps:
-    the modules' product (src/ternel_mlx/modules.py:425-457)."""
+    """The library's own dispatch for ``x`` with any leading dimensions, which the
+    result keeps: the modules' product (src/ternel_mlx/modules.py:425-457)."""
     if x.shape[-1] != layout.columns:
         raise FormatError(f"activation has {x.shape[-1]} columns, weight expects {layout.columns}")
     flat = x if x.ndim == 2 else x.reshape(-1, layout.columns)

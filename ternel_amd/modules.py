@@ -43,13 +43,15 @@ from .kernels import (
 )
 from .layout import PackedTensorLayout, interleave_gate_up, unpack_blocks
 
-# Dispatch (src/ternel_mlx/modules.py:331-422, re-measured for MI355X): the
-# LUT23 kernels for small batches, the MFMA kernels above them. The LUT kernel's
-# cost grows linearly with the batch (one table set per vector) while its bytes
-# do not, so it only pays while the weight stream dominates. The rule lives in
-# the library (ternel_tq1_linear_kernel, replayed against a measured sweep in
-# tests/test_dispatch.py); LUT23_MAX_BATCH is its bound for matrices of 16 MiB
-# of packed weights or more, the 27B MLP shapes (smaller matrices: 4 rows).
+# Dispatch (src/ternel_mlx/modules.py:331-422, re-measured for MI355X). The rule
+# lives in the library: ternel_tq1_linear_kernel names the entry point a batch
+# takes (the matmul path for fp32 and the smallest batches, a GEMM form above),
+# ternel_tq1_linear_launches the kernel that runs there -- the strip form or the
+# LUT23 kernel, whose cost grows with every vector while its bytes do not, the
+# trit kernel from a few rows on and for larger batches of small matrices, the
+# wide and tile forms for prefill. tests/test_dispatch.py replays both against
+# measured sweeps. LUT23_MAX_BATCH is the matmul path's bound for matrices of
+# 16 MiB of packed weights or more, the 27B MLP shapes (smaller ones: 4 rows).
 LUT23_MAX_BATCH = 3
 _KERNEL_NAMES = {100: "lut23", 1: "gemm", 2: "gemm", 3: "gemm"}
 
