@@ -14,7 +14,8 @@ import torch
 
 from oracle import tq1_oracle as O
 from ternel_amd import synthetic
-from ternel_amd.kernels import GemmConfig, MatmulConfig, pack_weights, tq1_gemm_words, tq1_get_rows_words, tq1_matmul_words
+from ternel_amd.kernels import (GemmConfig, MatmulConfig, linear_kernel, pack_weights, tq1_gemm_words,
+                                tq1_get_rows_words, tq1_linear_words, tq1_matmul_words)
 from ternel_amd.layout import PackedTensorLayout
 
 pytestmark = pytest.mark.gpu
@@ -75,6 +76,23 @@ def test_small_batch_paths_agree_at_the_gate_shape(M: int) -> None:
     assert O.compare(lut[:, rows], want)["normalised_max_abs_error"] < 1e-3
     assert O.compare(mfma[:, rows], want)["normalised_max_abs_error"] < 1e-3
     assert O.compare(mfma, lut)["normalised_max_abs_error"] < 2e-3
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("M", (2, 8, 16, 24))
+def test_the_lut23_and_the_trit_kernel_agree_at_the_gate_shape(M: int, dtype) -> None:
+    """Two kernels (the LUT23 one by a batch tile given): fp32 sums in other
+    orders, so within the sum of their bounds, and one rounding each."""
+    K, N = 5120, 17408
+    lay = PackedTensorLayout.for_tensor(N, K)
+    assert linear_kernel(lay, M, dtype) == ("lut23" if dtype == torch.float32 and M == 2 else "trit")
+    blocks = synthetic.device_blocks(N, K, seed=synthetic.SEED_BASE + 2)
+    x = synthetic.device_activations(M, K, seed=M).to(dtype)
+    packed = pack_weights(blocks, layout=lay)
+    lut = tq1_matmul_words(packed, x, layout=lay, config=MatmulConfig(batch_tile=1)).float().cpu().numpy()
+    got = tq1_linear_words(packed, x, layout=lay).float().cpu().numpy()
+    tolerance = {torch.float16: 2e-3, torch.bfloat16: 2e-2, torch.float32: 1e-5}[dtype]
+    assert O.compare(got, lut)["normalised_max_abs_error"] < tolerance
 
 
 def test_embedding_gather_from_the_config4_table() -> None:

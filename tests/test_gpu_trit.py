@@ -4,7 +4,7 @@ the SwiGLU epilogues of the MFMA kernels against the linear they follow.
 Shapes sit where it can go wrong: row counts that are no multiple of a wave's
 32 or a workgroup's 128 rows, group counts below, at and past its windows (1,
 5, 9 and 17 groups unsplit, 40 split), batches on both sides of its 8-, 16-, 32-
-and 64-row tiles, a batch of several launches. Products of an activation with
+and 64-row tiles, several tiles in a launch and in several launches. Products of an activation with
 -1, 0 or +1 are exact (fp32 as three bf16 terms), so an output is held to the
 fp32 summation bound plus one rounding to its type.
 """
@@ -19,9 +19,9 @@ import torch
 
 from oracle import tq1_oracle as O
 from tests.gpu_util import layout, pack, random_blocks, to_dev
-from ternel_amd import _lib
-from ternel_amd.kernels import (GemmConfig, linear_kernel, tq1_gemm_words, tq1_linear_words, tq1_matmul_words,
-                                tq1_swiglu_words)
+from ternel_amd import _lib, synthetic
+from ternel_amd.kernels import (GemmConfig, linear_kernel, pack_weights, tq1_gemm_words, tq1_linear_words,
+                                tq1_matmul_words, tq1_swiglu_words)
 
 pytestmark = pytest.mark.gpu
 
@@ -49,7 +49,7 @@ CASES = [(dtype, rows, columns, batch) for dtype in (torch.float16, torch.bfloat
 # tiles of 64 rows and the remainder of a batch past them, split and unsplit
 CASES += [(dtype, rows, columns, batch) for dtype in (torch.float16, torch.bfloat16)
           for rows, columns, batch in ((257, 1152, 65), (1024, 5120, 130), (300, 640, 203), (4100, 1024, 193))]
-# fp32: matrices large enough for the trit kernel at each tile width, and batches of several launches
+# fp32: matrices large enough for the trit kernel at each tile width, and (LUT23) small ones
 CASES += [(torch.float32, 5121, 4608, 8), (torch.float32, 2562, 4608, 15), (torch.float32, 300, 640, 77),
           (torch.float32, 257, 1152, 130), (torch.float32, 130, 128, 65)]
 
@@ -199,3 +199,50 @@ def test_fp32_values_of_any_magnitude_match_the_oracle(rows, columns, batch, exp
     weights = O.dense_weights(blocks[sample], rows=len(sample), columns=columns)
     sums = (128 + columns // 128) * 2.0 ** -23 * (np.abs(x64) @ np.abs(weights).T) + (columns // 64) * 2.0 ** -149
     assert (np.abs(got.double().cpu().numpy()[:, sample] - want) <= sums).all()
+
+
+@pytest.mark.parametrize("batch", (64, 63))
+def test_a_batch_of_several_launches(batch) -> None:
+    """fp32 on down's shape: 17 K chunks whose partials leave room for one batch
+    tile of 32 rows within the matmul path's limit, so two launches share the
+    counters, the second one short; linear and SwiGLU."""
+    rows, columns = 5120, 17408
+    lay = layout(rows, columns)
+    assert linear_kernel(lay, batch, torch.float32) == "trit"
+    # one tile's partials, rather than two: 17 chunks of 40 row blocks x 4 waves x 4 quads
+    need = _lib.lib().ternel_tq1_matmul_workspace_bytes(batch, rows, columns, 0, 0)
+    tile = 17 * 40 * 4 * 4 * 1024
+    assert tile <= (16 << 20) < 2 * tile and need >= 65536 + tile
+    blocks = synthetic.device_blocks(rows, columns, seed=synthetic.SEED_BASE + 5)
+    packed = pack_weights(blocks, layout=lay)
+    x = synthetic.device_activations(batch, columns, seed=batch).to(torch.float32) * 0.05
+    got = tq1_linear_words(packed, x, layout=lay)
+    assert torch.equal(got, tq1_linear_words(packed, x, layout=lay))
+    sample = np.sort(np.random.default_rng(batch).choice(rows // 2, size=64, replace=False))
+    pairs = np.stack([2 * sample, 2 * sample + 1], axis=1).reshape(-1)
+    sampled = blocks[torch.from_numpy(pairs).cuda()].cpu().numpy()
+    x64 = x.double().cpu().numpy()
+    want = O.oracle_matmul(sampled, x64, rows=len(pairs), columns=columns)
+    assert (np.abs(got.double().cpu().numpy()[:, pairs] - want) <= bound(x64, sampled, want, torch.float32)).all()
+    gate, up = got[:, 0::2], got[:, 1::2]
+    silu = gate / (1.0 + torch.exp(-gate)) * up
+    diff = (tq1_swiglu_words(packed, x, layout=lay) - silu).abs()
+    assert bool((diff <= silu.abs() * 4 * ROUNDOFF[torch.float32] + 2.0 ** -126).all())
+
+
+def test_fp32_non_finite_values_follow_the_lut23_oracle() -> None:
+    """As above for fp32, on a matrix large enough for the trit kernel, at 16
+    and 24 rows a tile."""
+    rows, columns = 4096, 1152
+    for batch in (16, 72):
+        lay = layout(rows, columns)
+        assert linear_kernel(lay, batch, torch.float32) == "trit"
+        blocks = random_blocks(rows, columns, seed=3)
+        for row, value in {5: 0x7C00, 70: 0xFC00, 300: 0x7E00, rows - 1: 0x7C00}.items():
+            blocks[row, 1, 0:2] = np.frombuffer(np.uint16(value).tobytes(), dtype=np.uint8)
+        x = to_dev(np.random.default_rng(4).normal(0.0, 1.0, size=(batch, columns)).astype(np.float32))
+        x[1, 7], x[2, 639], x[batch - 1, 1151] = float("inf"), float("nan"), -float("inf")
+        sample = np.r_[0:96, 280:320, rows - 40:rows]
+        tables = O.lut23_matmul(blocks[sample], x.cpu().numpy(), rows=len(sample), columns=columns)
+        got = tq1_linear_words(pack(blocks), x, layout=lay).cpu().numpy()[:, sample]
+        assert O.compare(got, tables)["pattern_mismatches"] == 0

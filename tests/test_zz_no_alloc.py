@@ -52,13 +52,15 @@ def weight(rows: int, columns: int, seed: int):
 
 
 # (rows, columns, M, dtype, batch_tile, k_split): the first call of each pair
-# is the larger. 64 gate/up vectors need 44.6 MB of partials, so the
-# workspace-free call runs them as three launches of at most 24 vectors, where
-# the workspace call runs two (its counter region holds 60).
+# is the larger. 64 gate/up vectors run the trit kernel in one launch (as three
+# LUT23 launches of at most 24 vectors with a batch tile given, below); the
+# fp32 batches run it in several launches, whose partials do not fit at once.
 CALL_PAIRS = (
     ((17408, 5120, 64, torch.float16, 0, 0), (4096, 4096, 1, torch.float16, 0, 0)),
     ((5120, 17408, 6, torch.bfloat16, 2, 0), (5120, 8192, 2, torch.bfloat16, 1, 8)),
     ((8192, 5120, 4, torch.float32, 4, 10), (640, 1024, 3, torch.float32, 1, 2)),
+    ((17408, 5120, 64, torch.float16, 1, 0), (4096, 4096, 3, torch.float16, 1, 0)),
+    ((5120, 17408, 64, torch.float32, 0, 0), (5120, 17408, 63, torch.float32, 0, 0)),
     # one vector over 136 and then 64 groups: the strip GEMV in four, then
     # two, K chunks, met in the scratch's counter region
     ((5120, 17408, 1, torch.float16, 0, 0), (5120, 8192, 1, torch.float16, 0, 0)),
