@@ -1708,7 +1708,7 @@ __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (
 // (t - 1) * scale weights together and took only fp16 (bf16 ran the wide form
 // after a scaling pass, fp32 the LUT23 kernel): fp16 M=8 17.9 / 20.3 / 12.8 ->
 // 14.1 / 14.3 / 9.9, M=32 20.6 / 23.6 / 15.5 -> 18.1 / 21.3 / 13.3; bf16 M=8
-// 27.2 / 34.8 / 24.6 -> 14.1 / 14.3 / 9.9; fp32 QKV M=24 41.7 -> 20.5.
+// 27.2 / 34.8 / 24.6 -> 14.1 / 14.3 / 9.9; fp32 QKV M=24 41.7 -> 19.7.
 //
 // Weights never touch LDS: lane l of a wave decodes half l / 32 of the block
 // of weight row l % 32 straight into an operand of v_mfma_f32_32x32x16, in the
@@ -1778,14 +1778,10 @@ struct TritOperand<_Float16> {
 // 2^-149, the last bit of a subnormal, is 2^-133 in lo, bf16's own last bit).
 // inf and NaN go in hi alone.
 __device__ __forceinline__ void split_bf16x3(float v, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
-    const uint32_t u = __float_as_uint(v);
-    if ((u & 0x7f800000u) == 0x7f800000u) {
-        hi = (u & 0x007fffffu) ? u | 0x00400000u : u;
-        mid = lo = 0u;
-        return;
-    }
-    hi = u & 0xffff0000u;
-    const float r = (v - __uint_as_float(hi)) * 256.0f;
+    v = __builtin_canonicalizef(v);  // (a NaN's quiet bit is one of hi's)
+    hi = __float_as_uint(v) & 0xffff0000u;
+    float r = (v - __uint_as_float(hi)) * 256.0f;
+    r = r == r ? r : 0.0f;  // inf - inf, NaN
     mid = __float_as_uint(r) & 0xffff0000u;
     lo = __float_as_uint((r - __uint_as_float(mid)) * 256.0f);
 }
@@ -2027,7 +2023,7 @@ __global__ __launch_bounds__(kDirectThreads, SR > 32 ? 2 : 3) void trit_gemm_ker
         // Errors against fp64, one sum / two (the LUT23 kernel's): 5839 x 15872,
         // M=11 1.57e-7 / 1.14e-7 (1.52e-7), QKV M=24 1.23e-7 / 0.78e-7
         // (1.26e-7). The second sum and the last terms' own operand cost QKV
-        // M=24 18.7 -> 20.5 us (LUT23 41.7).
+        // M=24 18.7 -> 19.7 us (LUT23 41.7).
         float16v sum[NB], low[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
