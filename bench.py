@@ -255,10 +255,9 @@ def main() -> int:
     import torch
 
     from ternel_amd import _lib, synthetic
-    from ternel_amd.kernels import (GemmConfig, MatmulConfig, pack_weights, tq1_gemm_words, tq1_get_rows_words, tq1_linear_words,
+    from ternel_amd.kernels import (GemmConfig, MatmulConfig, linear_kernel, pack_weights, tq1_gemm_words, tq1_get_rows_words, tq1_linear_words,
                                     tq1_matmul_words, tq1_swiglu_words)
     from ternel_amd.layout import PackedTensorLayout
-    from ternel_amd.modules import select_kernel
 
     dev = torch.device("cuda", 0)
     torch.cuda.set_device(dev)
@@ -400,7 +399,7 @@ def main() -> int:
     c0_x = synthetic.device_activations(1, C0_K, seed=synthetic.SEED_BASE)
     config0 = {"workload": "BASELINE configs[0]: M=1, K=N=4096, fp16 activations, LUT23 GEMV "
                            "(the automatic configuration: the strip form)",
-               "packed_bytes": c0_bytes, "kernel": select_kernel(c0_layout, 1, torch.float16),
+               "packed_bytes": c0_bytes, "kernel": linear_kernel(c0_layout, 1, torch.float16),
                "form": m1_form(_lib.lib(), C0_N, C0_K)}
     for label, copies in (("cold", c0_ring), ("warm", 1)):
         launches = max(c0_ring, 200)
@@ -428,7 +427,7 @@ def main() -> int:
                 row[name] = {"us": round(ms * 1e3, 2),
                              "GB/s": round(packed_bytes(K, N) / (ms * 1e-3) / 1e9, 1),
                              "TFLOP/s": round(2 * M * K * N / (ms * 1e-3) / 1e12, 2),
-                             "kernel": select_kernel(layouts[i], M, torch.float16)}
+                             "kernel": linear_kernel(layouts[i], M, torch.float16)}
             small_batch[f"M={M}"] = row
             del xm
     traffic = measured_traffic()
@@ -592,9 +591,10 @@ def phase_profile(torch, dev, synthetic, pack_weights, tq1_matmul_words, tq1_lin
                 "p95_us": round(values[int(0.95 * (len(values) - 1))], 2), "max_us": round(values[-1], 2)}
 
     for i, (name, K, N) in enumerate(C1_SHAPES):
-        wide = batch > 1 and handle.ternel_tq1_linear_kernel(batch, N, K, 0) == 3  # TERNEL_TQ1_GEMM_WIDE
+        launched = handle.ternel_tq1_linear_launches(batch, N, K, 0)
+        wide = batch > 1 and launched == 3  # TERNEL_TQ1_GEMM_WIDE
         strip = batch == 1 and m1_form(handle, N, K).startswith("strip")
-        lut = handle.ternel_tq1_linear_kernel(batch, N, K, 0) == 100  # TERNEL_TQ1_KERNEL_LUT23
+        lut = launched == 100  # TERNEL_TQ1_KERNEL_LUT23
         names = WIDE_PHASES if wide else (STRIP_PHASES if strip else PHASES)
         lay = PackedTensorLayout.for_tensor(N, K)
         ring = ring_copies(packed_bytes(K, N))
@@ -633,7 +633,7 @@ def phase_profile(torch, dev, synthetic, pack_weights, tq1_matmul_words, tq1_lin
                     durations.setdefault(f"{names[a]} -> {names[b]}", []).append((st[b] - st[a]) / 100)
         if not spans:  # the dispatch picked a kernel without phase stamps (the tile form)
             print(json.dumps({"phase_profile": name, "K": K, "N": N, "M": batch,
-                              "kernel": handle.ternel_tq1_linear_kernel(batch, N, K, 0),
+                              "kernel": launched,
                               "note": "no phase stamps: the kernel the dispatch picks here is not stamped"}),
                   flush=True)
             del weights
