@@ -4582,8 +4582,13 @@ size_t ternel_tq1_swiglu_workspace_bytes(int64_t M, int64_t rows, int64_t column
                    ? std::max(lut, trit_workspace_bytes(trit))
                    : lut;
     }
-    if (swiglu_gemm_uses_trit(M, rows, columns, dtype))
-        return plan_trit(M, rows, columns, dtype, 0, &trit, true) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
+    if (swiglu_gemm_uses_trit(M, rows, columns, dtype)) {
+        const size_t need = plan_trit(M, rows, columns, dtype, 0, &trit, true) == TERNEL_TQ1_OK ? trit_workspace_bytes(trit) : 0;
+        if (dtype != TERNEL_TQ1_BF16) return need;
+        // bf16, as for the linear: no less than the wide form's, which grows with
+        // the batch, so that a workspace for the largest batch holds the others.
+        return std::max(need, ternel_tq1_gemm_workspace_bytes(M, rows, columns, TERNEL_TQ1_GEMM_WIDE, 0));
+    }
     if (resolve_gemm_form(M, rows, columns, linear_gemm_form(M, rows, columns, dtype), 0) == TERNEL_TQ1_GEMM_WIDE)
         return ternel_tq1_gemm_workspace_bytes(M, rows, columns, TERNEL_TQ1_GEMM_WIDE, 0);
     return swiglu_pairs_offset(M, rows, columns, dtype) + static_cast<size_t>(M) * rows * sizeof(_Float16);

@@ -200,3 +200,12 @@ def test_the_kernel_sweep_covers_every_kernel_of_every_type() -> None:
     runs = {(row["dtype"], row["runs"]) for row in KERNEL_SWEEP["rows"]}
     assert runs == {(t, k) for t in ("float16", "bfloat16") for k in ("strip", "lut23", "trit", "wide")} | \
         {("float16", "tile")} | {("float32", k) for k in ("strip", "lut23", "trit")}
+
+
+@pytest.mark.parametrize("name", ("ternel_tq1_linear_workspace_bytes", "ternel_tq1_swiglu_workspace_bytes"))
+def test_a_bf16_workspace_for_the_largest_batch_holds_the_smaller_ones(name) -> None:
+    size = getattr(_lib.lib(), name)
+    for rows, columns in ((34816, 5120), (8192, 5120), (5120, 6144), (4096, 4096), (1024, 5120), (300, 1152)):
+        for largest in (512, 768, 2048):
+            need = size(largest, rows, columns, _lib.DTYPE_BF16)
+            assert max(size(M, rows, columns, _lib.DTYPE_BF16) for M in range(33, largest)) <= need, (rows, columns)
