@@ -3571,18 +3571,27 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
         // partials' limit). us, equal chunks alone / now: 4096 x 8576 fp32 M=9
         // 71.7 / 14.0, 1024 x 8576 fp16 M=2 30.4 / 7.4, 4096 x 16768 bf16 M=32
         // 80.9 / 17.5, 16749 x 9728 (76 groups) fp32 M=10 83.5 / 43.6.
+        const int64_t most_chunks =
+            plan->row_blocks > kUsableCounters ? 1 : std::min(G, std::max<int64_t>(most_bytes / split_bytes, 1));
         auto chunk_of = [&](int64_t k, int64_t granule, bool equal) -> int64_t {  // groups; 0: no such split
-            if (k > 1 && (k * split_bytes > most_bytes || plan->row_blocks > kUsableCounters)) return 0;
+            if (k > most_chunks) return 0;
             if (equal) return G % k == 0 && (G / k) % granule == 0 ? G / k : 0;
             const int64_t chunk = ceil_div(ceil_div(G, k), granule) * granule;
             return ceil_div(G, chunk) == k ? chunk : 0;
         };
-        auto search = [&](int64_t granule, bool equal) {
+        // (This runs in every call: no loop over splits that cannot be.)
+        const int64_t wanted = ceil_div(kDirectTargetWorkgroups, blocks);
+        auto search = [&](int64_t granule, bool equal) -> int {
+            if (!equal) {  // the longest chunk that gives the wanted splits, else the shortest there is
+                const int64_t longest = wanted > 1 ? (G - 1) / (wanted - 1) / granule * granule : G;
+                if (longest >= granule && ceil_div(G, longest) <= most_chunks) return static_cast<int>(ceil_div(G, longest));
+                return static_cast<int>(ceil_div(G, ceil_div(ceil_div(G, most_chunks), granule) * granule));
+            }
             int best = 0;
-            for (int64_t k = 1; k <= G; ++k) {
-                if (!chunk_of(k, granule, equal)) continue;
+            for (int64_t k = 1, runs = G % granule ? 0 : std::min(G / granule, most_chunks); k <= runs; ++k) {
+                if (G / granule % k) continue;
                 best = static_cast<int>(k);
-                if (blocks * k >= kDirectTargetWorkgroups) break;
+                if (k >= wanted) break;
             }
             return best;
         };
@@ -3605,7 +3614,7 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
             double least = 0;
             for (const bool equal : {true, false}) {
                 const double most_us = best ? kTritUnequalGain * least : HUGE_VAL;
-                for (int64_t k = 1; k <= G; ++k) {
+                for (int64_t k = 1; k <= std::min(ceil_div(G, 4), most_chunks); ++k) {
                     const int64_t chunk = chunk_of(k, 4, equal);
                     if (!chunk) continue;
                     const int64_t n = blocks * k, per_cu = ceil_div(n, cus), rounds = ceil_div(n, 2 * cus);
@@ -3628,14 +3637,15 @@ int plan_trit(int64_t M, int64_t rows, int64_t columns, int dtype, int k_split, 
         // (Short rows that only 4 divides take equal chunks of 4: 9052 x 2560 M=6
         // 7.8 us, 8.2 in 8 + 8 + 4.)
         const bool fours = (f32 && plan->staged_rows >= 16) || (G % 8 == 4 && G <= 40);
-        int best = plan->staged_rows > 32 ? fastest() : widest(fours ? 4 : 8);
-        if (plan->staged_rows == 32 && G % 4 == 0 && blocks * widest(4) >= kDirectTargetWorkgroups) best = widest(4);
+        const int in_fours = plan->staged_rows > 32 ? 0 : widest(4);
+        int best = plan->staged_rows > 32 ? fastest() : (fours ? in_fours : widest(8));
+        if (plan->staged_rows == 32 && G % 4 == 0 && blocks * in_fours >= kDirectTargetWorkgroups) best = in_fours;
         // More chunks of 4 than the reduction loads in one batch pay only where
         // next to no workgroups are (us, chunks of 4 / 8: 2048 x 10752 M=3 11.0
         // / 9.5, 768 x 17408 9.4 / 8.9, but 128 x 12800 7.1 / 7.6).
         if (plan->staged_rows <= 32 && blocks * best < kDirectMinWorkgroups &&
-            (widest(4) <= kTritReduceBatch || blocks <= 4))
-            best = std::max(best, widest(4));
+            (in_fours <= kTritReduceBatch || blocks <= 4))
+            best = std::max(best, in_fours);
         // Other equal chunks where they do better: a few groups on a few rows in
         // chunks of one or two, that many workgroups at once (129 x 1280 M=6 4.6
         // us, 5.4 in 4 + 4 + 2); fewer chunks that all but reach the target
