@@ -105,8 +105,8 @@ __host__ __device__ inline uint32_t selector_entry(int i) {
 }
 
 // Pair tables: the same pairs of trits directly as two 16-bit MFMA operand
-// values, -1, 0 and +1 in a type whose 1 has the bits `one` (fp16 0x3c00, bf16
-// 0x3f80). Tables read eight bytes at a time hold two dwords per entry:
+// values, -1, 0 and +1 times a power of two whose bits are `one` (fp16 1, 0x3c00;
+// bf16 2^-8, 0x3b80; the terms of fp32 2^-1 in bf16, 0x3f00). Tables read eight bytes at a time hold two dwords per entry:
 //   T27a[a / 9] = (a2, a3), (a4, 0)      T27b[b % 27] = (0, b0), (b1, b2)
 //   T9a[a % 9] = (a0, a1), unused        T9b[b / 27] = (b3, b4), one dword
 // Each table spans at most 58 dwords, so a wave's lookups into one never

@@ -1714,12 +1714,13 @@ __device__ __forceinline__ int direct_source_unit(int u) { return u < 15 ? u : (
 // of weight row l % 32 straight into an operand of v_mfma_f32_32x32x16, in the
 // K order of the direct forms (half h: code bytes 12h .. 12h+11 as positions
 // 0..59, then four trits of code byte 24 and the tail). The trits themselves
-// are the operand: -1, 0 and +1 in the activations' MFMA type, looked up in
-// pairs (pair tables in LDS, tq1_bytes.h: two dwords per code byte pair half,
-// no permute per pair), and the block's scale multiplies the fp32 group sums,
-// acc = fma(scale, sum, acc), the LUT23 kernels' order. So one kernel serves
-// every activation type with no conversion of the weights or activations:
-//   fp16, bf16  the activations as they are (products with -1/0/+1 exact);
+// are the operand: -1, 0 and +1 in the activations' MFMA type (times a power of
+// two that the scale takes back, TritOperand), looked up in pairs (pair tables
+// in LDS, tq1_bytes.h: two dwords per code byte pair half, no permute per
+// pair), and the block's scale multiplies the fp32 group sums, acc =
+// fma(scale, sum, acc), the LUT23 kernels' order. So one kernel serves every
+// activation type with no conversion of the weights or activations:
+//   fp16, bf16  the activations as they are (products with a trit exact);
 //   fp32        each value as three bf16 terms (its significand's upper,
 //               middle and lower 8 bits, the lower ones scaled up so that
 //               none is lost: exact), three MFMAs per K slice.
@@ -3938,16 +3939,15 @@ int linear_gemm_form(int64_t M, int64_t rows, int64_t columns, int dtype) {
 }
 
 // The trit kernel runs the direct form (fp16), and batches of the automatic
-// forms that it is faster for (never a form asked for by name): bf16 up to 32 rows, and
-// tiles of up to 64 rows above that (fp16 where the direct form ends). Small
+// forms that it is faster for (never a form asked for by name): bf16 up to 32
+// rows, and tiles of up to 64 rows above that (fp16 where the direct form ends). Small
 // matrices give the wide form's 256-row tiles too few CUs or too long a
 // reduction, and the tile form waits for each group's loads. Measured on MI355X
 // (us, trit / best other fp16 form; the bf16 wide form is 2-8 us slower than
 // the fp16 one for its scaling pass):
 //   under 4 MB: 4096 square M=128 17 / 26, M=768 44 / 47; k_proj M=128 16 / 27,
-//   M=768 26 / 30, M=1024 34 / 33; 3000 x 3072 M=768 35 / 35; short rows under
-//   64 KB the tile form's one short launch: 57 x 1152 M=90 10.8 / 10.1, 110 x 1664 M=81
-//   11.8 / 11.0;
+//   M=768 26 / 30, M=1024 34 / 33; 3000 x 3072 M=768 35 / 35; but short rows
+//   under 64 KB 57 x 1152 M=90 10.8 / 10.1, 110 x 1664 M=81 11.8 / 11.0;
 //   under 12 MB: out_proj M=128 22 / 29, M=384 39 / 44, M=512 58 / 54; QKV M=203
 //   34 / 41, M=384 52 / 52; 12288 x 2048 M=128 17 / 29, M=384 37 / 37, bf16 M=512
 //   40 / 42; but on long rows 1500 x 17408 M=128 30 / 29, M=203 42 / 34, where

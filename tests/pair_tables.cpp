@@ -33,7 +33,8 @@ int main() {
     const int spans[4] = {kPairT27b - kPairT27a, kPairT9a - kPairT27b, kPairT9b - kPairT9a, kPairEntries - kPairT9b};
     for (int i = 0; i < 4; ++i) expect(spans[i] <= 64, "a table spans at most the 64 banks", i, 0);
     const uint32_t ones[2] = {0x3c00u, 0x3f80u};
-    for (uint32_t one : ones) {
+    const uint32_t scaled[4] = {ones[0], ones[1], 0x3b80u, 0x3f00u};  // and bf16's 2^-8, fp32's 2^-1
+    for (uint32_t one : scaled) {
         for (int i = 0; i < kPairEntries; ++i)  // every half is -1, 0 or +1, illegal bytes' too
             for (int h = 0; h < 2; ++h) {
                 const uint32_t half = (pair_entry(i, one) >> (16 * h)) & 0xffffu;
